@@ -1899,8 +1899,10 @@ __global__ __launch_bounds__(NT_SCF) void k_scf_fock(const Scf3* __restrict__ ss
 }
 
 // generalized eigh of Fd: Fp = X^T Fd X (symmetrised), Fp = Z diag(e) Z^T in LDS, C = X Z,
-// D = 2 C_occ C_occ^T.  One workgroup of 1024 threads.
-constexpr int NT_EIG = 1024;
+// D = 2 C_occ C_occ^T.  One workgroup of NT_EIG threads.
+constexpr int NT_EIG = 512;  // 8 waves: 256 registers a lane for the eigensolver's patches and columns
+static_assert(NT_EIG >= qexeig::NT_MIN, "eigensolver threads");
+constexpr int NT_VJP = 1024;
 size_t eigh_lds(int n) { return (size_t)2 * n * (n + 1) * 8; }
 
 // full = 0 (the SCF cycles): only the orbitals the cycle uses (the n_occ + 2 lowest; C's other
@@ -1909,7 +1911,7 @@ size_t eigh_lds(int n) { return (size_t)2 * n * (n + 1) * 8; }
 __global__ __launch_bounds__(NT_EIG) void k_scf_eigh(const Scf3* __restrict__ ss, int full) {
   const Scf3 s = ss[blockIdx.x];
   if (s.ist[0] && !full) return;
-  extern __shared__ double sm[];
+  extern __shared__ __attribute__((aligned(16))) double sm[];
   __shared__ qexeig::Smem sh;
   const int n = s.n, nn = n * n, S = n + 1;
   double* A = sm;
@@ -1933,7 +1935,7 @@ __global__ __launch_bounds__(NT_EIG) void k_scf_eigh(const Scf3* __restrict__ ss
 // batched generalized eigh F C = S C e, one workgroup per matrix (scratch: 8 n^2 doubles each)
 __global__ __launch_bounds__(NT_EIG) void k_gen_eigh(int n, const double* F, const double* Sm, double* mo, double* C,
                                                      double* scratch) {
-  extern __shared__ double sm[];
+  extern __shared__ __attribute__((aligned(16))) double sm[];
   __shared__ qexeig::Smem sh;
   const size_t nn = (size_t)n * n, b = blockIdx.x;
   const int S = n + 1;
@@ -1960,7 +1962,7 @@ __global__ __launch_bounds__(NT_EIG) void k_gen_eigh(int n, const double* F, con
 //   M = F o (U gV) + diag(gw),  F_ij = 1 / (w_j - w_i), 0 where |w_j - w_i| < eps^0.6,
 //   gA = sym(V M U);
 // either cotangent may be absent.  One workgroup per matrix; products on FP64 matrix cores.
-__global__ __launch_bounds__(NT_EIG) void k_eigh_vjp(int n, const double* w, const double* v, const double* gw,
+__global__ __launch_bounds__(NT_VJP) void k_eigh_vjp(int n, const double* w, const double* v, const double* gw,
                                                      const double* gv, double* gA, double* ws, int exact) {
   const size_t nn = (size_t)n * n, b = blockIdx.x;
   const double* W = w + b * n;
@@ -3136,7 +3138,7 @@ int qex3d_eigh_vjp(int32_t batch, int32_t n, const double* w, const double* v, c
     return fail3(QEX_E_BADARG, "bad eigh_vjp arguments (n must be in [1, %d])", QEX3D_MAX_NAO);
   const size_t need = qex3d_eigh_vjp_workspace_bytes(batch, n);
   if (!workspace || workspace_bytes < need) return fail3(QEX_E_WORKSPACE, "workspace too small: need %zu", need);
-  hipLaunchKernelGGL(k_eigh_vjp, dim3(batch), dim3(NT_EIG), 0, (hipStream_t)stream, n, w, v, gw, gv, gA,
+  hipLaunchKernelGGL(k_eigh_vjp, dim3(batch), dim3(NT_VJP), 0, (hipStream_t)stream, n, w, v, gw, gv, gA,
                      (double*)workspace, exact);
   return launch_status("qex3d_eigh_vjp");
 }

@@ -1,18 +1,25 @@
-// symeig.h -- dense symmetric eigensolver for one workgroup (n <= 96, FP64, matrix in LDS).
+// symeig.h -- dense symmetric eigensolver for one workgroup (n <= 96, FP64).
 //
-//   1. Householder tridiagonalisation: for k = 0..n-3 the reflector H_k = I - 2 v v^T (|v| = 1)
-//      annihilates column k below the subdiagonal; the trailing block is updated as
-//      A <- A - v w^T - w v^T with p = A v, beta = v^T p, w = 2 p - 2 beta v.  v is kept in column k
-//      of A (below the diagonal), d / e collect the tridiagonal.
-//   2. T splits into unreduced blocks where |e_k| <= eps (|d_k| + |d_k+1|).
-//   3. Eigenvalues: multisection on Sturm counts (negative pivots of the LDL^T of T - x), G threads
-//      per eigenvalue, a fixed number of rounds (interval / (G+1) per round).
-//   4. Eigenvectors of T: inverse iteration (3 steps with the LDL^T pivots of T - lam, pivots
-//      smaller than eps |T| replaced by +-eps |T|) from a fixed pseudo-random start; eigenvalues of one block
-//      closer than 1e-8 |T| form a cluster whose vectors one thread computes in order, removing
-//      the earlier members' components after every solve.
-//   5. Ascending sort and back-transformation Z <- H_0 ... H_{n-3} Y.
+//   1. Householder tridiagonalisation with the matrix in registers (256 threads, each a cyclic
+//      patch): for k = 0..n-3 the reflector H_k = I - tau v v^T annihilates column k below the
+//      subdiagonal; the trailing block becomes A - v w^T - w v^T with p = tau A v,
+//      w = p - (tau / 2)(v^T p) v.  The rows v_k go to global scratch, d / e collect the tridiagonal.
+//   2. T, scaled by a power of two to norm 1..2, splits into unreduced blocks where
+//      |e_k| <= eps (|d_k| + |d_k+1|).
+//   3. Eigenvalues: multisection on Sturm counts (sign changes of the leading minors of T - x), three
+//      lanes per eigenvalue, a fixed number of rounds (interval / 4 per round).
+//   4. Eigenvectors of T: two inverse iterations (LDL^T pivots of T - lam, pivots smaller than
+//      eps |T| replaced by +-eps |T|) from a fixed pseudo-random start, one lane per vector; eigenvalues
+//      of one block closer than 1e-5 |T| form a cluster, whose vectors are orthogonalised after every
+//      solve.  Rayleigh quotients give the eigenvalues.
+//   5. Ascending sort and back-transformation Z <- H_0 ... H_{n-3} Y, four lanes per column.
 // All reductions run in a fixed order: the result does not depend on timing.
+//
+// What bounds it: every stage is a chain of dependent steps of one workgroup, so its time is
+// barriers and latencies, not arithmetic.  Hence the matrix stays in registers (two barriers and a
+// few LDS words per Householder step; the LDS-resident form took three barriers over 16 waves and
+// re-read the block), the counts need no reciprocal and no barrier, and a column of the
+// back-transformation stays in four lanes' registers from the first reflector to the last.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -20,6 +27,23 @@ namespace qexeig {
 
 constexpr double EPS = 2.220446049250313e-16;
 constexpr int MAXN = 96;
+// eigenvalues of a block closer than CLUSTER |T| are orthogonalised against each other: two inverse
+// iterations leave vectors eps / gap apart from orthogonal, 1e-11 at this gap
+constexpr double CLUSTER = 1e-5;
+constexpr int NT_MIN = 512;  // threads the solver needs (it uses the first 512 of the workgroup)
+
+// f(0), ..., f(N - 1) with compile-time indices (register arrays stay in registers)
+template <int I>
+struct Index {
+  static constexpr int value = I;
+};
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(Index<I>{});
+    static_for<I + 1, N>(f);
+  }
+}
 
 // one DPP move of a double (both halves)
 template <int CTRL>
@@ -44,14 +68,34 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
+__device__ __forceinline__ double wave_max(double x) {
+  x = fmax(x, dpp_f64<0xB1>(x));
+  x = fmax(x, dpp_f64<0x4E>(x));
+  x = fmax(x, dpp_f64<0x141>(x));
+  x = fmax(x, dpp_f64<0x140>(x));
+  return fmax(fmax(read_lane(x, 0), read_lane(x, 16)), fmax(read_lane(x, 32), read_lane(x, 48)));
+}
+
+// sum over an aligned group of 4 / 8 lanes, the same value in each of them
+__device__ __forceinline__ double group4_sum(double x) {
+  x += dpp_f64<0xB1>(x);
+  x += dpp_f64<0x4E>(x);
+  return x;
+}
+__device__ __forceinline__ double group8_sum(double x) {
+  x = group4_sum(x);
+  x += dpp_f64<0x141>(x);
+  return x;
+}
+
 // Shared state of the solver (static LDS besides the two n x S matrices).
 struct Smem {
-  double d[MAXN], e[MAXN], e2[MAXN], lam[MAXN], lo[MAXN], rq[MAXN];
-  double sg, alpha, iv, v0;  // reflector scalars of the current Householder step
-  int bs[MAXN], bt[MAXN], loc[MAXN], perm[MAXN];
-  unsigned char cnt[2][1024];
+  double d[MAXN], e[MAXN], lam[MAXN], rq[MAXN], tau[MAXN], nv[MAXN];
+  double x[MAXN + 8], p[MAXN + 8];   // column being reduced; p = tau A v
+  double2 de[MAXN + 8];              // (d_i, e_{i-1}^2) for the Sturm counts
+  int bs[MAXN], bt[MAXN], perm[MAXN];
+  unsigned long long cut[2];
   unsigned char need[MAXN];  // slot's vector wanted (nvec < n: its eigenvalue ranks below nvec)
-  double norm;
 };
 
 // 1/d: hardware reciprocal refined by one Newton step (relative error ~1e-15)
@@ -60,32 +104,35 @@ __device__ __forceinline__ double rcp_nr(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
-// number of eigenvalues of the block below x (negative pivots of the LDL^T of T - x); e2 = e^2
-// The reciprocal of a pivot is clamped to +-rmax = 1/pivmin instead of testing the pivot; the
-// sign bit of each pivot is counted with integer arithmetic.
-// The diagonal and e^2 are read from LDS 8 entries at a time, so the LDS latency is paid once
-// per 8 steps of the pivot recurrence.
-__device__ __forceinline__ int sturm_count(const double* d, const double* e2, int s, int t, double x, double rmax) {
-  double q = d[s] - x;
-  unsigned c = (unsigned)((unsigned long long)__double_as_longlong(q) >> 63);
-  auto step = [&](double dj, double ej) {
-    const double r = fmin(fmax(rcp_nr(q), -rmax), rmax);
-    q = fma(-ej, r, dj - x);
-    c += (unsigned)((unsigned long long)__double_as_longlong(q) >> 63);
+// Number of eigenvalues of rows s..t-1 of T below x: the sign changes of the leading minors
+// p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}.  No division, so a row is one dependent FMA (a pivot
+// recurrence needs a reciprocal, a Newton step and two clamps in the chain: 60 cycles a row against
+// 16).  T is scaled to norm 1..2 and e^2 floored at 1e-60, so 8 rows change a minor by less than
+// 1e-250 .. 1e6 and both minors never vanish together; they are rescaled by a power of two every 8 rows.
+__device__ __forceinline__ int sturm_count(const double2* de, int s, int t, double x) {
+  double p0 = 0.0, p1 = 1.0;
+  unsigned bits = 0, c = 0;
+  auto step = [&](double2 v) {
+    const double pn = fma(v.x - x, p1, -(v.y * p0));
+    p0 = p1;
+    p1 = pn;
+    bits = __builtin_amdgcn_alignbit(bits, (unsigned)__double2hiint(pn), 31);  // bits << 1 | sign
   };
-  int j = s + 1;
+  int j = s;
   for (; j + 8 <= t; j += 8) {
-    double dv[8], ev[8];
+    double2 v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      dv[u] = d[j + u];
-      ev[u] = e2[j + u - 1];
-    }
+    for (int u = 0; u < 8; ++u) v[u] = de[j + u];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) step(dv[u], ev[u]);
+    for (int u = 0; u < 8; ++u) step(v[u]);
+    c += __popc((bits ^ (bits >> 1)) & 0xFFu);
+    const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+    p0 = ldexp(p0, ex);
+    p1 = ldexp(p1, ex);
   }
-  for (; j < t; ++j) step(d[j], e2[j - 1]);
-  return (int)c;
+  const int left = t - j;
+  for (; j < t; ++j) step(de[j]);
+  return (int)(c + __popc((bits ^ (bits >> 1)) & ((1u << left) - 1u)));
 }
 
 // deterministic start vector entry in [-1, 1)
@@ -97,145 +144,263 @@ __device__ __forceinline__ double start_entry(int slot, int i) {
   return (double)(x & 0xFFFFFF) / 8388608.0 - 1.0;
 }
 
-// Inverse pivots 1/D_i of the LDL^T factorisation of T_block - lam (|D| >= tiny), stored in column
-// `col` of Dm (row stride S).  d and e^2 are read 4 rows per LDS wait (one thread runs the whole
-// recurrence, so only the arithmetic stays on its dependency chain; 8 rows spill registers).
-__device__ __forceinline__ void ldl_pivots(const double* d, const double* e2, int s, int t, double lam, double tiny, double* Dm,
-                           int S, int col) {
-  double q = d[s] - lam;
-  if (fabs(q) < tiny) q = q < 0.0 ? -tiny : tiny;
-  double qi = 1.0 / q;
-  Dm[s * S + col] = qi;
-  auto step = [&](int i, double di, double ei) {
-    q = (di - lam) - ei * qi;
-    if (fabs(q) < tiny) q = q < 0.0 ? -tiny : tiny;
-    qi = 1.0 / q;
-    Dm[i * S + col] = qi;
-  };
-  int i = s + 1;
-  for (; i + 4 <= t; i += 4) {
-    double dv[4], ev[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      dv[u] = d[i + u];
-      ev[u] = e2[i + u - 1];
+// One thread: column `col` of Y <- (T_block - lam)^-1 b, rows s..t-1, with the inverse pivots 1/D_i
+// of T_block - lam (|1/D| <= rmax) in column `col` of Dm.  FIRST: b is the start vector, and the
+// pivots are computed along with the forward solve; else b = scale * Y and the pivots are read.
+// Returns |x|^2.  The operands of 8 rows are in flight per LDS wait.
+template <bool FIRST>
+__device__ __forceinline__ double ldl_solve(const double* d, const double* e, int s, int t, double lam, double rmax,
+                                            double* Dm, double* Y, int S, int col, double scale) {
+  double y = 0.0, qi = 0.0, ep = 0.0;
+  auto fwd = [&](int i, double di, double ei, double bi, double ri) {
+    // row i: l = e_{i-1} / D_{i-1}; D_i = d_i - lam - e_{i-1} l; y_i = b_i - l y_{i-1}
+    const double l = ep * qi;
+    y = fma(-l, y, bi);
+    if (FIRST) {
+      const double q = fma(-ep, l, di - lam);
+      qi = fmin(fmax(rcp_nr(q), -rmax), rmax);
+      Dm[i * S + col] = qi;
+    } else {
+      qi = ri;
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) step(i + u, dv[u], ev[u]);
-  }
-  for (; i < t; ++i) step(i, d[i], e2[i - 1]);
-}
-
-// (T_block - lam) x = b in place in column `col` of Y, with the inverse pivots from ldl_pivots:
-// forward y_i = b_i - e_i-1 (1/D_i-1) y_i-1, then x_i = (y_i - e_i x_i+1) / D_i.  The operands of
-// 4 rows are loaded per LDS wait; the chain carries one FMA (and one multiply) per row.
-__device__ __forceinline__ void ldl_solve(const double* e, int s, int t, const double* Dm, double* Y, int S, int col) {
-  double prev = Y[s * S + col];
-  int i = s + 1;
-  for (; i + 4 <= t; i += 4) {
-    double yv[4], cv[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      yv[u] = Y[(i + u) * S + col];
-      cv[u] = e[i + u - 1] * Dm[(i + u - 1) * S + col];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      prev = yv[u] - cv[u] * prev;
-      Y[(i + u) * S + col] = prev;
-    }
-  }
-  for (; i < t; ++i) {
-    const double y = Y[i * S + col] - e[i - 1] * Dm[(i - 1) * S + col] * prev;
     Y[i * S + col] = y;
-    prev = y;
-  }
-  double next = Y[(t - 1) * S + col] * Dm[(t - 1) * S + col];
-  Y[(t - 1) * S + col] = next;
-  i = t - 2;
-  for (; i - 3 >= s; i -= 4) {
-    double yv[4], ev[4], dv[4];
+    ep = ei;
+  };
+  int i = s;
+  for (; i + 8 <= t; i += 8) {
+    double dv[8], ev[8], bv[8], rv[8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      yv[u] = Y[(i - u) * S + col];
-      ev[u] = e[i - u];
-      dv[u] = Dm[(i - u) * S + col];
+    for (int u = 0; u < 8; ++u) {
+      ev[u] = e[i + u];
+      if (FIRST) {
+        dv[u] = d[i + u];
+        bv[u] = start_entry(col, i + u);
+        rv[u] = 0.0;
+      } else {
+        dv[u] = 0.0;
+        bv[u] = scale * Y[(i + u) * S + col];
+        rv[u] = Dm[(i + u) * S + col];
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      next = (yv[u] - ev[u] * next) * dv[u];
-      Y[(i - u) * S + col] = next;
+    for (int u = 0; u < 8; ++u) fwd(i + u, dv[u], ev[u], bv[u], rv[u]);
+  }
+  for (; i < t; ++i)
+    fwd(i, d[i], e[i], FIRST ? start_entry(col, i) : scale * Y[i * S + col], FIRST ? 0.0 : Dm[i * S + col]);
+  // x_i = y_i / D_i - (e_i / D_i) x_{i+1}; e_{t-1} = 0 at a block's end
+  double x = 0.0, n0 = 0.0;
+  i = t - 1;
+  for (; i - 7 >= s; i -= 8) {
+    double yv[8], rv[8], lv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      rv[u] = Dm[(i - u) * S + col];
+      yv[u] = Y[(i - u) * S + col] * rv[u];
+      lv[u] = e[i - u] * rv[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      x = fma(-lv[u], x, yv[u]);
+      n0 = fma(x, x, n0);
+      Y[(i - u) * S + col] = x;
     }
   }
   for (; i >= s; --i) {
-    next = (Y[i * S + col] - e[i] * next) * Dm[i * S + col];
-    Y[i * S + col] = next;
+    const double r = Dm[i * S + col];
+    x = fma(-(e[i] * r), x, Y[i * S + col] * r);
+    n0 = fma(x, x, n0);
+    Y[i * S + col] = x;
   }
+  return n0;
 }
 
-// sum over the 8 lanes of an aligned lane group by DPP moves (swap within pairs, within quads,
-// then the half-row mirror pairs each quad with the other one); every lane receives the same value
-__device__ __forceinline__ double group8_sum(double x) {
-  x += dpp_f64<0xB1>(x);   // quad_perm [1, 0, 3, 2]
-  x += dpp_f64<0x4E>(x);   // quad_perm [2, 3, 0, 1]
-  x += dpp_f64<0x141>(x);  // row_half_mirror
-  return x;
-}
-
-// sum_{i<m} a[i*sa] * b[i*sb] with 8 independent partial sums (shorter dependency chains on LDS
-// loads), combined in a fixed order
-__device__ __forceinline__ double dot8(const double* a, int sa, const double* b, int sb, int m) {
-  double c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  int i = 0;
-  for (; i + 7 < m; i += 8) {
+// Householder tridiagonalisation of A (n x n in LDS, row stride S; only read).  NC >= ceil(n / 8).
+// Threads 0..255: thread (r, c) = (tid / 8, tid % 8) holds A[r + 32 i][c + 8 j] in registers; the other
+// waves only take part in the barriers.  32 x 8 rather than 16 x 16: row sums then cross 8 lanes (three
+// DPP steps for 3 rows) instead of 16 (four steps for 6 rows).  Per step: the owners of column k put it
+// in LDS | every thread forms v, tau and its rows of p = tau A v | p in LDS | rank-2 update.
+// Row k of f (stride 8 NC, zero padded) receives v_k; sh.d, sh.e, sh.tau the rest.
+template <int NC>
+__device__ __forceinline__ void tridiagonalise(int n, const double* A, int S, double* f, Smem& sh) {
+  constexpr int NR = (NC + 3) / 4, SP = 8 * NC;
+  const int tid = threadIdx.x;
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) >= 4) {
+    __syncthreads();
+    for (int q = 1; q <= n - 2; ++q) {
+      __syncthreads();
+      __syncthreads();
+    }
+    __syncthreads();
+    return;
+  }
+  const int r = tid >> 3, c = tid & 7;
+  double a[NR][NC];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) c[u] = fma(a[(i + u) * sa], b[(i + u) * sb], c[u]);
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int row = r + 32 * i, col = c + 8 * j;
+      a[i][j] = row < n && col < n ? A[row * S + col] : 0.0;
+    }
+  // column 0 below the diagonal
+  if (c == 0) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) sh.x[r + 32 * i] = r + 32 * i >= 1 ? a[i][0] : 0.0;
+    if (r == 0) sh.d[0] = a[0][0];
   }
-  for (; i < m; ++i) c[0] = fma(a[i * sa], b[i * sb], c[0]);
-  return ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+  __syncthreads();
+  static_for<0, NC>([&](auto block) {
+    constexpr int jb = decltype(block)::value, ib = jb / 4;
+    for (int c0 = 0; c0 < 8; ++c0) {
+      const int q = 8 * jb + c0;  // reduces column q - 1 to rows <= q
+      if (q < 1) continue;
+      if (q > n - 2) break;
+      double vc[NC], vr[NR];
+#pragma unroll
+      for (int j = jb; j < NC; ++j) vc[j] = sh.x[c + 8 * j];
+#pragma unroll
+      for (int i = ib; i < NR; ++i) vr[i] = sh.x[r + 32 * i];
+      const double x0 = sh.x[q];
+      double tail = 0.0;
+      {
+        const double t = c == c0 ? 0.0 : vc[jb];
+        tail = t * t;
+#pragma unroll
+        for (int j = jb + 1; j < NC; ++j) tail = fma(vc[j], vc[j], tail);
+      }
+      tail = group8_sum(tail);
+      const bool skip = !(tail > 0.0);
+      const double nx = sqrt(fma(x0, x0, tail));
+      const double alpha = x0 >= 0.0 ? -nx : nx;
+      const double v0 = skip ? 0.0 : x0 - alpha;
+      const double tau = skip ? 0.0 : rcp_nr(nx * (nx + fabs(x0)));
+      double u[NR];
+#pragma unroll
+      for (int i = ib; i < NR; ++i) {
+        u[i] = 0.0;
+#pragma unroll
+        for (int j = jb + 1; j < NC; ++j) u[i] = fma(a[i][j], vc[j], u[i]);
+      }
+      if (c == c0) vc[jb] = v0;
+      if (r == (q & 31)) vr[ib] = v0;
+#pragma unroll
+      for (int i = ib; i < NR; ++i) {
+        u[i] = tau * group8_sum(fma(a[i][jb], vc[jb], u[i]));
+        if (c == 0) sh.p[r + 32 * i] = u[i];
+      }
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+        if (r == j) f[(size_t)(q - 1) * SP + c + 8 * j] = j < jb ? 0.0 : vc[j];
+      if (tid == 0) {
+        sh.e[q - 1] = skip ? x0 : alpha;
+        sh.tau[q - 1] = tau;
+      }
+      __syncthreads();
+      double wc[NC];
+      double vp = 0.0;
+#pragma unroll
+      for (int j = jb; j < NC; ++j) {
+        wc[j] = sh.p[c + 8 * j];
+        vp = fma(vc[j], wc[j], vp);
+      }
+      const double K = 0.5 * tau * group8_sum(vp);
+#pragma unroll
+      for (int j = jb; j < NC; ++j) wc[j] = fma(-K, vc[j], wc[j]);
+#pragma unroll
+      for (int i = ib; i < NR; ++i) {
+        const double wr = fma(-K, vr[i], u[i]);
+#pragma unroll
+        for (int j = jb; j < NC; ++j) a[i][j] = fma(-vr[i], wc[j], fma(-wr, vc[j], a[i][j]));
+      }
+      // column q, the next one, and d_q (x was last read before the barrier above)
+      if (c == c0) {
+#pragma unroll
+        for (int i = ib; i < NR; ++i) {
+          const int row = r + 32 * i;
+          sh.x[row] = row > q ? a[i][jb] : 0.0;
+          if (row == q) sh.d[q] = a[i][jb];
+        }
+      }
+      __syncthreads();
+    }
+  });
+  if (tid == 0) sh.e[n - 2] = sh.x[n - 1];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (r + 32 * i == n - 1 && c + 8 * j == n - 1) sh.d[n - 1] = a[i][j];
+  __syncthreads();
 }
 
-// sum_i a[i * S] b[i * S] over rows s..t-1 of two columns: 4 rows per LDS wait, 4 partial sums
-// combined in a fixed order
-__device__ __forceinline__ double col_dot4(const double* a, const double* b, int S, int s, int t) {
-  double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
-  int i = s;
-  for (; i + 4 <= t; i += 4) {
-    const double a0 = a[i * S], a1 = a[(i + 1) * S], a2 = a[(i + 2) * S], a3 = a[(i + 3) * S];
-    const double b0 = b[i * S], b1 = b[(i + 1) * S], b2 = b[(i + 2) * S], b3 = b[(i + 3) * S];
-    c0 = fma(a0, b0, c0);
-    c1 = fma(a1, b1, c1);
-    c2 = fma(a2, b2, c2);
-    c3 = fma(a3, b3, c3);
+// Z <- H_0 ... H_{n-3} Y: column c of the result from column perm[c] of Y (in Z), scaled by nv.
+// Four lanes hold a column: lane q the rows 8 i + 2 q + {0, 1}.  V (n - 2 rows of stride 8 NC) is
+// read into the LDS of both matrices once every column is in registers.
+template <int NC>
+__device__ __forceinline__ void back_transform(int n, int nvec, double* A, double* Z, int S, const double* f, Smem& sh) {
+  constexpr int SP = 8 * NC;
+  const int tid = threadIdx.x, nt = blockDim.x, c = tid >> 2, q4 = tid & 3;
+  const bool act = c < nvec;
+  double2 z[NC];
+  {
+    const int sl = act ? sh.perm[c] : 0;
+    const double sc = act ? sh.nv[sl] : 0.0;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int row = 8 * i + 2 * q4;
+      z[i].x = act && row < n ? sc * Z[row * S + sl] : 0.0;
+      z[i].y = act && row + 1 < n ? sc * Z[(row + 1) * S + sl] : 0.0;
+    }
   }
-  for (; i < t; ++i) c0 = fma(a[i * S], b[i * S], c0);
-  return (c0 + c1) + (c2 + c3);
-}
-
-__device__ __forceinline__ double col_norm2(const double* Y, int S, int s, int t, int col) {
-  return col_dot4(Y + col, Y + col, S, s, t);
-}
-
-// x[i * S] *= f over rows s..t-1, 4 rows per LDS wait
-__device__ __forceinline__ void col_scale4(double* x, int S, int s, int t, double f) {
-  int i = s;
-  for (; i + 4 <= t; i += 4) {
-    const double x0 = x[i * S], x1 = x[(i + 1) * S], x2 = x[(i + 2) * S], x3 = x[(i + 3) * S];
-    x[i * S] = x0 * f;
-    x[(i + 1) * S] = x1 * f;
-    x[(i + 2) * S] = x2 * f;
-    x[(i + 3) * S] = x3 * f;
+  __syncthreads();
+  for (int idx = tid; idx < (n - 2) * SP; idx += nt) A[idx] = f[idx];
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(c & ~15) < nvec) {  // (16 columns a wave)
+    static_for<0, NC>([&](auto block) {
+      constexpr int jb = NC - 1 - decltype(block)::value;
+      for (int c0 = 7; c0 >= 0; --c0) {
+        const int k = 8 * jb + c0 - 1;  // rows > k
+        if (k > n - 3) continue;
+        if (k < 0) break;
+        const double2* v = reinterpret_cast<const double2*>(A + (size_t)k * SP) + q4;
+        double2 vv[NC];
+        double acc0 = 0.0, acc1 = 0.0;
+#pragma unroll
+        for (int i = jb; i < NC; ++i) {
+          vv[i] = v[4 * i];
+          acc0 = fma(vv[i].x, z[i].x, acc0);
+          acc1 = fma(vv[i].y, z[i].y, acc1);
+        }
+        const double s = sh.tau[k] * group4_sum(acc0 + acc1);
+#pragma unroll
+        for (int i = jb; i < NC; ++i) {
+          z[i].x = fma(-s, vv[i].x, z[i].x);
+          z[i].y = fma(-s, vv[i].y, z[i].y);
+        }
+      }
+    });
   }
-  for (; i < t; ++i) x[i * S] *= f;
+  __syncthreads();
+  if (c < n) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int row = 8 * i + 2 * q4;
+      if (row < n) Z[row * S + c] = z[i].x;
+      if (row + 1 < n) Z[(row + 1) * S + c] = z[i].y;
+    }
+  }
+  __syncthreads();
 }
 
-// A: n x n symmetric in LDS (row stride S, destroyed); Z: n x n LDS output, column j = eigenvector
-// of the j-th smallest eigenvalue; w: ascending eigenvalues (any memory).  f: global scratch of
-// 2 n^2 doubles (3 n^2 are reserved by the callers).  Must be called by every thread of the workgroup (blockDim.x a multiple of 64,
-// blockDim.x >= n).
+// A: n x n symmetric in LDS (row stride S = n + 1, 16-byte aligned, destroyed), directly followed in LDS by
+// Z: n x n output, column j = eigenvector of the j-th smallest eigenvalue; w: ascending eigenvalues (any
+// memory).  f: global scratch of 3 n^2 doubles (the reflectors: (n - 2) 8 NC <= 3 n^2, and <= 2 n S of
+// LDS, with NC = 2, 4, 8, 12 for n <= 16, 32, 64, 96).  Must be called by every thread of the workgroup
+// (blockDim.x a multiple of 64, >= NT_MIN).
 // nvec < n: only the eigenvectors of the nvec smallest eigenvalues (ranked by their multisection
 // values, whole clusters) are computed and back-transformed, into columns 0..nvec-1 of Z, exactly as
-// the full solve computes them; the other eigenvalues are the multisection values (not refined).
+// the full solve computes them (the other columns are zero); the other eigenvalues are the
+// multisection values (not refined).
 __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, double* w, double* f, Smem& sh,
                                        int nvec = 1 << 30) {
   if (nvec > n) nvec = n;
@@ -249,151 +414,99 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
     return;
   }
   // ---- 1. tridiagonalisation ----
-  const int grp = tid >> 3, sub = tid & 7;  // 8-lane groups
-  for (int k = 0; k + 2 < n; ++k) {
-    const int m = n - k - 1;
-    const double* colk = A + (size_t)(k + 1) * S + k;  // x_i = colk[i * S]
-    // (a) u_i = sum_{j>=1} A22[i][j] x_j (one 8-lane group per row); |x_1..|^2 by the last group
-    if (grp < m) {
-      const double* row = A + (size_t)(k + 1 + grp) * S + k + 1;
-      double acc = 0.0;
-      for (int j = 1 + sub; j < m; j += 8) acc = fma(row[j], colk[j * S], acc);
-      acc = group8_sum(acc);
-      if (sub == 0) sh.lo[grp] = acc;
-    } else if (grp == (nt >> 3) - 1) {
-      // the last group also forms the reflector's scalars (square roots and a division done once
-      // instead of in every wave); the other threads read them after the barrier
-      double acc = 0.0;
-      for (int i = 1 + sub; i < m; i += 8) acc = fma(colk[i * S], colk[i * S], acc);
-      acc = group8_sum(acc);
-      if (sub == 0) {
-        const double x0 = colk[0];
-        const double nx = sqrt(x0 * x0 + acc);
-        const double alpha = x0 >= 0.0 ? -nx : nx;
-        const double iv = !(acc > 0.0) ? 0.0 : 1.0 / sqrt(acc + (x0 - alpha) * (x0 - alpha));
-        sh.sg = acc;
-        sh.alpha = alpha;
-        sh.iv = iv;
-        sh.v0 = (x0 - alpha) * iv;
-      }
-    }
-    __syncthreads();
-    const double sg = sh.sg, x0 = colk[0], alpha = sh.alpha, iv = sh.iv, v0 = sh.v0;
-    const bool skip = !(sg > 0.0);
-    auto vget = [&](int i) -> double { return i == 0 ? v0 : colk[i * S] * iv; };
-    // p_i = A22[i][0] v0 + iv u_i
-    auto pget = [&](int i) -> double { return fma(A[(size_t)(k + 1 + i) * S + k + 1], v0, iv * sh.lo[i]); };
-    if (tid == 0) {
-      sh.d[k] = A[k * S + k];
-      sh.e[k] = skip ? x0 : alpha;
-    }
-    if (!skip) {
-      // (b) beta = v . p, reduced inside every wave (identical in all lanes and waves)
-      double bt = 0.0;
-      for (int j = lane; j < m; j += 64) bt = fma(vget(j), pget(j), bt);
-      bt = wave_sum(bt);
-      // (c) A22 -= v w^T + w v^T, w = 2 p - 2 beta v: rows by wave, columns by lane
-      const int j0 = lane, j1 = lane + 64;
-      const double vj0 = j0 < m ? vget(j0) : 0.0, wj0 = j0 < m ? 2.0 * (pget(j0) - bt * vj0) : 0.0;
-      const double vj1 = j1 < m ? vget(j1) : 0.0, wj1 = j1 < m ? 2.0 * (pget(j1) - bt * vj1) : 0.0;
-      __syncthreads();  // every p_j is read before row 0 of A22 (which holds A22[i][0]) changes
-      for (int i = wv; i < m; i += nw) {
-        const double vi = vget(i), wi = 2.0 * (pget(i) - bt * vi);
-        double* row = A + (size_t)(k + 1 + i) * S + k + 1;
-        if (j0 < m) row[j0] -= vi * wj0 + wi * vj0;
-        if (j1 < m) row[j1] -= vi * wj1 + wi * vj1;
-      }
-    }
-    __syncthreads();
-    // keep v in column k (read above by every thread, so store after the barrier)
-    for (int i = tid; i < m; i += nt) A[(k + 1 + i) * S + k] = skip ? 0.0 : vget(i);
-    // the next step reads only rows / columns > k + 1 of the trailing block and column k + 1
-  }
-  __syncthreads();
-  if (tid == 0) {
-    sh.d[n - 2] = A[(n - 2) * S + n - 2];
-    sh.e[n - 2] = A[(n - 1) * S + n - 2];
-    sh.d[n - 1] = A[(n - 1) * S + n - 1];
-    // ---- 2. split into unreduced blocks; slot -> (block, local index) ----
-    double nrm = 0.0;
-    for (int i = 0; i < n; ++i) {
-      const double r = fabs(sh.d[i]) + (i > 0 ? fabs(sh.e[i - 1]) : 0.0) + (i < n - 1 ? fabs(sh.e[i]) : 0.0);
-      nrm = fmax(nrm, r);
-    }
-    sh.norm = nrm > 0.0 ? nrm : 1e-300;
-    int s = 0;
-    for (int k = 0; k < n; ++k) {
-      const bool cut = k == n - 1 || fabs(sh.e[k]) <= EPS * (fabs(sh.d[k]) + fabs(sh.d[k + 1]));
-      if (k < n - 1 && cut) sh.e[k] = 0.0;
-      if (k < n - 1) sh.e2[k] = sh.e[k] * sh.e[k];
-      if (cut) {
-        for (int q = s; q <= k; ++q) {
-          sh.bs[q] = s;
-          sh.bt[q] = k + 1;
-          sh.loc[q] = q - s;
-        }
-        s = k + 1;
-      }
-    }
-  }
-  // reflectors (strict lower part of A) to f, so that A can hold the LDL^T pivots of phase 4
-  for (int idx = tid; idx < n * n; idx += nt)
-    if (idx / n > idx % n) f[idx] = A[(idx / n) * S + idx % n];
-  __syncthreads();
-  // ---- 3. eigenvalues by multisection ----
+  if (n <= 16)
+    tridiagonalise<2>(n, A, S, f, sh);
+  else if (n <= 32)
+    tridiagonalise<4>(n, A, S, f, sh);
+  else if (n <= 64)
+    tridiagonalise<8>(n, A, S, f, sh);
+  else
+    tridiagonalise<12>(n, A, S, f, sh);
+  // ---- 2. norm, scaling, unreduced blocks ----
+  double scale, unscale;  // powers of two
   {
-    // G shifts per eigenvalue (>= 10 for n <= 96 and 1024 threads), at most 32: every thread scans
-    // its eigenvalue's G counts after each round, so small n gains nothing from more
-    const int G = nt / n < 32 ? nt / n : 32;
-    const int slot = tid / G, g = tid % G;
-    const bool act = slot < n;
-    double lo = 0.0, hi = 0.0, rmax = 0.0;
-    int s = 0, t = 0, li = 0;
-    if (act) {
-      s = sh.bs[slot];
-      t = sh.bt[slot];
-      li = sh.loc[slot];
-      double emax = 0.0;
-      lo = 1e300;
-      hi = -1e300;
-      for (int j = s; j < t; ++j) {
-        const double r = (j > s ? fabs(sh.e[j - 1]) : 0.0) + (j < t - 1 ? fabs(sh.e[j]) : 0.0);
-        lo = fmin(lo, sh.d[j] - r);
-        hi = fmax(hi, sh.d[j] + r);
-        if (j < t - 1) emax = fmax(emax, sh.e2[j]);
-      }
-      const double span = fmax(hi - lo, EPS * sh.norm);
-      lo -= 1e-12 * span + 1e-300;
-      hi += 1e-12 * span + 1e-300;
-      rmax = 1.0 / fmax(1e-300, 1e-290 * emax);  // bound on |1 / pivot|
+    double nrm = 0.0;  // every wave by itself
+    for (int i = lane; i < n; i += 64)
+      nrm = fmax(nrm, fabs(sh.d[i]) + (i > 0 ? fabs(sh.e[i - 1]) : 0.0) + (i < n - 1 ? fabs(sh.e[i]) : 0.0));
+    nrm = wave_max(nrm);
+    int ex = nrm > 0.0 ? __builtin_amdgcn_frexp_exp(nrm) - 1 : 0;
+    ex = ex < -1000 ? -1000 : ex > 1000 ? 1000 : ex;
+    scale = ldexp(1.0, -ex);
+    unscale = ldexp(1.0, ex);
+  }
+  __syncthreads();
+  if (wv < 2) {
+    const int k = tid;  // 0 .. 127
+    double dk = 0.0, ek = 0.0;
+    bool cut = false;
+    if (k < n) {
+      dk = sh.d[k] * scale;
+      ek = k < n - 1 ? sh.e[k] * scale : 0.0;
+      cut = k == n - 1 || fabs(ek) <= EPS * (fabs(dk) + fabs(sh.d[k + 1] * scale));
     }
-    // the interval shrinks (G+1)-fold per round; 2^-35 of its width (ln = 24.3) is enough because
-    // inverse iteration refines the vector and the Rayleigh quotient then gives the eigenvalue
-    const int rounds = (int)ceil(24.3 / log((double)(G + 1))) + 1;
-    const double ig = 1.0 / (double)(G + 1);
-    for (int r = 0; r < rounds; ++r) {
-      unsigned char* cb = sh.cnt[r & 1];
-      const double wd = (hi - lo) * ig;
-      if (act) cb[slot * G + g] = (unsigned char)sturm_count(sh.d, sh.e2, s, t, fma(wd, (double)(g + 1), lo), rmax);
-      __syncthreads();
+    const unsigned long long m = __ballot(cut);
+    if (lane == 0) sh.cut[wv] = m;
+    if (k < n) {
+      sh.lam[k] = cut ? 0.0 : ek;  // (parked until every d, e is read)
+      sh.rq[k] = dk;
+    }
+  }
+  __syncthreads();
+  if (tid < n) {
+    const int k = tid;
+    const double ek = sh.lam[k], dk = sh.rq[k], em = k > 0 ? sh.lam[k - 1] : 0.0;
+    sh.d[k] = dk;
+    sh.e[k] = ek;
+    sh.de[k] = make_double2(dk, fmax(em * em, 1e-60));
+    const unsigned long long m0 = sh.cut[0], m1 = sh.cut[1];
+    // block of row k: after the last cut below k, up to the first cut at or above k
+    const unsigned long long b1 = k > 64 ? m1 & ((1ull << (k - 64)) - 1) : 0ull;
+    const unsigned long long b0 = k < 64 ? m0 & ((1ull << k) - 1) : m0;
+    sh.bs[k] = b1 ? 128 - __clzll((long long)b1) : b0 ? 64 - __clzll((long long)b0) : 0;
+    const unsigned long long a0 = k < 64 ? m0 >> k : 0ull;
+    const unsigned long long a1 = k < 64 ? m1 : m1 >> (k - 64);
+    sh.bt[k] = a0 ? k + __ffsll((long long)a0) : (k < 64 ? 64 : k) + __ffsll((long long)a1);
+  }
+  __syncthreads();
+  // ---- 3. eigenvalues by multisection: lanes 3 v .. 3 v + 2 of a wave for its slot v, no barriers ----
+  // 4^-25 of a width <= 4: 2^-48 of the norm.  Three lanes each: with n = 80 four waves, one per SIMD
+  // (more lanes per eigenvalue share the SIMDs and gain fewer bits per unit of time).
+  {
+    const int v = lane / 3, g = lane - 3 * v, slot = wv * 21 + v;
+    const bool act = v < 21 && slot < n;
+    if (__any(act)) {
+      double lo = 0.0, hi = 0.0;
+      int s = 0, t = 0, li = 0;
       if (act) {
-        double nlo = lo, nhi = hi;
-        for (int q = 0; q < G; ++q) {
-          const double x = fma(wd, (double)(q + 1), lo);
-          if (cb[slot * G + q] <= li)
-            nlo = fmax(nlo, x);
-          else
-            nhi = fmin(nhi, x);
+        s = sh.bs[slot];
+        t = sh.bt[slot];
+        li = slot - s;
+        lo = 1e300;
+        hi = -1e300;
+        for (int j = s; j < t; ++j) {
+          const double r = (j > s ? fabs(sh.e[j - 1]) : 0.0) + fabs(sh.e[j]);
+          lo = fmin(lo, sh.d[j] - r);
+          hi = fmax(hi, sh.d[j] + r);
         }
-        lo = nlo;
-        hi = nhi;
+        const double span = fmax(hi - lo, EPS);
+        lo -= 1e-12 * span;
+        hi += 1e-12 * span;
       }
+      for (int r = 0; r < 25; ++r) {
+        const double wd = 0.25 * (hi - lo);
+        const int c = act ? sturm_count(sh.de, s, t, fma(wd, (double)(g + 1), lo)) : 0;
+        const unsigned long long m = __ballot(act && c <= li);
+        const int below = __popcll((m >> (lane - g)) & 7ull);
+        lo = fma(wd, (double)below, lo);
+        hi = lo + wd;
+      }
+      if (act && g == 0) sh.lam[slot] = 0.5 * (lo + hi);
     }
-    if (act && g == 0) sh.lam[slot] = 0.5 * (lo + hi);
   }
   __syncthreads();
   // wanted vectors: every slot when nvec = n; else the slots whose multisection value ranks below
-  // nvec (ties by slot)
+  // nvec (ties by slot), and the rest of their clusters
+  const double ctol = CLUSTER;
   for (int i = tid; i < n; i += nt) {
     int r = 0;
     if (nvec < n)
@@ -403,102 +516,103 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
   // ---- 4. eigenvectors of T (column `slot` of Z holds the block's rows) ----
   for (int idx = tid; idx < n * n; idx += nt) Z[(idx / n) * S + idx % n] = 0.0;
   __syncthreads();
-  {
-    const double tiny = EPS * sh.norm, ctol = 1e-8 * sh.norm;
-    const int slot = tid;
-    if (slot < n) {
-      const int s = sh.bs[slot], t = sh.bt[slot];
-      const bool leader = slot == s || sh.lam[slot] - sh.lam[slot - 1] >= ctol;
-      int last = slot;
-      bool want = false;
-      if (leader) {
-        while (last + 1 < t && sh.lam[last + 1] - sh.lam[last] < ctol) ++last;
-        for (int a = slot; a <= last; ++a) want = want || sh.need[a];
-        if (!want)
-          for (int a = slot; a <= last; ++a) sh.rq[a] = sh.lam[a];  // not refined: no vector
+  // 16 vectors a wave: lanes of one wave read neighbouring columns
+  const int slot = (tid >> 6) * 16 + lane;
+  const bool vact = lane < 16 && slot < n;
+  int bs = 0, bt = 0;
+  bool want = false;
+  if (vact) {
+    bs = sh.bs[slot];
+    bt = sh.bt[slot];
+    // the cluster's slots: neighbours closer than ctol
+    int a = slot, b = slot;
+    while (a > bs && sh.lam[a] - sh.lam[a - 1] < ctol) --a;
+    while (b + 1 < bt && sh.lam[b + 1] - sh.lam[b] < ctol) ++b;
+    for (int q = a; q <= b; ++q) want = want || sh.need[q];
+  }
+  // Orthonormalises the vectors of each cluster of two or more (a wave per cluster), in slot order
+  auto orthogonalise = [&](int passes) {
+    for (int a = wv; a < n; a += nw) {
+      const int s = sh.bs[a], t = sh.bt[a];
+      if (a > s && sh.lam[a] - sh.lam[a - 1] < ctol) continue;  // not a cluster's first
+      int last = a;
+      while (last + 1 < t && sh.lam[last + 1] - sh.lam[last] < ctol) ++last;
+      if (last == a) continue;
+      bool any = false;
+      for (int q = a; q <= last; ++q) any = any || sh.need[q];
+      if (!any) continue;
+      const int i0 = s + lane, i1 = s + lane + 64;
+      for (int p = a; p <= last; ++p) {
+        double y0 = i0 < t ? Z[i0 * S + p] * sh.nv[p] : 0.0, y1 = i1 < t ? Z[i1 * S + p] * sh.nv[p] : 0.0;
+        for (int pass = 0; pass < passes; ++pass)
+          for (int b = a; b < p; ++b) {
+            const double z0 = i0 < t ? Z[i0 * S + b] : 0.0, z1 = i1 < t ? Z[i1 * S + b] : 0.0;
+            const double dp = wave_sum(fma(y0, z0, y1 * z1));
+            y0 = fma(-dp, z0, y0);
+            y1 = fma(-dp, z1, y1);
+          }
+        const double in = 1.0 / sqrt(wave_sum(fma(y0, y0, y1 * y1)));
+        if (i0 < t) Z[i0 * S + p] = y0 * in;
+        if (i1 < t) Z[i1 * S + p] = y1 * in;
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) sh.nv[p] = 1.0;
       }
-      if (leader && want) {
-        for (int a = slot; a <= last; ++a) {
-          if (t - s == 1) {
-            Z[s * S + a] = 1.0;
-            sh.rq[a] = sh.d[s];
-            continue;
-          }
-          ldl_pivots(sh.d, sh.e2, s, t, sh.lam[a], tiny, A, S, a);
-          for (int i = s; i < t; ++i) Z[i * S + a] = start_entry(a, i);
-          for (int it = 0; it < 3; ++it) {
-            col_scale4(Z + a, S, s, t, 1.0 / sqrt(col_norm2(Z, S, s, t, a)));
-            ldl_solve(sh.e, s, t, A, Z, S, a);
-            for (int b = slot; b < a; ++b) {
-              const double dp = col_dot4(Z + b, Z + a, S, s, t);
-              for (int i = s; i < t; ++i) Z[i * S + a] = fma(-dp, Z[i * S + b], Z[i * S + a]);
-            }
-          }
-          col_scale4(Z + a, S, s, t, 1.0 / sqrt(col_norm2(Z, S, s, t, a)));
-          // Rayleigh quotient z^T T z = sum_i d_i z_i^2 + 2 sum_i e_i z_i z_i+1 (the eigenvalue to
-          // ~eps |T|), 4 partial sums
-          double q0 = 0.0, q1 = 0.0, q2 = 0.0, q3 = 0.0;
-          {
-            const double* z = Z + a;
-            int i = s;
-            for (; i + 4 <= t; i += 4) {
-              const double z0 = z[i * S], z1 = z[(i + 1) * S], z2 = z[(i + 2) * S], z3 = z[(i + 3) * S];
-              const double z4 = i + 4 < t ? z[(i + 4) * S] : 0.0;
-              q0 = fma(z0, fma(sh.d[i], z0, 2.0 * sh.e[i] * z1), q0);
-              q1 = fma(z1, fma(sh.d[i + 1], z1, 2.0 * sh.e[i + 1] * z2), q1);
-              q2 = fma(z2, fma(sh.d[i + 2], z2, 2.0 * sh.e[i + 2] * z3), q2);
-              q3 = fma(z3, fma(sh.d[i + 3], z3, i + 4 < t ? 2.0 * sh.e[i + 3] * z4 : 0.0), q3);
-            }
-            for (; i < t; ++i) {
-              const double zi = z[i * S];
-              q0 = fma(zi, fma(sh.d[i], zi, i + 1 < t ? 2.0 * sh.e[i] * z[(i + 1) * S] : 0.0), q0);
-            }
-          }
-          sh.rq[a] = (q0 + q1) + (q2 + q3);
-        }
-      }
+    }
+  };
+  const double rmax = 1.0 / (EPS * 2.0);
+  if (vact) {
+    sh.nv[slot] = 1.0;
+    if (want) {
+      if (bt - bs == 1)
+        Z[bs * S + slot] = 1.0;
+      else
+        sh.nv[slot] = 1.0 / sqrt(ldl_solve<true>(sh.d, sh.e, bs, bt, sh.lam[slot], rmax, A, Z, S, slot, 1.0));
     }
   }
   __syncthreads();
-  // ---- 5. sort ascending (rank; ties by slot), permute columns through A, back-transform ----
+  orthogonalise(1);
+  __syncthreads();
+  if (vact && want && bt - bs > 1)
+    sh.nv[slot] =
+        1.0 / sqrt(ldl_solve<false>(sh.d, sh.e, bs, bt, sh.lam[slot], rmax, A, Z, S, slot, sh.nv[slot]));
+  __syncthreads();
+  orthogonalise(2);
+  __syncthreads();
+  // Rayleigh quotients z^T T z / z^T z (the eigenvalue to ~eps |T|): four lanes per vector
+  {
+    const int c = tid >> 2, q4 = tid & 3;
+    double num = 0.0, den = 0.0;
+    if (c < n) {
+      for (int i = q4; i < n; i += 4) {
+        const double zi = Z[i * S + c], zn = i + 1 < n ? Z[(i + 1) * S + c] : 0.0;
+        num = fma(zi, fma(sh.d[i], zi, 2.0 * sh.e[i] * zn), num);
+        den = fma(zi, zi, den);
+      }
+    }
+    num = group4_sum(num);
+    den = group4_sum(den);
+    if (c < n && q4 == 0) {
+      sh.rq[c] = (den > 0.0 ? num / den : sh.lam[c]) * unscale;  // no vector: the multisection value
+      sh.nv[c] = den > 0.0 ? 1.0 / sqrt(den) : 0.0;
+    }
+  }
+  __syncthreads();
+  // ---- 5. sort ascending (rank; ties by slot), back-transform ----
   for (int i = tid; i < n; i += nt) {
     int r = 0;
     for (int j = 0; j < n; ++j) r += (sh.rq[j] < sh.rq[i]) || (sh.rq[j] == sh.rq[i] && j < i);
     sh.perm[r] = i;
+    w[r] = sh.rq[i];
   }
   __syncthreads();
-  // permuted copy through global scratch (f + n^2); reflectors back into A's strict lower part
-  double* g = f + (size_t)n * n;
-  for (int idx = tid; idx < n * n; idx += nt) {
-    const int i = idx / n, c = idx % n;
-    g[idx] = Z[i * S + sh.perm[c]];
-    if (i > c) A[i * S + c] = f[idx];
-  }
-  for (int i = tid; i < n; i += nt) w[i] = sh.rq[sh.perm[i]];
-  __syncthreads();
-  for (int idx = tid; idx < n * n; idx += nt) Z[(idx / n) * S + idx % n] = g[idx];
-  __syncthreads();
-  for (int k = n - 3; k >= 0; --k) {
-    const int m = n - k - 1;
-    const double* vk = A + (size_t)(k + 1) * S + k;  // v_i = vk[i * S]
-    // sh.lo[c] = v^T Z[k+1:, c], one thread per column
-    if (grp < nvec) {
-      double acc = 0.0;
-      for (int i = sub; i < m; i += 8) acc = fma(vk[i * S], Z[(size_t)(k + 1 + i) * S + grp], acc);
-      acc = group8_sum(acc);
-      if (sub == 0) sh.lo[grp] = acc;
-    }
-    __syncthreads();
-    const int c0 = lane, c1 = lane + 64;
-    const double s0 = c0 < nvec ? 2.0 * sh.lo[c0] : 0.0, s1 = c1 < nvec ? 2.0 * sh.lo[c1] : 0.0;
-    for (int i = wv; i < m; i += nw) {
-      const double vi = vk[i * S];
-      double* row = Z + (size_t)(k + 1 + i) * S;
-      if (c0 < nvec) row[c0] -= vi * s0;
-      if (c1 < nvec) row[c1] -= vi * s1;
-    }
-    __syncthreads();
-  }
+  if (n <= 16)
+    back_transform<2>(n, nvec, A, Z, S, f, sh);
+  else if (n <= 32)
+    back_transform<4>(n, nvec, A, Z, S, f, sh);
+  else if (n <= 64)
+    back_transform<8>(n, nvec, A, Z, S, f, sh);
+  else
+    back_transform<12>(n, nvec, A, Z, S, f, sh);
 }
 
 }  // namespace qexeig

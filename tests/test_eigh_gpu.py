@@ -131,3 +131,21 @@ def test_degen_eigh_autograd():
     loss.backward()
     ref = otd.degen_eigh_bwd(w.detach().cpu().numpy(), v.detach().cpu().numpy(), c, G, exact=True)
     np.testing.assert_allclose(A.grad.cpu().numpy(), ref, rtol=0, atol=1e-11 * max(1.0, np.abs(ref).max()))
+
+
+@pytest.mark.parametrize("n", [4, 8, 9, 15, 17, 31, 32, 33, 63, 64, 65, 79, 81, 95])
+def test_register_patch_edges(geigh, n):
+    """Sizes at the edges of the register patches (8 columns, 32 rows) and of the size classes; a random
+    spectrum, one with 3 levels of multiplicity n / 3, a graded one and a shifted glued-Wilkinson-like
+    tridiagonal with pairs closer than the cluster threshold, at norms 1, 1e-30 and 1e30."""
+    rng = np.random.default_rng(100 + n)
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    M = rng.standard_normal((n, n))
+    lv = Q @ np.diag(np.repeat([-1.0, 0.5, 2.0], (n + 2) // 3)[:n]) @ Q.T
+    gr = Q @ np.diag(np.geomspace(1e-12, 1.0, n)) @ Q.T
+    wk = np.diag(np.abs(np.arange(n) - (n - 1) / 2)) + np.diag(np.ones(n - 1), 1) + np.diag(np.ones(n - 1), -1)
+    for f in (1.0, 1e-30, 1e30):
+        As = np.stack([f * 0.5 * (X + X.T) for X in (M, lv, gr, wk)])
+        w, v = geigh(As, np.broadcast_to(np.eye(n), As.shape).copy())
+        for k in range(len(As)):
+            _check(w[k].cpu().numpy() / f, v[k].cpu().numpy(), As[k] / f, np.eye(n))
