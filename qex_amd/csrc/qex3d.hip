@@ -1665,84 +1665,59 @@ __global__ __launch_bounds__(NT) void k_coulomb(int n, int npair, const double* 
 }
 
 // ---------------------------------------------------------------------------------------------
-// small dense linear algebra in one workgroup (row-major n x n in global memory, n <= 128)
+// small dense linear algebra in one workgroup (row-major n x n, n <= 96)
 // ---------------------------------------------------------------------------------------------
-// C = op(A) op(B) (+ beta C); ta/tb transpose flags
-__device__ void mm(int n, const double* A, bool ta, const double* B, bool tb, double* C, double alpha, double beta) {
-  for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) {
-    const int i = idx / n, j = idx % n;
-    double s = 0.0;
-    for (int k = 0; k < n; ++k) {
-      const double a = ta ? A[k * n + i] : A[i * n + k];
-      const double b = tb ? B[j * n + k] : B[k * n + j];
-      s = fma(a, b, s);
-    }
-    C[idx] = alpha * s + (beta != 0.0 ? beta * C[idx] : 0.0);
-  }
-  __syncthreads();
-}
-
-__device__ double dot_all(int len, const double* a, const double* b, double* red) {
-  double s = 0.0;
-  for (int t = threadIdx.x; t < len; t += blockDim.x) s = fma(a[t], b[t], s);
-  return bsum(s, red);
-}
-
 // C[M x N] = alpha op(A) op(B), K the inner dimension, on FP64 matrix cores: one 16 x 16 output
 // tile per wave at a time (lane l supplies A[l%16][l/16] and B[l/16][l%16] of each 16 x 4 x 16
-// step and receives C[4v + l/16][l%16] in element v).  Operands in LDS or global memory.
-__device__ void mfma_gemm(int M, int N, int K, const double* A, int lda, bool ta, const double* B, int ldb, bool tb,
-                          double* C, int ldc, double alpha) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int mb = (M + 15) / 16, nb = (N + 15) / 16;
+// step and receives C[4v + l/16][l%16] in element v).  Operands in LDS or global memory (glob / lds
+// below), row-major or, with T, transposed.  The matrices are at most 96 wide and come from L2, so the
+// time is load latency: GEMM_U steps' operands are in flight together, read from clamped addresses
+// and zeroed past K instead of behind branches (n = 80, one workgroup: see k_scf_fock).
+typedef const __attribute__((address_space(1))) double* gptr_t;
+typedef const __attribute__((address_space(3))) double* lptr_t;
+template <class P>
+struct Mat {
+  P p;
+  int sr, sk;  // strides of op's row (A) or column (B) and of the inner dimension
+};
+__device__ __forceinline__ Mat<gptr_t> glob(const double* p, int s_outer, int s_inner) {
+  return {(gptr_t)(uintptr_t)p, s_outer, s_inner};
+}
+__device__ __forceinline__ Mat<lptr_t> lds(const double* p, int s_outer, int s_inner) {
+  return {(lptr_t)p, s_outer, s_inner};
+}
+constexpr int GEMM_U = 8;
+template <class PA, class PB>
+__device__ __forceinline__ void mfma_gemm(int M, int N, int K, Mat<PA> A, Mat<PB> B, double* C, int ldc, double alpha) {
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int mb = (M + 15) / 16, nb = (N + 15) / 16, kl = lane >> 4;
   for (int tile = wv; tile < mb * nb; tile += nw) {
     const int bi = tile / nb, bj = tile % nb;
-    const int r = bi * 16 + (lane & 15), c = bj * 16 + (lane & 15);
+    const int r = min(bi * 16 + (lane & 15), M - 1), c = min(bj * 16 + (lane & 15), N - 1);
+    const PA pa = A.p + r * A.sr;
+    const PB pb = B.p + c * B.sr;
     d4_t acc = (d4_t){0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < K; k0 += 4) {
-      const int k = k0 + (lane >> 4);
-      double a = 0.0, b = 0.0;
-      if (r < M && k < K) a = ta ? A[k * lda + r] : A[r * lda + k];
-      if (c < N && k < K) b = tb ? B[c * ldb + k] : B[k * ldb + c];
-      acc = mfma64(a, b, acc);
+    for (int k0 = 0; k0 < K; k0 += 4 * GEMM_U) {
+      double a[GEMM_U], b[GEMM_U];
+#pragma unroll
+      for (int u = 0; u < GEMM_U; ++u) {
+        const int k = min(k0 + 4 * u + kl, K - 1);
+        a[u] = pa[k * A.sk];
+        b[u] = pb[k * B.sk];
+      }
+#pragma unroll
+      for (int u = 0; u < GEMM_U; ++u) {
+        if (k0 + 4 * u < K) {
+          const bool in = k0 + 4 * u + kl < K;
+          acc = mfma64(in ? a[u] : 0.0, in ? b[u] : 0.0, acc);
+        }
+      }
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int row = bi * 16 + 4 * v + (lane >> 4), col = bj * 16 + (lane & 15);
+      const int row = bi * 16 + 4 * v + kl, col = bj * 16 + (lane & 15);
       if (row < M && col < N) C[row * ldc + col] = alpha * acc[v];
-    }
-  }
-  __syncthreads();
-}
-
-// Cholesky S = L L^T (in place, lower), then X = L^-T (upper): C = X V solves F C = S C e.
-__device__ void orthogonaliser(int n, const double* S, double* L, double* X) {
-  const int NT = blockDim.x;
-  for (int t = threadIdx.x; t < n * n; t += NT) L[t] = S[t];
-  __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    if (threadIdx.x == 0) L[k * n + k] = sqrt(L[k * n + k]);
-    __syncthreads();
-    const double dkk = L[k * n + k];
-    for (int i = k + 1 + threadIdx.x; i < n; i += NT) L[i * n + k] /= dkk;
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < (n - k - 1) * (n - k - 1); idx += NT) {
-      const int i = k + 1 + idx / (n - k - 1), j = k + 1 + idx % (n - k - 1);
-      if (j <= i) L[i * n + j] -= L[i * n + k] * L[j * n + k];
-    }
-    __syncthreads();
-  }
-  for (int t = threadIdx.x; t < n * n; t += NT) {
-    const int i = t / n, j = t % n;
-    if (j > i) L[t] = 0.0;
-  }
-  __syncthreads();
-  // Linv (lower) column by column: Linv[:, c] solves L x = e_c; X = Linv^T
-  for (int c = threadIdx.x; c < n; c += NT) {
-    for (int i = 0; i < n; ++i) {
-      double s = i == c ? 1.0 : 0.0;
-      for (int k = c; k < i; ++k) s -= L[i * n + k] * X[c * n + k];  // X row c holds Linv[:, c]
-      X[c * n + i] = i < c ? 0.0 : s / L[i * n + i];
     }
   }
   __syncthreads();
@@ -1759,7 +1734,6 @@ struct Scf3 {
   const double* S;
   const double* H;
   double* X;   // orthogonaliser
-  double* Lc;  // Cholesky factor of S (scratch)
   int* status_out;
   const double* eri;
   const double* ao;
@@ -1802,8 +1776,8 @@ __global__ __launch_bounds__(NT_SCF) void k_scf_fock(const Scf3* __restrict__ ss
     return;
   }
   // error e = F D S - S D F
-  mfma_gemm(n, n, n, s.F, n, false, s.D, n, false, s.tmp1, n, 1.0);     // FD
-  mfma_gemm(n, n, n, s.tmp1, n, false, s.S, n, false, s.tmp2, n, 1.0);  // FDS
+  mfma_gemm(n, n, n, glob(s.F, n, 1), glob(s.D, 1, n), s.tmp1, n, 1.0);     // FD
+  mfma_gemm(n, n, n, glob(s.tmp1, n, 1), glob(s.S, 1, n), s.tmp2, n, 1.0);  // FDS
   // S D F = (F D S)^T for symmetric F, D, S
   const int cnt = s.ist[2], head = s.ist[3];
   const int slot = head;
@@ -1916,8 +1890,8 @@ __global__ __launch_bounds__(NT_EIG) void k_scf_eigh(const Scf3* __restrict__ ss
   const int n = s.n, nn = n * n, S = n + 1;
   double* A = sm;
   double* Z = A + (size_t)n * S;
-  mfma_gemm(n, n, n, s.Fd, n, false, s.X, n, false, s.tmp1, n, 1.0);  // Fd X
-  mfma_gemm(n, n, n, s.X, n, true, s.tmp1, n, false, A, S, 1.0);      // X^T Fd X (into LDS)
+  mfma_gemm(n, n, n, glob(s.Fd, n, 1), glob(s.X, 1, n), s.tmp1, n, 1.0);  // Fd X
+  mfma_gemm(n, n, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), A, S, 1.0);      // X^T Fd X (into LDS)
   for (int t = threadIdx.x; t < nn; t += blockDim.x) {
     const int i = t / n, j = t % n;
     if (i < j) {
@@ -1928,8 +1902,8 @@ __global__ __launch_bounds__(NT_EIG) void k_scf_eigh(const Scf3* __restrict__ ss
   }
   __syncthreads();
   qexeig::symeig(n, A, Z, S, s.mo, s.eigf, sh, full ? n : s.nocc + 2);
-  mfma_gemm(n, n, n, s.X, n, false, Z, S, false, s.C, n, 1.0);  // C = X Z
-  mfma_gemm(n, n, s.nocc, s.C, n, false, s.C, n, true, s.D, n, 2.0);  // D = 2 C_occ C_occ^T
+  mfma_gemm(n, n, n, glob(s.X, n, 1), lds(Z, 1, S), s.C, n, 1.0);  // C = X Z
+  mfma_gemm(n, n, s.nocc, glob(s.C, n, 1), glob(s.C, n, 1), s.D, n, 2.0);  // D = 2 C_occ C_occ^T
 }
 
 // batched generalized eigh F C = S C e, one workgroup per matrix (scratch: 8 n^2 doubles each)
@@ -1940,10 +1914,11 @@ __global__ __launch_bounds__(NT_EIG) void k_gen_eigh(int n, const double* F, con
   const size_t nn = (size_t)n * n, b = blockIdx.x;
   const int S = n + 1;
   double* w = scratch + b * 8 * nn;
-  double *L = w, *X = w + nn, *t1 = w + 2 * nn, *t2 = w + 3 * nn, *Zg = w + 4 * nn, *f = w + 5 * nn;
-  orthogonaliser(n, Sm + b * nn, L, X);
-  mfma_gemm(n, n, n, F + b * nn, n, false, X, n, false, t1, n, 1.0);
-  mfma_gemm(n, n, n, X, n, true, t1, n, false, t2, n, 1.0);
+  double *X = w, *t1 = w + nn, *t2 = w + 2 * nn, *f = w + 3 * nn;
+  // Cholesky S = L L^T, X = L^-T: C = X V solves F C = S C e
+  qexeig::by_size(n, [&](auto nc) { qexeig::inverse_cholesky<decltype(nc)::value>(n, Sm + b * nn, X, sh); });
+  mfma_gemm(n, n, n, glob(F + b * nn, n, 1), glob(X, 1, n), t1, n, 1.0);
+  mfma_gemm(n, n, n, glob(X, 1, n), glob(t1, 1, n), t2, n, 1.0);
   double* A = sm;
   double* Z = A + (size_t)n * S;
   for (int t = threadIdx.x; t < (int)nn; t += blockDim.x) {
@@ -1952,8 +1927,7 @@ __global__ __launch_bounds__(NT_EIG) void k_gen_eigh(int n, const double* F, con
   }
   __syncthreads();
   qexeig::symeig(n, A, Z, S, mo + b * n, f, sh);
-  mfma_gemm(n, n, n, X, n, false, Z, S, false, C + b * nn, n, 1.0);
-  (void)Zg;
+  mfma_gemm(n, n, n, glob(X, n, 1), lds(Z, 1, S), C + b * nn, n, 1.0);
 }
 
 // Reverse pass of the symmetric eigendecomposition A = V diag(w) V^T with degenerate pairs masked
@@ -1971,7 +1945,7 @@ __global__ __launch_bounds__(NT_VJP) void k_eigh_vjp(int n, const double* w, con
   double* T = M + nn;
   double* G = gA + b * nn;
   const bool ut = exact != 0;  // U = V^T: op(U) reads V transposed
-  if (gv) mfma_gemm(n, n, n, V, n, ut, gv + b * nn, n, false, M, n, 1.0);  // U gV
+  if (gv) mfma_gemm(n, n, n, glob(V, ut ? 1 : n, ut ? n : 1), glob(gv + b * nn, 1, n), M, n, 1.0);  // U gV
   const double thr = 4.05381695970951e-10;  // float64 eps^0.6, eps = 2^-52
   for (size_t t = threadIdx.x; t < nn; t += blockDim.x) {
     const int i = (int)(t / n), j = (int)(t % n);
@@ -1981,8 +1955,8 @@ __global__ __launch_bounds__(NT_VJP) void k_eigh_vjp(int n, const double* w, con
     M[t] = m;
   }
   __syncthreads();
-  mfma_gemm(n, n, n, M, n, false, V, n, ut, T, n, 1.0);  // M U
-  mfma_gemm(n, n, n, V, n, false, T, n, false, G, n, 1.0);  // V M U
+  mfma_gemm(n, n, n, glob(M, n, 1), glob(V, ut ? n : 1, ut ? 1 : n), T, n, 1.0);  // M U
+  mfma_gemm(n, n, n, glob(V, n, 1), glob(T, 1, n), G, n, 1.0);  // V M U
   for (size_t t = threadIdx.x; t < nn; t += blockDim.x) {
     const int i = (int)(t / n), j = (int)(t % n);
     if (i < j) {
@@ -2026,9 +2000,9 @@ __global__ __launch_bounds__(NT_SCF) void k_scf_energy(const Scf3* __restrict__ 
     s.F[t] = f;
   }
   __syncthreads();
-  mfma_gemm(n, nocc, n, s.F, n, false, s.C, n, false, s.tmp1, n, 1.0);    // tmp1 = F C_occ   (n x nocc)
-  mfma_gemm(n, nocc, n, s.X, n, true, s.tmp1, n, false, s.tmp2, n, 1.0);  // tmp2 = X^T F C_occ
-  mfma_gemm(nocc, nocc, n, s.C, n, true, s.tmp1, n, false, s.Cp, n, 1.0); // Cp = C_occ^T F C_occ
+  mfma_gemm(n, nocc, n, glob(s.F, n, 1), glob(s.C, 1, n), s.tmp1, n, 1.0);    // tmp1 = F C_occ   (n x nocc)
+  mfma_gemm(n, nocc, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), s.tmp2, n, 1.0);  // tmp2 = X^T F C_occ
+  mfma_gemm(nocc, nocc, n, glob(s.C, 1, n), glob(s.tmp1, 1, n), s.Cp, n, 1.0); // Cp = C_occ^T F C_occ
   double a = 0.0, b = 0.0;
   for (int t = threadIdx.x; t < n * nocc; t += NT_SCF) {
     const double v = s.tmp2[(t / nocc) * n + t % nocc];
@@ -2073,18 +2047,12 @@ __global__ __launch_bounds__(NT) void k_scf_init(const Scf3* __restrict__ ss) {
   }
 }
 
-// Cholesky and triangular inverse on LDS copies (2 n^2 doubles of dynamic LDS), X written out
-__global__ __launch_bounds__(NT_SCF) void k_scf_orthogonaliser(const Scf3* __restrict__ ss) {
-  extern __shared__ double sm[];
+// X = L^-T of S = L L^T
+constexpr int NT_ORTH = 256;
+__global__ __launch_bounds__(NT_ORTH) void k_scf_orthogonaliser(const Scf3* __restrict__ ss) {
+  __shared__ qexeig::Smem sh;
   const Scf3 s = ss[blockIdx.x];
-  const int nn = s.n * s.n;
-  double* Ls = sm;
-  double* Xs = sm + nn;
-  orthogonaliser(s.n, s.S, Ls, Xs);
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    s.X[t] = Xs[t];
-    s.Lc[t] = Ls[t];
-  }
+  qexeig::by_size(s.n, [&](auto nc) { qexeig::inverse_cholesky<decltype(nc)::value>(s.n, s.S, s.X, sh); });
 }
 
 // fill e_hist beyond the last cycle with the final energy (frozen state repeats); status out
@@ -3229,7 +3197,6 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     s.ao32 = ins[b].ao_f32;
     s.prec = p->method == QEX3D_RHF ? QEX3D_PRECISION_FP64 : p->precision;
     s.x32blk = x32_blocks(ng);
-    s.Lc = (double*)(w + L.total);
     s.X = (double*)(w + L.total + al((size_t)n * n * 8));
     s.status_out = outs[b].status;
     s.F = (double*)(w + L.F);
@@ -3378,11 +3345,7 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
   per_mol(qexprof::K_OTHER, k_scf_init);
   {
     qexprof::Scope ps_(qexprof::K_OTHER, st);
-    const size_t lds_o = (size_t)2 * nmax * nmax * 8;
-    if (lds_o > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)k_scf_orthogonaliser, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds_o);
-    hipLaunchKernelGGL(k_scf_orthogonaliser, dim3(nb), dim3(NT_SCF), lds_o, st, dss);
+    hipLaunchKernelGGL(k_scf_orthogonaliser, dim3(nb), dim3(NT_ORTH), 0, st, dss);
   }
   per_mol_wide(qexprof::K_FOCK, k_scf_fock, -1);
   eigh(0);

@@ -1,22 +1,22 @@
 // symeig.h -- dense symmetric eigensolver for one workgroup (n <= 96, FP64).
 //
-//   1. Householder tridiagonalisation with the matrix in registers (256 threads, each a cyclic
-//      patch): for k = 0..n-3 the reflector H_k = I - tau v v^T annihilates column k below the
-//      subdiagonal; the trailing block becomes A - v w^T - w v^T with p = tau A v,
-//      w = p - (tau / 2)(v^T p) v.  The rows v_k go to global scratch, d / e collect the tridiagonal.
+//   1. Householder tridiagonalisation with the matrix in registers (each thread a cyclic patch): for
+//      k = 0..n-3 the reflector H_k = I - tau v v^T annihilates column k below the subdiagonal; the
+//      trailing block becomes A - v w^T - w v^T with p = tau A v, w = p - (tau / 2)(v^T p) v.  d / e collect
+//      the tridiagonal.
 //   2. T, scaled by a power of two to norm 1..2, splits into unreduced blocks where
 //      |e_k| <= eps (|d_k| + |d_k+1|).
 //   3. Eigenvalues: multisection on Sturm counts (sign changes of the leading minors of T - x), three
-//      lanes per eigenvalue, a fixed number of rounds (interval / 4 per round).
+//      lanes per eigenvalue, a fixed number of rounds (interval / 7 per round).
 //   4. Eigenvectors of T: two inverse iterations (LDL^T pivots of T - lam, pivots smaller than
-//      eps |T| replaced by +-eps |T|) from a fixed pseudo-random start, one lane per vector; eigenvalues
+//      eps |T| replaced by +-eps |T|) from a fixed pseudo-random start, two lanes per vector; eigenvalues
 //      of one block closer than 1e-5 |T| form a cluster, whose vectors are orthogonalised after every
 //      solve.  Rayleigh quotients give the eigenvalues.
 //   5. Ascending sort and back-transformation Z <- H_0 ... H_{n-3} Y, four lanes per column.
 // All reductions run in a fixed order: the result does not depend on timing.
 //
 // What bounds it: every stage is a chain of dependent steps of one workgroup, so its time is
-// barriers and latencies, not arithmetic.  Hence the matrix stays in registers (two barriers and a
+// barriers and latencies, not arithmetic.  Hence the matrix stays in registers (one barrier and a
 // few LDS words per Householder step; the LDS-resident form took three barriers over 16 waves and
 // re-read the block), the counts need no reciprocal and no barrier, and a column of the
 // back-transformation stays in four lanes' registers from the first reflector to the last.
@@ -60,7 +60,10 @@ __device__ __forceinline__ double read_lane(double x, int l) {
 
 // Sum over the 64 lanes (all active), the same value in every lane: DPP within each row of 16
 // lanes (pairs, quads, half-row mirror, row mirror), then the four row sums in a fixed order.
+// No contraction in these sums: a product fused into its lane's first addition, but rounded on its way to
+// the neighbour, would make the lanes' sums differ.
 __device__ __forceinline__ double wave_sum(double x) {
+#pragma clang fp contract(off)
   x += dpp_f64<0xB1>(x);   // quad_perm [1, 0, 3, 2]
   x += dpp_f64<0x4E>(x);   // quad_perm [2, 3, 0, 1]
   x += dpp_f64<0x141>(x);  // row_half_mirror
@@ -78,11 +81,13 @@ __device__ __forceinline__ double wave_max(double x) {
 
 // sum over an aligned group of 4 / 8 lanes, the same value in each of them
 __device__ __forceinline__ double group4_sum(double x) {
+#pragma clang fp contract(off)
   x += dpp_f64<0xB1>(x);
   x += dpp_f64<0x4E>(x);
   return x;
 }
 __device__ __forceinline__ double group8_sum(double x) {
+#pragma clang fp contract(off)
   x = group4_sum(x);
   x += dpp_f64<0x141>(x);
   return x;
@@ -91,7 +96,7 @@ __device__ __forceinline__ double group8_sum(double x) {
 // Shared state of the solver (static LDS besides the two n x S matrices).
 struct Smem {
   double d[MAXN], e[MAXN], lam[MAXN], rq[MAXN], tau[MAXN], nv[MAXN];
-  double x[MAXN + 8], p[MAXN + 8];   // column being reduced; p = tau A v
+  double p[2][MAXN + 40], col[2][MAXN + 40];  // exchanged per step (alternating): p = tau A v and a column of A
   double2 de[MAXN + 8];              // (d_i, e_{i-1}^2) for the Sturm counts
   int bs[MAXN], bt[MAXN], perm[MAXN];
   unsigned long long cut[2];
@@ -104,35 +109,55 @@ __device__ __forceinline__ double rcp_nr(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
-// Number of eigenvalues of rows s..t-1 of T below x: the sign changes of the leading minors
-// p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}.  No division, so a row is one dependent FMA (a pivot
-// recurrence needs a reciprocal, a Newton step and two clamps in the chain: 60 cycles a row against
-// 16).  T is scaled to norm 1..2 and e^2 floored at 1e-60, so 8 rows change a minor by less than
-// 1e-250 .. 1e6 and both minors never vanish together; they are rescaled by a power of two every 8 rows.
-__device__ __forceinline__ int sturm_count(const double2* de, int s, int t, double x) {
+// Running minors of T - x, p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, whose sign changes count the
+// eigenvalues below x.  No division, so a row is one dependent FMA (a pivot recurrence has a reciprocal, a
+// Newton step and two clamps in the chain).  T is scaled to norm 1..2 and e^2 floored at 1e-60, so 8 rows
+// change a minor by less than 1e-250 .. 1e6 and two neighbouring minors never vanish together;
+// rescale() divides both by a power of two every 8 rows.
+struct Minors {
   double p0 = 0.0, p1 = 1.0;
-  unsigned bits = 0, c = 0;
-  auto step = [&](double2 v) {
-    const double pn = fma(v.x - x, p1, -(v.y * p0));
+  unsigned bits = 0;
+  __device__ __forceinline__ void step(double2 de, double x) {
+    const double pn = fma(de.x - x, p1, -(de.y * p0));
     p0 = p1;
     p1 = pn;
     bits = __builtin_amdgcn_alignbit(bits, (unsigned)__double2hiint(pn), 31);  // bits << 1 | sign
-  };
+  }
+  // sign changes of the last m <= 16 rows
+  __device__ __forceinline__ int changes(int m) const { return __popc((bits ^ (bits >> 1)) & ((1u << m) - 1u)); }
+  __device__ __forceinline__ void rescale() {
+    const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+    p0 = ldexp(p0, ex);
+    p1 = ldexp(p1, ex);
+  }
+};
+
+// eigenvalues of rows s..t-1 of T below x and below y, (d_i, e_{i-1}^2) in LDS.  Two shifts a lane: one leaves
+// the pipeline idle between dependent operations and reads LDS for half the arithmetic.
+__device__ __forceinline__ int2 sturm_count2(const double2* de, int s, int t, double x, double y) {
+  Minors m, l;
+  int2 c = make_int2(0, 0);
   int j = s;
   for (; j + 8 <= t; j += 8) {
     double2 v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = de[j + u];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) step(v[u]);
-    c += __popc((bits ^ (bits >> 1)) & 0xFFu);
-    const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
-    p0 = ldexp(p0, ex);
-    p1 = ldexp(p1, ex);
+    for (int u = 0; u < 8; ++u) {
+      m.step(v[u], x);
+      l.step(v[u], y);
+    }
+    c.x += m.changes(8);
+    c.y += l.changes(8);
+    m.rescale();
+    l.rescale();
   }
   const int left = t - j;
-  for (; j < t; ++j) step(de[j]);
-  return (int)(c + __popc((bits ^ (bits >> 1)) & ((1u << left) - 1u)));
+  for (; j < t; ++j) {
+    m.step(de[j], x);
+    l.step(de[j], y);
+  }
+  return make_int2(c.x + m.changes(left), c.y + l.changes(left));
 }
 
 // deterministic start vector entry in [-1, 1)
@@ -144,21 +169,25 @@ __device__ __forceinline__ double start_entry(int slot, int i) {
   return (double)(x & 0xFFFFFF) / 8388608.0 - 1.0;
 }
 
-// One thread: column `col` of Y <- (T_block - lam)^-1 b, rows s..t-1, with the inverse pivots 1/D_i
-// of T_block - lam (|1/D| <= rmax) in column `col` of Dm.  FIRST: b is the start vector, and the
-// pivots are computed along with the forward solve; else b = scale * Y and the pivots are read.
-// Returns |x|^2.  The operands of 8 rows are in flight per LDS wait.
+// A pair of lanes: column `col` of Y <- (T_block - lam)^-1 b, rows s..t-1.  The even lane eliminates from
+// the top, the odd one (bot) from the bottom, to the row h = (s + t) / 2, which they solve together; each
+// then substitutes back outward over its own half (half the dependent chain of a one-sided solve).  The
+// inverse pivots 1/D_i (|1/D| <= rmax) are kept in column `col` of Dm.  FIRST: b is the start vector, and the
+// pivots are computed along with the elimination; else b = scale * Y and the pivots are read.  Returns
+// |x|^2 in both lanes.  The operands of 8 rows are in flight per LDS wait.
 template <bool FIRST>
-__device__ __forceinline__ double ldl_solve(const double* d, const double* e, int s, int t, double lam, double rmax,
-                                            double* Dm, double* Y, int S, int col, double scale) {
+__device__ __forceinline__ double ldl_solve(const double* d, const double* e, int s, int t, bool bot, double lam,
+                                            double rmax, double* Dm, double* Y, int S, int col, double scale) {
+  const int h = (s + t) >> 1, m = bot ? t - 1 - h : h - s;  // rows of this side
+  const int i0 = bot ? t - 1 : s, st = bot ? -1 : 1;
+  const double* ec = bot ? e - 1 : e;  // ec[i] couples row i to its neighbour toward h
   double y = 0.0, qi = 0.0, ep = 0.0;
   auto fwd = [&](int i, double di, double ei, double bi, double ri) {
-    // row i: l = e_{i-1} / D_{i-1}; D_i = d_i - lam - e_{i-1} l; y_i = b_i - l y_{i-1}
+    // l = e / D of the row before; D_i = d_i - lam - e l; y_i = b_i - l y
     const double l = ep * qi;
     y = fma(-l, y, bi);
     if (FIRST) {
-      const double q = fma(-ep, l, di - lam);
-      qi = fmin(fmax(rcp_nr(q), -rmax), rmax);
+      qi = fmin(fmax(rcp_nr(fma(-ep, l, di - lam)), -rmax), rmax);
       Dm[i * S + col] = qi;
     } else {
       qi = ri;
@@ -166,111 +195,124 @@ __device__ __forceinline__ double ldl_solve(const double* d, const double* e, in
     Y[i * S + col] = y;
     ep = ei;
   };
-  int i = s;
-  for (; i + 8 <= t; i += 8) {
+  int k = 0;
+  for (; k + 8 <= m; k += 8) {
     double dv[8], ev[8], bv[8], rv[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      ev[u] = e[i + u];
-      if (FIRST) {
-        dv[u] = d[i + u];
-        bv[u] = start_entry(col, i + u);
-        rv[u] = 0.0;
-      } else {
-        dv[u] = 0.0;
-        bv[u] = scale * Y[(i + u) * S + col];
-        rv[u] = Dm[(i + u) * S + col];
-      }
+      const int i = i0 + st * (k + u);
+      ev[u] = ec[i];
+      dv[u] = FIRST ? d[i] : 0.0;
+      bv[u] = FIRST ? start_entry(col, i) : scale * Y[i * S + col];
+      rv[u] = FIRST ? 0.0 : Dm[i * S + col];
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) fwd(i + u, dv[u], ev[u], bv[u], rv[u]);
+    for (int u = 0; u < 8; ++u) fwd(i0 + st * (k + u), dv[u], ev[u], bv[u], rv[u]);
   }
-  for (; i < t; ++i)
-    fwd(i, d[i], e[i], FIRST ? start_entry(col, i) : scale * Y[i * S + col], FIRST ? 0.0 : Dm[i * S + col]);
-  // x_i = y_i / D_i - (e_i / D_i) x_{i+1}; e_{t-1} = 0 at a block's end
-  double x = 0.0, n0 = 0.0;
-  i = t - 1;
-  for (; i - 7 >= s; i -= 8) {
-    double yv[8], rv[8], lv[8];
+  for (; k < m; ++k) {
+    const int i = i0 + st * k;
+    fwd(i, FIRST ? d[i] : 0.0, ec[i], FIRST ? start_entry(col, i) : scale * Y[i * S + col], FIRST ? 0.0 : Dm[i * S + col]);
+  }
+  // row h, in both lanes (a side without rows contributes l = 0)
+  const double l = ep * qi, el = ep * l, ly = l * y;
+  const double elo = dpp_f64<0xB1>(el), lyo = dpp_f64<0xB1>(ly);
+  const double bh = FIRST ? start_entry(col, h) : scale * Y[h * S + col];
+  const double qh = FIRST ? fmin(fmax(rcp_nr((d[h] - lam) - (bot ? elo + el : el + elo)), -rmax), rmax) : Dm[h * S + col];
+  double x = (bh - (bot ? lyo + ly : ly + lyo)) * qh;
+  double n0 = bot ? 0.0 : x * x;
+  if (!bot) {
+    if (FIRST) Dm[h * S + col] = qh;
+    Y[h * S + col] = x;
+  }
+  // outward: x_i = y_i / D_i - (e / D_i) x of the row toward h
+  k = m - 1;
+  for (; k - 7 >= 0; k -= 8) {
+    double yv[8], lv[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      rv[u] = Dm[(i - u) * S + col];
-      yv[u] = Y[(i - u) * S + col] * rv[u];
-      lv[u] = e[i - u] * rv[u];
+      const int i = i0 + st * (k - u);
+      const double r = Dm[i * S + col];
+      yv[u] = Y[i * S + col] * r;
+      lv[u] = ec[i] * r;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       x = fma(-lv[u], x, yv[u]);
       n0 = fma(x, x, n0);
-      Y[(i - u) * S + col] = x;
+      Y[(i0 + st * (k - u)) * S + col] = x;
     }
   }
-  for (; i >= s; --i) {
+  for (; k >= 0; --k) {
+    const int i = i0 + st * k;
     const double r = Dm[i * S + col];
-    x = fma(-(e[i] * r), x, Y[i * S + col] * r);
+    x = fma(-(ec[i] * r), x, Y[i * S + col] * r);
     n0 = fma(x, x, n0);
     Y[i * S + col] = x;
   }
-  return n0;
+  return n0 + dpp_f64<0xB1>(n0);
 }
 
-// Householder tridiagonalisation of A (n x n in LDS, row stride S; only read).  NC >= ceil(n / 8).
-// Threads 0..255: thread (r, c) = (tid / 8, tid % 8) holds A[r + 32 i][c + 8 j] in registers; the other
-// waves only take part in the barriers.  32 x 8 rather than 16 x 16: row sums then cross 8 lanes (three
-// DPP steps for 3 rows) instead of 16 (four steps for 6 rows).  Per step: the owners of column k put it
-// in LDS | every thread forms v, tau and its rows of p = tau A v | p in LDS | rank-2 update.
-// Row k of f (stride 8 NC, zero padded) receives v_k; sh.d, sh.e, sh.tau the rest.
+// 1/sqrt(d) to double precision (NaN for d <= 0)
+__device__ __forceinline__ double rsqrt_nr(double d) {
+  double y = __builtin_amdgcn_rsq(d);
+  y = fma(y, fma(-0.5 * d * y, y, 0.5), y);
+  return fma(y, fma(-0.5 * d * y, y, 0.5), y);
+}
+
+// Householder tridiagonalisation of A (n x n in LDS, row stride S).  NC >= ceil(n / 8).
+// Thread (r, c) = (tid / 8, tid % 8) of 512 holds A[r + 64 i][c + 8 j] in registers: row sums cross 8
+// lanes (three DPP steps), and two waves per SIMD fill each other's dependency stalls (four waves of
+// 32 x 8 patches: 1.03 us a step at n = 80, bound by the instructions one wave issues).  One barrier per
+// step: every thread keeps the column x being reduced for its rows and columns; its rows of p = tau A v
+// and column q of A as it still is go to LDS together, and after the barrier every thread forms its part
+// of the updated column q, the next x, itself.  Row k of V (stride 8 NC, zero padded, over A's own LDS)
+// receives v_k; sh.d, sh.e, sh.tau the rest.
 template <int NC>
-__device__ __forceinline__ void tridiagonalise(int n, const double* A, int S, double* f, Smem& sh) {
-  constexpr int NR = (NC + 3) / 4, SP = 8 * NC;
-  const int tid = threadIdx.x;
-  if (__builtin_amdgcn_readfirstlane(tid >> 6) >= 4) {
-    __syncthreads();
-    for (int q = 1; q <= n - 2; ++q) {
-      __syncthreads();
-      __syncthreads();
-    }
-    __syncthreads();
-    return;
-  }
-  const int r = tid >> 3, c = tid & 7;
+__device__ __forceinline__ void tridiagonalise(int n, double* A, int S, Smem& sh) {
+  constexpr int NR = (NC + 7) / 8, SP = 8 * NC;
+  const int tid = threadIdx.x, r = tid >> 3, c = tid & 7;
   double a[NR][NC];
 #pragma unroll
   for (int i = 0; i < NR; ++i)
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      const int row = r + 32 * i, col = c + 8 * j;
+      const int row = r + 64 * i, col = c + 8 * j;
       a[i][j] = row < n && col < n ? A[row * S + col] : 0.0;
     }
-  // column 0 below the diagonal
-  if (c == 0) {
+  // x = column 0 below the diagonal, at this thread's columns, rows and at row q = 1
+  double xc[NC], xr[NR], x0 = A[S];
 #pragma unroll
-    for (int i = 0; i < NR; ++i) sh.x[r + 32 * i] = r + 32 * i >= 1 ? a[i][0] : 0.0;
-    if (r == 0) sh.d[0] = a[0][0];
+  for (int j = 0; j < NC; ++j) {
+    const int col = c + 8 * j;
+    xc[j] = col >= 1 && col < n ? A[col * S] : 0.0;
   }
-  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int row = r + 64 * i;
+    xr[i] = row >= 1 && row < n ? A[row * S] : 0.0;
+  }
+  if (tid == 0) sh.d[0] = a[0][0];
+  __syncthreads();  // A is in registers; its LDS takes V
   static_for<0, NC>([&](auto block) {
-    constexpr int jb = decltype(block)::value, ib = jb / 4;
+    constexpr int jb = decltype(block)::value, ib = jb / 8;
+#pragma unroll 1
     for (int c0 = 0; c0 < 8; ++c0) {
       const int q = 8 * jb + c0;  // reduces column q - 1 to rows <= q
       if (q < 1) continue;
       if (q > n - 2) break;
-      double vc[NC], vr[NR];
-#pragma unroll
-      for (int j = jb; j < NC; ++j) vc[j] = sh.x[c + 8 * j];
-#pragma unroll
-      for (int i = ib; i < NR; ++i) vr[i] = sh.x[r + 32 * i];
-      const double x0 = sh.x[q];
-      double tail = 0.0;
+      double* pb = sh.p[q & 1];
+      double* ab = sh.col[q & 1];
+      double* vrow = A + (size_t)(q - 1) * SP;
+      double tail;
       {
-        const double t = c == c0 ? 0.0 : vc[jb];
+        const double t = c == c0 ? 0.0 : xc[jb];
         tail = t * t;
 #pragma unroll
-        for (int j = jb + 1; j < NC; ++j) tail = fma(vc[j], vc[j], tail);
+        for (int j = jb + 1; j < NC; ++j) tail = fma(xc[j], xc[j], tail);
       }
       tail = group8_sum(tail);
       const bool skip = !(tail > 0.0);
-      const double nx = sqrt(fma(x0, x0, tail));
+      const double s2 = fma(x0, x0, tail), nx = s2 * rsqrt_nr(s2);
       const double alpha = x0 >= 0.0 ? -nx : nx;
       const double v0 = skip ? 0.0 : x0 - alpha;
       const double tau = skip ? 0.0 : rcp_nr(nx * (nx + fabs(x0)));
@@ -279,63 +321,153 @@ __device__ __forceinline__ void tridiagonalise(int n, const double* A, int S, do
       for (int i = ib; i < NR; ++i) {
         u[i] = 0.0;
 #pragma unroll
-        for (int j = jb + 1; j < NC; ++j) u[i] = fma(a[i][j], vc[j], u[i]);
+        for (int j = jb + 1; j < NC; ++j) u[i] = fma(a[i][j], xc[j], u[i]);
       }
-      if (c == c0) vc[jb] = v0;
-      if (r == (q & 31)) vr[ib] = v0;
+      if (c == c0) xc[jb] = v0;  // x becomes v
+      if (r == (q & 63)) xr[ib] = v0;
 #pragma unroll
-      for (int i = ib; i < NR; ++i) {
-        u[i] = tau * group8_sum(fma(a[i][jb], vc[jb], u[i]));
-        if (c == 0) sh.p[r + 32 * i] = u[i];
+      for (int i = ib; i < NR; ++i) u[i] = tau * group8_sum(fma(a[i][jb], xc[jb], u[i]));
+      if (c == c0) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          const int row = r + 64 * i;
+          if (row < 8 * NC) {
+            if (i >= ib) {
+              pb[row] = u[i];
+              ab[row] = a[i][jb];
+            }
+            vrow[row] = i < ib ? 0.0 : xr[i];
+          }
+        }
       }
-#pragma unroll
-      for (int j = 0; j < NC; ++j)
-        if (r == j) f[(size_t)(q - 1) * SP + c + 8 * j] = j < jb ? 0.0 : vc[j];
       if (tid == 0) {
         sh.e[q - 1] = skip ? x0 : alpha;
         sh.tau[q - 1] = tau;
       }
       __syncthreads();
-      double wc[NC];
+      double wc[NC], nc[NC], nr[NR];
+      const double pq = pb[q], pq1 = pb[q + 1], aq1 = ab[q + 1], vq1 = vrow[q + 1];
       double vp = 0.0;
 #pragma unroll
       for (int j = jb; j < NC; ++j) {
-        wc[j] = sh.p[c + 8 * j];
-        vp = fma(vc[j], wc[j], vp);
+        wc[j] = pb[c + 8 * j];
+        nc[j] = ab[c + 8 * j];
+        vp = fma(xc[j], wc[j], vp);
       }
-      const double K = 0.5 * tau * group8_sum(vp);
 #pragma unroll
-      for (int j = jb; j < NC; ++j) wc[j] = fma(-K, vc[j], wc[j]);
+      for (int i = ib; i < NR; ++i) nr[i] = ab[r + 64 * i];
+      const double K = 0.5 * tau * group8_sum(vp);
+      const double wq = fma(-K, v0, pq);
+      if (tid == 0) sh.d[q] = fma(-v0, wq, fma(-wq, v0, ab[q]));
+      x0 = fma(-vq1, wq, fma(-fma(-K, vq1, pq1), v0, aq1));
+#pragma unroll
+      for (int j = jb; j < NC; ++j) wc[j] = fma(-K, xc[j], wc[j]);
 #pragma unroll
       for (int i = ib; i < NR; ++i) {
-        const double wr = fma(-K, vr[i], u[i]);
+        const double wr = fma(-K, xr[i], u[i]);
 #pragma unroll
-        for (int j = jb; j < NC; ++j) a[i][j] = fma(-vr[i], wc[j], fma(-wr, vc[j], a[i][j]));
+        for (int j = jb; j < NC; ++j) a[i][j] = fma(-xr[i], wc[j], fma(-wr, xc[j], a[i][j]));
+        xr[i] = fma(-xr[i], wq, fma(-wr, v0, nr[i]));
       }
-      // column q, the next one, and d_q (x was last read before the barrier above)
-      if (c == c0) {
+      if (r + 64 * ib <= q) xr[ib] = 0.0;  // (rows of later blocks lie below q)
 #pragma unroll
-        for (int i = ib; i < NR; ++i) {
-          const int row = r + 32 * i;
-          sh.x[row] = row > q ? a[i][jb] : 0.0;
-          if (row == q) sh.d[q] = a[i][jb];
-        }
-      }
-      __syncthreads();
+      for (int j = jb; j < NC; ++j) xc[j] = fma(-xc[j], wq, fma(-wc[j], v0, nc[j]));
+      if (c <= c0) xc[jb] = 0.0;
     }
   });
-  if (tid == 0) sh.e[n - 2] = sh.x[n - 1];
+  if (tid == 0) sh.e[n - 2] = x0;
 #pragma unroll
   for (int i = 0; i < NR; ++i)
 #pragma unroll
     for (int j = 0; j < NC; ++j)
-      if (r + 32 * i == n - 1 && c + 8 * j == n - 1) sh.d[n - 1] = a[i][j];
+      if (r + 64 * i == n - 1 && c + 8 * j == n - 1) sh.d[n - 1] = a[i][j];
   __syncthreads();
 }
 
+// X = L^-T (upper triangle, row-major n x n) of the Cholesky factorisation S = L L^T, both in registers: thread
+// (r, c) of 32 x 8 holds the elements [r + 32 i][c + 8 j] (the other waves only take part in the barriers); step k eliminates below the diagonal of S and applies the same row operations to
+// W = I, which ends as L^-1; column k of S and row k of W go to LDS, one barrier a step (a
+// barrier and an LDS or L2 pass per division, column and update took 226 us from LDS, 450 us from L2).
+template <int NC>
+__device__ __forceinline__ void inverse_cholesky(int n, const double* Sm, double* X, Smem& sh) {
+  constexpr int NR = (NC + 3) / 4;
+  const int tid = threadIdx.x;
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) >= 4) {
+    for (int k = 0; k <= n; ++k) __syncthreads();
+    return;
+  }
+  const int r = tid >> 3, c = tid & 7;
+  double a[NR][NC], w[NR][NC];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int row = r + 32 * i, col = c + 8 * j;
+      a[i][j] = row < n && col < n ? Sm[row * n + col] : 0.0;
+      w[i][j] = row == col ? 1.0 : 0.0;
+    }
+  static_for<0, NC>([&](auto block) {
+    constexpr int jb = decltype(block)::value, ib = jb / 4;
+#pragma unroll 1
+    for (int c0 = 0; c0 < 8; ++c0) {
+      const int k = 8 * jb + c0;
+      if (k >= n) break;
+      double* cb = sh.col[k & 1];
+      double* rb = sh.p[k & 1];
+      if (c == c0) {
+#pragma unroll
+        for (int i = ib; i < NR; ++i) cb[r + 32 * i] = a[i][jb];
+      }
+      if (r == (k & 31)) {
+#pragma unroll
+        for (int j = 0; j <= jb; ++j) rb[c + 8 * j] = w[ib][j];
+      }
+      __syncthreads();
+      const double rs = rsqrt_nr(cb[k]);
+      double lc[NC], wk[NC];
+#pragma unroll
+      for (int j = jb; j < NC; ++j) lc[j] = cb[c + 8 * j] * rs;
+#pragma unroll
+      for (int j = 0; j <= jb; ++j) wk[j] = rb[c + 8 * j] * rs;
+#pragma unroll
+      for (int i = ib; i < NR; ++i) {
+        const int row = r + 32 * i;
+        const double lr = row > k ? cb[row] * rs : 0.0;
+#pragma unroll
+        for (int j = jb; j < NC; ++j) a[i][j] = fma(-lr, lc[j], a[i][j]);
+#pragma unroll
+        for (int j = 0; j <= jb; ++j) w[i][j] = row == k ? wk[j] : fma(-lr, wk[j], w[i][j]);
+      }
+    }
+  });
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int row = r + 32 * i, col = c + 8 * j;
+      if (row < n && col < n) X[col * n + row] = row >= col ? w[i][j] : 0.0;
+    }
+  __syncthreads();
+}
+
+// f<NC>() of the size class of n
+template <class F>
+__device__ __forceinline__ void by_size(int n, F&& f) {
+  if (n <= 16)
+    f(Index<2>{});
+  else if (n <= 32)
+    f(Index<4>{});
+  else if (n <= 64)
+    f(Index<8>{});
+  else
+    f(Index<12>{});
+}
+
 // Z <- H_0 ... H_{n-3} Y: column c of the result from column perm[c] of Y (in Z), scaled by nv.
-// Four lanes hold a column: lane q the rows 8 i + 2 q + {0, 1}.  V (n - 2 rows of stride 8 NC) is
-// read into the LDS of both matrices once every column is in registers.
+// Four lanes hold a column, lane q the rows 8 i + 2 q + {0, 1}; the next reflector's LDS reads are in
+// flight during the current one.  (Two columns per lane group halve those reads but leave three waves:
+// 26 us against 20 at n = 80.)  V (n - 2 rows of stride 8 NC) is read into the LDS of both matrices once
+// every column is in registers.
 template <int NC>
 __device__ __forceinline__ void back_transform(int n, int nvec, double* A, double* Z, int S, const double* f, Smem& sh) {
   constexpr int SP = 8 * NC;
@@ -358,20 +490,30 @@ __device__ __forceinline__ void back_transform(int n, int nvec, double* A, doubl
   if (__builtin_amdgcn_readfirstlane(c & ~15) < nvec) {  // (16 columns a wave)
     static_for<0, NC>([&](auto block) {
       constexpr int jb = NC - 1 - decltype(block)::value;
-      for (int c0 = 7; c0 >= 0; --c0) {
-        const int k = 8 * jb + c0 - 1;  // rows > k
-        if (k > n - 3) continue;
-        if (k < 0) break;
-        const double2* v = reinterpret_cast<const double2*>(A + (size_t)k * SP) + q4;
-        double2 vv[NC];
-        double acc0 = 0.0, acc1 = 0.0;
+      const int kt = min(8 * jb + 6, n - 3), kb = max(8 * jb - 1, 0);  // reflectors k with k + 1 in this block
+      if (kt < kb) return;
+      const double2* v = reinterpret_cast<const double2*>(A) + q4;
+      double2 vn[NC], vv[NC];
+#pragma unroll
+      for (int i = jb; i < NC; ++i) vn[i] = v[kt * (SP / 2) + 4 * i];
+      double tau_n = sh.tau[kt];
+#pragma unroll 1
+      for (int k = kt; k >= kb; --k) {
+        const double tau = tau_n;
+        const int kn = max(k - 1, kb);
+        double s0 = 0.0, s1 = 0.0;
 #pragma unroll
         for (int i = jb; i < NC; ++i) {
-          vv[i] = v[4 * i];
-          acc0 = fma(vv[i].x, z[i].x, acc0);
-          acc1 = fma(vv[i].y, z[i].y, acc1);
+          vv[i] = vn[i];
+          vn[i] = v[kn * (SP / 2) + 4 * i];
         }
-        const double s = sh.tau[k] * group4_sum(acc0 + acc1);
+        tau_n = sh.tau[kn];
+#pragma unroll
+        for (int i = jb; i < NC; ++i) {
+          s0 = fma(vv[i].x, z[i].x, s0);
+          s1 = fma(vv[i].y, z[i].y, s1);
+        }
+        const double s = tau * group4_sum(s0 + s1);
 #pragma unroll
         for (int i = jb; i < NC; ++i) {
           z[i].x = fma(-s, vv[i].x, z[i].x);
@@ -414,14 +556,12 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
     return;
   }
   // ---- 1. tridiagonalisation ----
-  if (n <= 16)
-    tridiagonalise<2>(n, A, S, f, sh);
-  else if (n <= 32)
-    tridiagonalise<4>(n, A, S, f, sh);
-  else if (n <= 64)
-    tridiagonalise<8>(n, A, S, f, sh);
-  else
-    tridiagonalise<12>(n, A, S, f, sh);
+  by_size(n, [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    tridiagonalise<NC>(n, A, S, sh);
+    // V to scratch: the pivots of phase 4 take its place
+    for (int idx = tid; idx < (n - 2) * 8 * NC; idx += nt) f[idx] = A[idx];
+  });
   // ---- 2. norm, scaling, unreduced blocks ----
   double scale, unscale;  // powers of two
   {
@@ -469,8 +609,8 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
   }
   __syncthreads();
   // ---- 3. eigenvalues by multisection: lanes 3 v .. 3 v + 2 of a wave for its slot v, no barriers ----
-  // 4^-25 of a width <= 4: 2^-48 of the norm.  Three lanes each: with n = 80 four waves, one per SIMD
-  // (more lanes per eigenvalue share the SIMDs and gain fewer bits per unit of time).
+  // 7^-18 of a width <= 4: 2^-48 of the norm.  Three lanes of two shifts each: with n = 80 four waves, one
+  // per SIMD (more lanes per eigenvalue share the SIMDs and gain fewer bits per unit of time).
   {
     const int v = lane / 3, g = lane - 3 * v, slot = wv * 21 + v;
     const bool act = v < 21 && slot < n;
@@ -492,11 +632,12 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
         lo -= 1e-12 * span;
         hi += 1e-12 * span;
       }
-      for (int r = 0; r < 25; ++r) {
-        const double wd = 0.25 * (hi - lo);
-        const int c = act ? sturm_count(sh.de, s, t, fma(wd, (double)(g + 1), lo)) : 0;
-        const unsigned long long m = __ballot(act && c <= li);
-        const int below = __popcll((m >> (lane - g)) & 7ull);
+      for (int r = 0; r < 18; ++r) {
+        const double wd = (hi - lo) * (1.0 / 7.0);
+        const int2 c = act ? sturm_count2(sh.de, s, t, fma(wd, (double)(2 * g + 1), lo), fma(wd, (double)(2 * g + 2), lo))
+                           : make_int2(0, 0);
+        const unsigned long long m0 = __ballot(act && c.x <= li), m1 = __ballot(act && c.y <= li);
+        const int below = __popcll((m0 >> (lane - g)) & 7ull) + __popcll((m1 >> (lane - g)) & 7ull);
         lo = fma(wd, (double)below, lo);
         hi = lo + wd;
       }
@@ -516,9 +657,9 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
   // ---- 4. eigenvectors of T (column `slot` of Z holds the block's rows) ----
   for (int idx = tid; idx < n * n; idx += nt) Z[(idx / n) * S + idx % n] = 0.0;
   __syncthreads();
-  // 16 vectors a wave: lanes of one wave read neighbouring columns
-  const int slot = (tid >> 6) * 16 + lane;
-  const bool vact = lane < 16 && slot < n;
+  // 16 vectors a wave, two lanes each: the lanes of a wave read neighbouring columns
+  const int slot = (tid >> 6) * 16 + (lane >> 1);
+  const bool vact = lane < 32 && slot < n, bot = lane & 1;
   int bs = 0, bt = 0;
   bool want = false;
   if (vact) {
@@ -561,20 +702,22 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
   };
   const double rmax = 1.0 / (EPS * 2.0);
   if (vact) {
-    sh.nv[slot] = 1.0;
+    double nv = 1.0;
     if (want) {
       if (bt - bs == 1)
         Z[bs * S + slot] = 1.0;
       else
-        sh.nv[slot] = 1.0 / sqrt(ldl_solve<true>(sh.d, sh.e, bs, bt, sh.lam[slot], rmax, A, Z, S, slot, 1.0));
+        nv = 1.0 / sqrt(ldl_solve<true>(sh.d, sh.e, bs, bt, bot, sh.lam[slot], rmax, A, Z, S, slot, 1.0));
     }
+    sh.nv[slot] = nv;
   }
   __syncthreads();
   orthogonalise(1);
   __syncthreads();
-  if (vact && want && bt - bs > 1)
-    sh.nv[slot] =
-        1.0 / sqrt(ldl_solve<false>(sh.d, sh.e, bs, bt, sh.lam[slot], rmax, A, Z, S, slot, sh.nv[slot]));
+  if (vact && want && bt - bs > 1) {
+    const double nv = sh.nv[slot];
+    sh.nv[slot] = 1.0 / sqrt(ldl_solve<false>(sh.d, sh.e, bs, bt, bot, sh.lam[slot], rmax, A, Z, S, slot, nv));
+  }
   __syncthreads();
   orthogonalise(2);
   __syncthreads();
@@ -605,14 +748,7 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
     w[r] = sh.rq[i];
   }
   __syncthreads();
-  if (n <= 16)
-    back_transform<2>(n, nvec, A, Z, S, f, sh);
-  else if (n <= 32)
-    back_transform<4>(n, nvec, A, Z, S, f, sh);
-  else if (n <= 64)
-    back_transform<8>(n, nvec, A, Z, S, f, sh);
-  else
-    back_transform<12>(n, nvec, A, Z, S, f, sh);
+  by_size(n, [&](auto nc) { back_transform<decltype(nc)::value>(n, nvec, A, Z, S, f, sh); });
 }
 
 }  // namespace qexeig
