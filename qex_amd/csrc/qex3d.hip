@@ -1741,7 +1741,7 @@ struct Scf3 {
   const float* ao32;  // QEX3D_PRECISION_FP32_GRID: AO values [rows][x32_ld(n)]
   int prec, x32blk;   // grid precision; workgroups of the FP32 grid kernels for this molecule
   // state (workspace)
-  double *F, *Fd, *D, *Dlast, *C, *Cp, *mo, *J, *K, *Vxc, *vpart, *spart, *rho, *tmp1, *tmp2;
+  double *Fd, *D, *C, *mo, *J, *K, *Vxc, *vpart, *spart, *rho, *tmp2;
   double *diisF, *diisE, *diisB;  // [space][n*n], [space][n*n], [(space+1)^2]
   double* scal;                    // [0] e_tot, [1] e_last, [2] nelec, [3] exc (LDA), [4] gnorm, [5] exc (network)
   int* ist;                        // [0] frozen, [1] cycles done, [2] diis count, [3] diis head, [4] converged
@@ -1755,155 +1755,365 @@ struct Scf3 {
   double* jpart;  // Coulomb tile partials (RKS): jtiles(npair) x 2 x JT
 };
 
-// Fock + CDIIS (one workgroup of NT_SCF threads).  cycle < 0: plain F = H + Veff (no DIIS).
-constexpr int NT_SCF = 1024;
-constexpr int NW_SCF = NT_SCF / 64;
-__global__ __launch_bounds__(NT_SCF) void k_scf_fock(const Scf3* __restrict__ ss, int cycle) {
-  const Scf3 s = ss[blockIdx.x];
-  if (s.ist[0]) return;
-  __shared__ double redm[QEX3D_MAX_DIIS][NW_SCF];
-  const int n = s.n, nn = n * n;
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    double f = s.H[t] + s.J[t];
-    if (s.method != 1) f += s.Vxc[t];
-    if (s.method == 1) f -= 0.5 * s.K[t];
-    s.F[t] = f;
-  }
-  __syncthreads();
-  if (cycle < 1 || s.diis_space < 1) {
-    for (int t = threadIdx.x; t < nn; t += NT_SCF) s.Fd[t] = s.F[t];
-    __syncthreads();
-    return;
-  }
-  // error e = F D S - S D F
-  mfma_gemm(n, n, n, glob(s.F, n, 1), glob(s.D, 1, n), s.tmp1, n, 1.0);     // FD
-  mfma_gemm(n, n, n, glob(s.tmp1, n, 1), glob(s.S, 1, n), s.tmp2, n, 1.0);  // FDS
-  // S D F = (F D S)^T for symmetric F, D, S
-  const int cnt = s.ist[2], head = s.ist[3];
-  const int slot = head;
-  double* Fi = s.diisF + (size_t)slot * nn;
-  double* Ei = s.diisE + (size_t)slot * nn;
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    const int i = t / n, j = t % n;
-    Ei[t] = s.tmp2[i * n + j] - s.tmp2[j * n + i];
-    Fi[t] = s.F[t];
-  }
-  __syncthreads();
-  const int m = cnt + 1 < s.diis_space ? cnt + 1 : s.diis_space;
-  // B (stored by slot) row/column of the new vector: the m dot products in one pass
-  const int M = s.diis_space;
-  {
-    double d[QEX3D_MAX_DIIS];
-#pragma unroll
-    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) d[q] = 0.0;
-    for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-      const double e = Ei[t];
-#pragma unroll
-      for (int q = 0; q < QEX3D_MAX_DIIS; ++q)
-        if (q < m) d[q] = fma(e, s.diisE[(size_t)q * nn + t], d[q]);
-    }
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-#pragma unroll
-    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) {
-      const double x = wsum(d[q]);
-      if (l == 0) redm[q][w] = x;
-    }
-    __syncthreads();
-    if (threadIdx.x < m) {
-      const int q = threadIdx.x;
-      double v = 0.0;
-      for (int k = 0; k < NW_SCF; ++k) v += redm[q][k];
-      s.diisB[slot * M + q] = v;
-      s.diisB[q * M + slot] = v;
-    }
-    __syncthreads();
-  }
-  // solve [0 -1; -1 B] [l; c] = [-1; 0] in the chronological order of the stored vectors
-  __shared__ double Bm[(QEX3D_MAX_DIIS + 1) * (QEX3D_MAX_DIIS + 2)];
-  __shared__ double coef[QEX3D_MAX_DIIS + 1];
-  __shared__ int order[QEX3D_MAX_DIIS];
-  if (threadIdx.x == 0) {
-    const int oldest = m < M ? 0 : (slot + 1) % M;
-    for (int q = 0; q < m; ++q) order[q] = (oldest + q) % M;
-    const int dim = m + 1, ld = m + 2;
-    for (int r = 0; r < dim; ++r)
-      for (int c = 0; c < dim; ++c) {
-        double v;
-        if (r == 0 && c == 0)
-          v = 0.0;
-        else if (r == 0 || c == 0)
-          v = -1.0;
-        else
-          v = s.diisB[order[r - 1] * M + order[c - 1]];
-        Bm[r * ld + c] = v;
-      }
-    for (int r = 0; r < dim; ++r) Bm[r * ld + dim] = r == 0 ? -1.0 : 0.0;
-    // Gaussian elimination with partial pivoting
-    for (int c = 0; c < dim; ++c) {
-      int pr = c;
-      for (int r = c + 1; r < dim; ++r)
-        if (fabs(Bm[r * ld + c]) > fabs(Bm[pr * ld + c])) pr = r;
-      if (pr != c)
-        for (int k = 0; k <= dim; ++k) {
-          const double t = Bm[c * ld + k];
-          Bm[c * ld + k] = Bm[pr * ld + k];
-          Bm[pr * ld + k] = t;
-        }
-      const double pv = Bm[c * ld + c];
-      for (int r = c + 1; r < dim; ++r) {
-        const double f = Bm[r * ld + c] / pv;
-        for (int k = c; k <= dim; ++k) Bm[r * ld + k] -= f * Bm[c * ld + k];
-      }
-    }
-    for (int r = dim - 1; r >= 0; --r) {
-      double v = Bm[r * ld + dim];
-      for (int k = r + 1; k < dim; ++k) v -= Bm[r * ld + k] * coef[k];
-      coef[r] = v / Bm[r * ld + r];
-    }
-    s.ist[2] = m;
-    s.ist[3] = (slot + 1) % M;
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    double f = 0.0;
-    for (int q = 0; q < m; ++q) f = fma(coef[q + 1], s.diisF[(size_t)order[q] * nn + t], f);
-    s.Fd[t] = f;
-  }
-  __syncthreads();
-}
-
-// generalized eigh of Fd: Fp = X^T Fd X (symmetrised), Fp = Z diag(e) Z^T in LDS, C = X Z,
-// D = 2 C_occ C_occ^T.  One workgroup of NT_EIG threads.
 constexpr int NT_EIG = 512;  // 8 waves: 256 registers a lane for the eigensolver's patches and columns
+constexpr int NW_EIG = NT_EIG / 64;
 static_assert(NT_EIG >= qexeig::NT_MIN, "eigensolver threads");
 constexpr int NT_VJP = 1024;
 size_t eigh_lds(int n) { return (size_t)2 * n * (n + 1) * 8; }
 
-// full = 0 (the SCF cycles): only the orbitals the cycle uses (the n_occ + 2 lowest; C's other
-// columns zero, their energies unrefined); full = 1 (after the last cycle, every molecule, frozen or
-// not): the whole solve, whose first n_occ + 2 columns equal the cycles' bit for bit.
-__global__ __launch_bounds__(NT_EIG) void k_scf_eigh(const Scf3* __restrict__ ss, int full) {
+// ---- one SCF step of one molecule in one workgroup of NT_EIG threads ----
+// A matrix over the workgroup: wave w holds rows w + 8 t, lane l the columns l and l + 64, so it moves
+// between global memory and LDS without index arithmetic and with every load in flight.
+constexpr int PATCH_T = QEX3D_MAX_NAO / NW_EIG;
+struct Patch {
+  double v[PATCH_T][2];
+  template <class F>  // v = f(row, column), row and column clamped into the matrix
+  __device__ __forceinline__ void fill(int n, int ncol, F f) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int t = 0; t < PATCH_T; ++t) {
+      if (NW_EIG * t < n) {
+        const int r = min(wv + NW_EIG * t, n - 1);
+        v[t][0] = f(r, min(lane, ncol - 1));
+        if (ncol > 64) v[t][1] = f(r, min(lane + 64, ncol - 1));
+      }
+    }
+  }
+  template <class F>  // f(row, column, v) for every element
+  __device__ __forceinline__ void each(int n, int ncol, F f) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int t = 0; t < PATCH_T; ++t) {
+      const int r = wv + NW_EIG * t;
+      if (r < n) {
+        if (lane < ncol) f(r, lane, v[t][0]);
+        if (ncol > 64 && lane + 64 < ncol) f(r, lane + 64, v[t][1]);
+      }
+    }
+  }
+};
+
+// global n x n (row length n) -> LDS with row stride S, the first ncol columns
+__device__ __forceinline__ void stage(int n, int ncol, const double* src, double* dst, int S) {
+  Patch p;
+  const gptr_t g = (gptr_t)(uintptr_t)src;
+  p.fill(n, ncol, [&](int r, int c) { return g[r * n + c]; });
+  p.each(n, ncol, [&](int r, int c, double x) { dst[r * S + c] = x; });
+}
+
+// op(A) op(B) with both operands in LDS (strides as in Mat); store(row, column, value) runs after every
+// operand has been read, so it may overwrite them.  Barriers on both sides of the stores.
+constexpr int GEMM_T = (QEX3D_MAX_NAO / 16 * QEX3D_MAX_NAO / 16 + NW_EIG - 1) / NW_EIG;
+template <class F>
+__device__ __forceinline__ void lds_gemm(int M, int N, int K, Mat<lptr_t> A, Mat<lptr_t> B, F store) {
+  const int lane = threadIdx.x & 63, kl = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = (N + 15) / 16, tiles = (M + 15) / 16 * nb;
+  d4_t acc[GEMM_T];
+#pragma unroll
+  for (int t = 0; t < GEMM_T; ++t) {
+    const int tile = wv + NW_EIG * t;
+    acc[t] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    if (tile < tiles) {
+      const int bi = tile / nb, bj = tile % nb;
+      const lptr_t pa = A.p + min(bi * 16 + (lane & 15), M - 1) * A.sr;
+      const lptr_t pb = B.p + min(bj * 16 + (lane & 15), N - 1) * B.sr;
+      for (int k0 = 0; k0 < K; k0 += 16) {
+        double a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int k = min(k0 + 4 * u + kl, K - 1);
+          a[u] = pa[k * A.sk];
+          b[u] = pb[k * B.sk];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (k0 + 4 * u < K) {
+            const bool in = k0 + 4 * u + kl < K;
+            acc[t] = mfma64(in ? a[u] : 0.0, in ? b[u] : 0.0, acc[t]);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < GEMM_T; ++t) {
+    const int tile = wv + NW_EIG * t;
+    if (tile < tiles) {
+      const int bi = tile / nb, bj = tile % nb;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = bi * 16 + 4 * v + kl, col = bj * 16 + (lane & 15);
+        if (row < M && col < N) store(row, col, acc[t][v]);
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// sums of M values over the workgroup, in a fixed order; every thread receives them
+template <int M>
+__device__ __forceinline__ void eig_sum(double (&x)[M], double (*red)[NW_EIG]) {
+  const int w = threadIdx.x >> 6;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const double y = qexeig::wave_sum(x[m]);
+    if ((threadIdx.x & 63) == 0) red[m][w] = y;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    double y = 0.0;
+#pragma unroll
+    for (int q = 0; q < NW_EIG; ++q) y += red[m][q];
+    x[m] = y;
+  }
+}
+
+// The CDIIS coefficients c_q of m vectors, from [0 -1; -1 B] [l; c] = [-1; 0] by Gaussian elimination with
+// partial pivoting: one wave, lane r holding row r of the bordered matrix (columns 0..m, right-hand side).
+// B(i, j) = b[order(i) * M + order(j)].  (A single thread walking the matrix in LDS took 33 us for m = 8.)
+__device__ __forceinline__ void diis_solve(int m, const double* b, int M, const int* order, double* coef) {
+  constexpr int DM = QEX3D_MAX_DIIS + 1;
+  const int r = threadIdx.x & 63, dim = m + 1;
+  double a[DM], rhs = r == 0 ? -1.0 : 0.0;
+#pragma unroll
+  for (int c = 0; c < DM; ++c) {
+    a[c] = 0.0;
+    if (c < dim && r < dim) a[c] = r == 0 && c == 0 ? 0.0 : r == 0 || c == 0 ? -1.0 : b[order[r - 1] * M + order[c - 1]];
+  }
+  int prow[DM];
+  bool used = r >= dim;
+#pragma unroll
+  for (int c = 0; c < DM; ++c) {
+    if (c < dim) {
+      const double v = used ? -1.0 : fabs(a[c]);
+      const double best = qexeig::wave_max(v);
+      const unsigned long long who = __ballot(!used && v == best);
+      const int p = who ? __ffsll((long long)who) - 1 : __ffsll((long long)__ballot(!used)) - 1;  // (NaN: any row left)
+      prow[c] = p;
+      const double pv = qexeig::read_lane(a[c], p), pr = qexeig::read_lane(rhs, p);
+      used = used || r == p;
+      const double f = used ? 0.0 : a[c] / pv;
+#pragma unroll
+      for (int k = c + 1; k < DM; ++k)
+        if (k < dim) a[k] = fma(-f, qexeig::read_lane(a[k], p), a[k]);
+      rhs = fma(-f, pr, rhs);
+    }
+  }
+#pragma unroll
+  for (int c = DM - 1; c >= 0; --c) {
+    if (c < dim) {
+      const double x = qexeig::read_lane(rhs / a[c], prow[c]);
+      rhs = fma(-a[c], x, rhs);
+      if (c > 0 && r == 0) coef[c - 1] = x;
+    }
+  }
+}
+
+// Everything of an SCF cycle that one workgroup does for its molecule, in one launch, with the matrices in
+// LDS between the products (as three kernels their products read each matrix from L2 with one tile's latency
+// at a time, 12..24 us each, and a single thread solved the DIIS equations: Fock 97, eigensolver 238 and
+// energy 25 us at n = 80):
+//   ecycle >= -1: total energy of the current density (J, Vxc and K are its own) and, for ecycle >= 0, the
+//     orbital gradient and the convergence test of that cycle; a molecule that ends here is frozen;
+//   fcycle >= -1: F = H + Veff, from cycle 1 on CDIIS with the error F D S - S D F, then the eigenproblem
+//     X^T F X = Z diag(e) Z^T, the n_occ occupied orbitals C = X Z and D = 2 C_occ C_occ^T;
+//   full (after the last cycle, frozen or not): all orbitals and orbital energies of the last Fock matrix
+//     used, whose first n_occ columns equal the cycle's bit for bit.
+__global__ __launch_bounds__(NT_EIG) void k_scf_step(const Scf3* __restrict__ ss, int ecycle, int fcycle, int full) {
   const Scf3 s = ss[blockIdx.x];
   if (s.ist[0] && !full) return;
   extern __shared__ __attribute__((aligned(16))) double sm[];
   __shared__ qexeig::Smem sh;
-  const int n = s.n, nn = n * n, S = n + 1;
+  __shared__ double red[QEX3D_MAX_DIIS][NW_EIG];
+  __shared__ double coef[QEX3D_MAX_DIIS];
+  __shared__ int order[QEX3D_MAX_DIIS];
+  __shared__ int frozen;
+  const int n = s.n, nocc = s.nocc, S = n + 1, tid = threadIdx.x;
+  const bool rhf = s.method == QEX3D_RHF;
   double* A = sm;
   double* Z = A + (size_t)n * S;
-  mfma_gemm(n, n, n, glob(s.Fd, n, 1), glob(s.X, 1, n), s.tmp1, n, 1.0);  // Fd X
-  mfma_gemm(n, n, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), A, S, 1.0);      // X^T Fd X (into LDS)
-  for (int t = threadIdx.x; t < nn; t += blockDim.x) {
-    const int i = t / n, j = t % n;
-    if (i < j) {
-      const double v = 0.5 * (A[i * S + j] + A[j * S + i]);
-      A[i * S + j] = v;
-      A[j * S + i] = v;
+  const gptr_t H = (gptr_t)(uintptr_t)s.H, J = (gptr_t)(uintptr_t)s.J, D = (gptr_t)(uintptr_t)s.D;
+  const gptr_t V = (gptr_t)(uintptr_t)(rhf ? s.K : s.Vxc);
+  auto rows = [&](const double* p) { return lds(p, S, 1); };  // operand as stored
+  auto cols = [&](const double* p) { return lds(p, 1, S); };  // operand transposed (or the right factor)
+  Patch F;
+  if (!full) {
+    Patch h, j;
+    h.fill(n, n, [&](int r, int c) { return H[r * n + c]; });
+    j.fill(n, n, [&](int r, int c) { return J[r * n + c]; });
+    F.fill(n, n, [&](int r, int c) { return V[r * n + c]; });
+    if (ecycle >= -1) {
+      double e[2] = {0.0, 0.0};  // tr(D H), tr(D (J / 2 [- K / 4]))
+      Patch d;
+      d.fill(n, n, [&](int r, int c) { return D[r * n + c]; });
+#pragma unroll
+      for (int t = 0; t < PATCH_T; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if ((threadIdx.x >> 6) + NW_EIG * t < n && (threadIdx.x & 63) + 64 * u < n) {
+            e[0] = fma(d.v[t][u], h.v[t][u], e[0]);
+            const double g = 0.5 * j.v[t][u];
+            e[1] = fma(d.v[t][u], rhf ? g - 0.25 * F.v[t][u] : g, e[1]);
+          }
+      eig_sum<2>(e, red);
+      const double etot =
+          e[0] + e[1] + (has_point_exc(s.method) ? s.scal[3] : s.method == QEX3D_RKS_NN_GLOBAL ? s.scal[5] : 0.0) + s.enuc;
+      if (ecycle < 0 && tid == 0) {
+        s.scal[0] = etot;
+        s.e_hist[0] = etot;
+      }
+      coef[0] = etot;  // (the same value from every thread)
     }
+#pragma unroll
+    for (int t = 0; t < PATCH_T; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const double f = h.v[t][u] + j.v[t][u];
+        F.v[t][u] = rhf ? f - 0.5 * F.v[t][u] : f + F.v[t][u];
+      }
   }
+  if (ecycle >= 0) {
+    // orbital gradient norm with the new Fock matrix: |C_vir^T F C_occ|^2 via the S^-1 projector
+    // = tr(Co^T F X X^T F Co) - |Co^T F Co|^2, times 4 (the factor 2 of pyscf's get_grad)
+    F.each(n, n, [&](int r, int c, double x) { A[r * S + c] = x; });
+    stage(n, nocc, s.C, Z, S);
+    __syncthreads();
+    lds_gemm(n, nocc, n, rows(A), cols(Z), [&](int r, int c, double x) { A[r * S + c] = x; });  // F C_occ
+    double ab[2] = {0.0, 0.0};
+    lds_gemm(nocc, nocc, n, cols(Z), cols(A), [&](int, int, double x) { ab[1] = fma(x, x, ab[1]); });
+    stage(n, n, s.X, Z, S);
+    __syncthreads();
+    lds_gemm(n, nocc, n, cols(Z), cols(A), [&](int, int, double x) { ab[0] = fma(x, x, ab[0]); });
+    eig_sum<2>(ab, red);
+    if (tid == 0) {
+      const double g2 = fmax(0.0, 4.0 * (ab[0] - ab[1]));
+      const int nvir = n - nocc;
+      const double gnorm = sqrt(g2) / sqrt((double)(nvir > 0 ? nvir * nocc : 1));
+      const double elast = s.scal[0], etot = coef[0];
+      s.scal[1] = elast;
+      s.scal[0] = etot;
+      s.scal[4] = gnorm;
+      s.e_hist[ecycle + 1] = etot;
+      s.ist[1] = ecycle + 1;
+      int fr = 0;
+      if (fabs(etot - elast) < s.conv_tol && gnorm < sqrt(s.conv_tol)) {
+        fr = 1;
+        s.ist[4] = 1;
+      } else if (ecycle + 1 >= s.max_cycle) {
+        fr = 1;  // out of cycles: frozen, not converged (a batch runs to its longest member)
+      }
+      if (fr) s.ist[0] = 1;
+      frozen = fr;
+    }
+    __syncthreads();
+    if (frozen) return;
+  }
+  if (fcycle < -1 && !full) return;
+  const int nn = n * n;
+  if (full) {
+    stage(n, n, s.Fd, A, S);
+  } else if (fcycle < 1 || s.diis_space < 1) {
+    F.each(n, n, [&](int r, int c, double x) {
+      s.Fd[r * n + c] = x;
+      A[r * S + c] = x;
+    });
+  } else {
+    const int M = s.diis_space, cnt = s.ist[2], slot = s.ist[3], m = cnt + 1 < M ? cnt + 1 : M;
+    double* Fi = s.diisF + (size_t)slot * nn;
+    double* Ei = s.diisE + (size_t)slot * nn;
+    // error e = F D S - S D F; S D F = (F D S)^T for symmetric F, D, S
+    F.each(n, n, [&](int r, int c, double x) {
+      A[r * S + c] = x;
+      Fi[r * n + c] = x;
+    });
+    stage(n, n, s.D, Z, S);
+    __syncthreads();
+    lds_gemm(n, n, n, rows(A), cols(Z), [&](int r, int c, double x) { A[r * S + c] = x; });
+    stage(n, n, s.S, Z, S);
+    __syncthreads();
+    lds_gemm(n, n, n, rows(A), cols(Z), [&](int r, int c, double x) { A[r * S + c] = x; });
+    Patch E;
+    E.fill(n, n, [&](int r, int c) { return A[r * S + c] - A[c * S + r]; });
+    E.each(n, n, [&](int r, int c, double x) { Ei[r * n + c] = x; });
+    // B (stored by slot): the new vector's products with the stored ones, each vector's loads in flight
+    double d[QEX3D_MAX_DIIS];
+#pragma unroll
+    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) {
+      d[q] = 0.0;
+      if (q < m) {
+        Patch p = E;
+        if (q != slot) {
+          const gptr_t g = (gptr_t)(uintptr_t)(s.diisE + (size_t)q * nn);
+          p.fill(n, n, [&](int r, int c) { return g[r * n + c]; });
+        }
+#pragma unroll
+        for (int t = 0; t < PATCH_T; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            if ((threadIdx.x >> 6) + NW_EIG * t < n && (threadIdx.x & 63) + 64 * u < n)
+              d[q] = fma(E.v[t][u], p.v[t][u], d[q]);
+      }
+    }
+    eig_sum<QEX3D_MAX_DIIS>(d, red);
+    if (tid < m) {
+      double v = 0.0;
+#pragma unroll
+      for (int q = 0; q < QEX3D_MAX_DIIS; ++q)
+        if (q == tid) v = d[q];
+      s.diisB[slot * M + tid] = v;
+      s.diisB[tid * M + slot] = v;
+      order[tid] = ((m < M ? 0 : slot + 1) + tid) % M;  // oldest first
+    }
+    __syncthreads();
+    if (tid < 64) diis_solve(m, s.diisB, M, order, coef);
+    if (tid == 0) {
+      s.ist[2] = m;
+      s.ist[3] = (slot + 1) % M;
+    }
+    __syncthreads();
+    Patch f;
+    f.fill(n, n, [](int, int) { return 0.0; });
+#pragma unroll
+    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) {
+      if (q < m) {
+        Patch p = F;
+        if (order[q] != slot) {
+          const gptr_t g = (gptr_t)(uintptr_t)(s.diisF + (size_t)order[q] * nn);
+          p.fill(n, n, [&](int r, int c) { return g[r * n + c]; });
+        }
+        const double cq = coef[q];
+#pragma unroll
+        for (int t = 0; t < PATCH_T; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) f.v[t][u] = fma(cq, p.v[t][u], f.v[t][u]);
+      }
+    }
+    f.each(n, n, [&](int r, int c, double x) {
+      s.Fd[r * n + c] = x;
+      A[r * S + c] = x;
+    });
+  }
+  stage(n, n, s.X, Z, S);
   __syncthreads();
-  qexeig::symeig(n, A, Z, S, s.mo, s.eigf, sh, full ? n : s.nocc + 2);
-  mfma_gemm(n, n, n, glob(s.X, n, 1), lds(Z, 1, S), s.C, n, 1.0);  // C = X Z
-  mfma_gemm(n, n, s.nocc, glob(s.C, n, 1), glob(s.C, n, 1), s.D, n, 2.0);  // D = 2 C_occ C_occ^T
+  lds_gemm(n, n, n, rows(A), cols(Z), [&](int r, int c, double x) { A[r * S + c] = x; });  // Fd X
+  lds_gemm(n, n, n, cols(Z), cols(A), [&](int r, int c, double x) { A[r * S + c] = x; });  // X^T Fd X
+  Patch p;
+  p.fill(n, n, [&](int r, int c) { return 0.5 * (A[r * S + c] + A[c * S + r]); });
+  __syncthreads();
+  p.each(n, n, [&](int r, int c, double x) { A[r * S + c] = x; });
+  __syncthreads();
+  qexeig::symeig(n, A, Z, S, s.mo, s.eigf, sh, full ? n : nocc + 2);
+  stage(n, n, s.X, A, S);
+  __syncthreads();
+  lds_gemm(n, full ? n : nocc, n, rows(A), cols(Z), [&](int r, int c, double x) {  // C = X Z
+    Z[r * S + c] = x;
+    s.C[r * n + c] = x;
+  });
+  lds_gemm(n, n, nocc, rows(Z), rows(Z), [&](int r, int c, double x) { s.D[r * n + c] = 2.0 * x; });
 }
 
 // batched generalized eigh F C = S C e, one workgroup per matrix (scratch: 8 n^2 doubles each)
@@ -1963,72 +2173,6 @@ __global__ __launch_bounds__(NT_VJP) void k_eigh_vjp(int n, const double* w, con
       const double s = 0.5 * (G[i * n + j] + G[j * n + i]);
       G[i * n + j] = s;
       G[j * n + i] = s;
-    }
-  }
-}
-
-// Energies and convergence (one workgroup of NT_SCF threads).
-__global__ __launch_bounds__(NT_SCF) void k_scf_energy(const Scf3* __restrict__ ss, int cycle) {
-  const Scf3 s = ss[blockIdx.x];
-  if (s.ist[0]) return;
-  __shared__ double red[NW_SCF];
-  const int n = s.n, nn = n * n, nocc = s.nocc;
-  double e1 = 0.0, e2 = 0.0;
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    e1 = fma(s.D[t], s.H[t], e1);
-    double g = 0.5 * s.J[t];
-    if (s.method == 1) g -= 0.25 * s.K[t];
-    e2 = fma(s.D[t], g, e2);
-  }
-  e1 = bsum(e1, red);
-  e2 = bsum(e2, red);
-  const double etot = e1 + e2 + (has_point_exc(s.method) ? s.scal[3] : s.method == QEX3D_RKS_NN_GLOBAL ? s.scal[5] : 0.0) +
-                      s.enuc;
-  if (cycle < 0) {
-    if (threadIdx.x == 0) {
-      s.scal[0] = etot;
-      s.e_hist[0] = etot;
-    }
-    return;
-  }
-  // orbital gradient norm with the new Fock matrix: |C_vir^T F C_occ|^2 via the S^-1 projector
-  // = tr(Co^T F X X^T F Co) - |Co^T F Co|^2, times 4 (the factor 2 of pyscf's get_grad)
-  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
-    double f = s.H[t] + s.J[t];
-    if (s.method != 1) f += s.Vxc[t];
-    if (s.method == 1) f -= 0.5 * s.K[t];
-    s.F[t] = f;
-  }
-  __syncthreads();
-  mfma_gemm(n, nocc, n, glob(s.F, n, 1), glob(s.C, 1, n), s.tmp1, n, 1.0);    // tmp1 = F C_occ   (n x nocc)
-  mfma_gemm(n, nocc, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), s.tmp2, n, 1.0);  // tmp2 = X^T F C_occ
-  mfma_gemm(nocc, nocc, n, glob(s.C, 1, n), glob(s.tmp1, 1, n), s.Cp, n, 1.0); // Cp = C_occ^T F C_occ
-  double a = 0.0, b = 0.0;
-  for (int t = threadIdx.x; t < n * nocc; t += NT_SCF) {
-    const double v = s.tmp2[(t / nocc) * n + t % nocc];
-    a = fma(v, v, a);
-  }
-  for (int t = threadIdx.x; t < nocc * nocc; t += NT_SCF) {
-    const double v = s.Cp[(t / nocc) * n + t % nocc];
-    b = fma(v, v, b);
-  }
-  a = bsum(a, red);
-  b = bsum(b, red);
-  if (threadIdx.x == 0) {
-    const double g2 = fmax(0.0, 4.0 * (a - b));
-    const int nvir = n - s.nocc;
-    const double gnorm = sqrt(g2) / sqrt((double)(nvir > 0 ? nvir * s.nocc : 1));
-    const double elast = s.scal[0];
-    s.scal[1] = elast;
-    s.scal[0] = etot;
-    s.scal[4] = gnorm;
-    s.e_hist[cycle + 1] = etot;
-    s.ist[1] = cycle + 1;
-    if (fabs(etot - elast) < s.conv_tol && gnorm < sqrt(s.conv_tol)) {
-      s.ist[0] = 1;
-      s.ist[4] = 1;
-    } else if (cycle + 1 >= s.max_cycle) {
-      s.ist[0] = 1;  // out of cycles: frozen, not converged (a batch runs to its longest member)
     }
   }
 }
@@ -2203,7 +2347,7 @@ __global__ __launch_bounds__(256) void k_coulomb_jsum_b(const Scf3* __restrict__
 }
 
 struct Lay3 {
-  size_t F, Fd, D, Dlast, C, Cp, mo, J, K, Vxc, vpart, spart, rho, tmp1, tmp2, diisF, diisE, diisB, scal, ist;
+  size_t Fd, D, J, K, Vxc, vpart, spart, rho, tmp2, diisF, diisE, diisB, scal, ist;
   size_t zpart, z1, dz1, wv, ex, eigf, jpart, total;
 };
 
@@ -2219,13 +2363,8 @@ Lay3 layout3(int n, long ng, int space, int h1 = 0) {
     off = al(off + b);
     return o;
   };
-  L.F = take(nn);
   L.Fd = take(nn);
   L.D = take(nn);
-  L.Dlast = take(nn);
-  L.C = take(nn);
-  L.Cp = take(nn);
-  L.mo = take((size_t)n * 8);
   L.J = take(nn);
   L.K = take(nn);
   L.Vxc = take(nn);
@@ -2233,7 +2372,6 @@ Lay3 layout3(int n, long ng, int space, int h1 = 0) {
   L.vpart = take(v64 > v32 ? v64 : v32);
   L.spart = take((size_t)nchunk * 16);
   L.rho = take((size_t)ng * 8);
-  L.tmp1 = take(nn);
   L.tmp2 = take(nn);
   L.diisF = take((size_t)space * nn);
   L.diisE = take((size_t)space * nn);
@@ -2920,11 +3058,11 @@ static bool nn_widths_ok(int h1, int h2) {
   return h1 >= 1 && h2 >= 1 && h1 <= QEX3D_MAX_NN_HIDDEN && h2 <= QEX3D_MAX_NN_HIDDEN;
 }
 
-// one molecule's region: the state layout, then the Cholesky factor and the orthogonaliser
+// one molecule's region: the state layout, then the orthogonaliser
 static size_t scf_mol_bytes(const qex3d_scf_problem* p) {
   if (!p || p->nao < 1 || p->nao > QEX3D_MAX_NAO || scf_ngrid(p) < 1) return 0;
   if (p->method == QEX3D_RKS_NN_GLOBAL && !nn_widths_ok(p->nn_h1, p->nn_h2)) return 0;
-  return al(layout3(p->nao, scf_ngrid(p), scf_space(p), scf_h1(p)).total + al((size_t)p->nao * p->nao * 8) * 2);
+  return al(layout3(p->nao, scf_ngrid(p), scf_space(p), scf_h1(p)).total + al((size_t)p->nao * p->nao * 8));
 }
 // the records of a batch and the host-poll counter come first
 static size_t scf_head_bytes(int B) { return al((size_t)B * sizeof(Scf3)) + al(64); }
@@ -3197,14 +3335,11 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     s.ao32 = ins[b].ao_f32;
     s.prec = p->method == QEX3D_RHF ? QEX3D_PRECISION_FP64 : p->precision;
     s.x32blk = x32_blocks(ng);
-    s.X = (double*)(w + L.total + al((size_t)n * n * 8));
+    s.X = (double*)(w + L.total);
     s.status_out = outs[b].status;
-    s.F = (double*)(w + L.F);
     s.Fd = (double*)(w + L.Fd);
     s.D = outs[b].dm;
-    s.Dlast = (double*)(w + L.Dlast);
     s.C = outs[b].mo_coeff;
-    s.Cp = (double*)(w + L.Cp);
     s.mo = outs[b].mo_energy;
     s.J = (double*)(w + L.J);
     s.K = (double*)(w + L.K);
@@ -3212,7 +3347,6 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     s.vpart = (double*)(w + L.vpart);
     s.spart = (double*)(w + L.spart);
     s.rho = (double*)(w + L.rho);
-    s.tmp1 = (double*)(w + L.tmp1);
     s.tmp2 = (double*)(w + L.tmp2);
     s.diisF = (double*)(w + L.diisF);
     s.diisE = (double*)(w + L.diisE);
@@ -3268,9 +3402,10 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
   }
   if (off > need) return fail3(QEX_E_WORKSPACE, "internal layout exceeds workspace");
   const size_t lds_eigh = eigh_lds(nmax);
-  if (lds_eigh + sizeof(qexeig::Smem) > 160 * 1024) return fail3(QEX_E_UNSUPPORTED, "nao too large for the LDS eigensolver");
+  constexpr size_t static_lds = sizeof(qexeig::Smem) + sizeof(double) * QEX3D_MAX_DIIS * (NW_EIG + 1) + 64;
+  if (lds_eigh + static_lds > 160 * 1024) return fail3(QEX_E_UNSUPPORTED, "nao too large for the LDS eigensolver");
   if (lds_eigh > 64 * 1024)
-    (void)hipFuncSetAttribute((const void*)k_scf_eigh, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_eigh);
+    (void)hipFuncSetAttribute((const void*)k_scf_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_eigh);
   if (lds_nnl > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)k_nn_local_b, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_nnl);
   for (int b0 = 0; b0 < B; b0 += PUT_N) {
@@ -3333,31 +3468,28 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     qexprof::Scope ps_(kind, st);
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(NT), 0, st, dss, args...);
   };
-  auto per_mol_wide = [&](int kind, auto kernel, auto... args) {
+  auto step = [&](int kind, int ecycle, int fcycle, int full) {
     qexprof::Scope ps_(kind, st);
-    hipLaunchKernelGGL(kernel, dim3(nb), dim3(NT_SCF), 0, st, dss, args...);
+    hipLaunchKernelGGL(k_scf_step, dim3(nb), dim3(NT_EIG), lds_eigh, st, dss, ecycle, fcycle, full);
   };
-  auto eigh = [&](int full) {
-    qexprof::Scope ps_(qexprof::K_EIGH, st);
-    hipLaunchKernelGGL(k_scf_eigh, dim3(nb), dim3(NT_EIG), lds_eigh, st, dss, full);
-  };
+  constexpr int NONE = -2;
   // core-Hamiltonian guess: F = H (k_scf_init zeroes J, K, Vxc and D with a kernel, not a memset)
   per_mol(qexprof::K_OTHER, k_scf_init);
   {
     qexprof::Scope ps_(qexprof::K_OTHER, st);
     hipLaunchKernelGGL(k_scf_orthogonaliser, dim3(nb), dim3(NT_ORTH), 0, st, dss);
   }
-  per_mol_wide(qexprof::K_FOCK, k_scf_fock, -1);
-  eigh(0);
+  step(qexprof::K_EIGH, NONE, -1, 0);
   veff();
-  per_mol_wide(qexprof::K_ENERGY, k_scf_energy, -1);
+  int done = -1;  // the cycle whose energy the next step evaluates
   for (int c = 0; c < max_cycle; ++c) {
-    per_mol_wide(qexprof::K_FOCK, k_scf_fock, c);
-    eigh(0);
+    step(qexprof::K_EIGH, done, c, 0);
     veff();
-    per_mol_wide(qexprof::K_ENERGY, k_scf_energy, c);
+    done = c;
     if (sync_every > 0 && (c + 1) % sync_every == 0 && c + 1 < max_cycle) {
       // optional host check: stop enqueueing cycles once every molecule is frozen
+      step(qexprof::K_ENERGY, done, NONE, 0);
+      done = NONE;
       int32_t left = 0;
       hipLaunchKernelGGL(k_scf_active, dim3(1), dim3(64), 0, st, dss, B, active);
       if (hipMemcpyAsync(&left, active, sizeof(int32_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -3366,7 +3498,8 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
       if (left == 0) break;
     }
   }
-  eigh(1);  // all orbitals and orbital energies of the final Fock matrix
+  if (done != NONE) step(qexprof::K_ENERGY, done, NONE, 0);
+  step(qexprof::K_EIGH, NONE, NONE, 1);  // all orbitals and orbital energies of the final Fock matrix
   per_mol(qexprof::K_OTHER, k_scf_finish);
   return launch_status(name);
 }
