@@ -27,6 +27,7 @@
 #include "qex.h"
 #include "prof.h"
 #include "band.h"
+#include "band_wave.h"
 
 namespace qexprof {
 bool g_on = false;
@@ -39,19 +40,15 @@ int g_pool_n = 0, g_pool_used = 0;
 
 namespace {
 
-using qexband::ldlt_backward;
-using qexband::ldlt_factor_forward;
-using qexband::ldlt_forward;
 using qexband::rcp64;
-using qexband::sturm_count;
 using qexband::Side;
+using qexband::middle_solve;
 using qexband::SideZ;
 using qexband::sturm_side;
 using qexband::sturm_join;
-using qexband::middle_solve;
-using qexband::ldlt_side_factor_forward;
-using qexband::ldlt_side_forward;
-using qexband::ldlt_side_backward;
+using qexband::wave_doubles;
+using qexband::wave_rows;
+using qexband::wave_solve;
 
 constexpr int NT = 256;     // threads per workgroup (4 wave64)
 constexpr int NWAVE = NT / 64;
@@ -98,6 +95,17 @@ __device__ __forceinline__ double wave_sum(double x) {
   x += dpp_f64<0x4E>(x);   // quad_perm [2, 3, 0, 1]
   x += dpp_f64<0x141>(x);  // row_half_mirror
   x += dpp_f64<0x140>(x);  // row_mirror
+  return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
+}
+
+// The same where every lane needs the very same bits (control flow): not contracted, since a product fused
+// into its own lane's first addition, but rounded on its way to the others, would make the lanes' sums differ.
+__device__ __forceinline__ double wave_sum_same(double x) {
+#pragma clang fp contract(off)
+  x += dpp_f64<0xB1>(x);
+  x += dpp_f64<0x4E>(x);
+  x += dpp_f64<0x141>(x);
+  x += dpp_f64<0x140>(x);
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
@@ -1027,6 +1035,286 @@ __device__ __forceinline__ double start_value(int i, int j) {
   return ((double)(h & 0xffffff) / 16777216.0) - 0.5;
 }
 
+// y <- (A - sigma)^-1 y / |.| on one wave
+__device__ __forceinline__ void inverse_step(const double* a, double* y, double* F, int N, double b, double c, double sigma) {
+  const int m = wave_rows(N), r0 = (threadIdx.x & 63) * m, r1 = min(N, r0 + m);
+  wave_solve<true>(a, y, N, b, c, sigma, F);
+  double n2 = 0.0;
+  for (int i = r0; i < r1; ++i) n2 = fma(y[i], y[i], n2);
+  const double sc = 1.0 / sqrt(wave_sum_same(n2));
+  for (int i = r0; i < r1; ++i) y[i] *= sc;
+}
+
+// The j-th eigenvalue to 1e-12 by Rayleigh-quotient iteration on one wave (all 64 lanes) from the vector in
+// y, until the residual |A y - rho y| is 1e-8 (the quotient's error is its square over the gap).
+//   check: at most 3 solves, the first with y's own quotient as shift; the eigenvalue count just above rho
+//     must then be j + 1.
+//   else: [slo, shi] is known to hold the j-th eigenvalue and no other; the shift is its middle until the
+//     quotient lies inside.
+// false if that does not end with the j-th pair; the caller brackets the eigenvalue further.
+__device__ bool refine_eigenvalue(const double* a, double* y, double* F, int N, double b, double c, double hnorm, int j,
+                                  double slo, double shi, bool check, double* rho_out) {
+  const int m = wave_rows(N), r0 = (threadIdx.x & 63) * m, r1 = min(N, r0 + m);
+  auto hy = [&](int i) {
+    double v = a[i] * y[i];
+    if (i >= 1) v = fma(b, y[i - 1], v);
+    if (i + 1 < N) v = fma(b, y[i + 1], v);
+    if (i >= 2) v = fma(c, y[i - 2], v);
+    if (i + 2 < N) v = fma(c, y[i + 2], v);
+    return v;
+  };
+  auto quotient = [&]() {
+    double q = 0.0;
+    for (int i = r0; i < r1; ++i) q = fma(y[i], hy(i), q);
+    return wave_sum_same(q);
+  };
+  double sigma = check ? quotient() : 0.5 * (slo + shi);
+  for (int it = 0; it < (check ? 3 : 6); ++it) {
+    inverse_step(a, y, F, N, b, c, sigma);
+    const double rho = quotient();
+    if (rho >= slo && rho <= shi) {
+      double r2 = 0.0;
+      for (int i = r0; i < r1; ++i) {
+        const double d = fma(-rho, y[i], hy(i));
+        r2 = fma(d, d, r2);
+      }
+      if (wave_sum_same(r2) <= 1e-16 * fmax(1.0, rho * rho)) {
+        *rho_out = rho;
+        const double tau = 1e-9 * fmax(1.0, fabs(rho)) + 64.0 * EPS * hnorm;
+        return !check || wave_solve<false>(a, y, N, b, c, rho + tau, F) == j + 1;
+      }
+      sigma = rho;
+    }
+  }
+  return false;
+}
+
+// Multisection bracket of the j-th eigenvalue: NS shifts per round, both ends included; first = index of the
+// first shift with more than j eigenvalues below it (NS: none).
+struct Bracket {
+  double lo, hi, gl, gu;
+  __device__ __forceinline__ double step(int NS) const { return (hi - lo) / (double)(NS - 1); }
+  __device__ __forceinline__ double shift(int me, int NS, double st) const { return me == NS - 1 ? hi : fma((double)me, st, lo); }
+  __device__ __forceinline__ bool small(double hnorm) const {
+    return hi - lo <= 1e-9 * fmax(1.0, fabs(0.5 * (lo + hi))) + 64.0 * EPS * hnorm;
+  }
+  // the next bracket; false if it does not change (rounding floor).  An eigenvalue outside: the adjacent
+  // interval 256 times as wide (clipped to the Gershgorin bounds), so a missed warm start costs about one round
+  __device__ __forceinline__ bool narrow(int first, int NS, double st) {
+    const double wide = 256.0 * (hi - lo);
+    double nlo, nhi;
+    if (first == 0) {
+      nhi = lo;
+      nlo = fmax(gl, lo - wide);
+      if (!(nlo < lo)) nlo = lo > gl ? gl : lo;
+    } else if (first == NS) {
+      nlo = hi;
+      nhi = fmin(gu, hi + wide);
+      if (!(nhi > hi)) nhi = hi < gu ? gu : hi;
+    } else {
+      nlo = first - 1 == 0 ? lo : fma((double)(first - 1), st, lo);
+      nhi = first == NS - 1 ? hi : fma((double)first, st, lo);
+    }
+    const bool moved = nlo != lo || nhi != hi;
+    lo = nlo;
+    hi = nhi;
+    return moved;
+  }
+};
+
+// Order of the rows for the two-sided chains: the top rows 0 .. kt - 1, the middle pair kt, kt + 1, then the bottom
+// rows from N - 1 up to kt + 2, so that both sides walk forward (LDS reads at constant offsets from one
+// address; with a per-lane direction every operand's address took its own instructions)
+__device__ __forceinline__ int side_pos(int t, int N, int kt) { return t <= kt + 1 ? t : N + 1 + kt - t; }
+
+// Inverse iteration without pivoting, by the whole workgroup: one LDL^T factorisation of A - sigma, twisted at rows
+// kt, kt + 1 (the top rows eliminated downwards by lane 0, the bottom rows upwards by lane 1), and two solves
+// from y, normalised after each; ap and y in the order of side_pos.  The recurrences are those of band.h's
+// ldlt_side_* and give the same bits; they are chains of what one wave can issue (7 cycles an instruction), so
+// a chain carries only what it must: wave 0 factorises a chunk of rows (pivots r and off-diagonals u) while
+// wave 1 forms the multipliers of the chunk before with all its lanes and runs the forward solve; z / d is a
+// parallel pass; the back substitution is two FMAs a row.  A single wave doing all of it took 29 + 17 us at
+// N = 513.  F: 5 N doubles: (r, u) and (l, m) per row, z.
+__device__ __forceinline__ void twisted_inverse_iteration(const double* ap, double* y, double* F, double* red, int N, int kt,
+                                                          double b, double c, double sigma, double tiny) {
+  constexpr int CH = 32;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kb = N - 2 - kt;
+  double2* ru = reinterpret_cast<double2*>(F);
+  double2* lm = ru + N;
+  double* z = reinterpret_cast<double*>(lm + N);
+  for (int t = tid; t < N; t += NT) z[t] = ap[t] - sigma;
+  __syncthreads();
+  // this lane's side: rows of them from position r0 on
+  const bool bot = lane & 1;
+  const int rows = bot ? kb : kt, r0 = bot ? kt + 2 : 0;
+  const double c2 = c * c, rtiny = 1.0 / tiny;
+  // forward solve of a row range: z_i = y_i - l_{i-1} z_{i-1} - m_{i-2} z_{i-2}
+  double z1 = 0.0, z2 = 0.0, lm1 = 0.0, mm1 = 0.0, mm2 = 0.0;
+  auto forward = [&](int i0, int i1) {
+    auto step = [&](double* zp, double yi, double2 q) {
+      const double zi = fma(-mm2, z2, fma(-lm1, z1, yi));
+      *zp = zi;
+      z2 = z1;
+      z1 = zi;
+      mm2 = mm1;
+      mm1 = q.y;
+      lm1 = q.x;
+    };
+    const double* yp = y + r0 + i0;
+    const double2* qp = lm + r0 + i0;
+    double* zp = z + r0 + i0;
+    int n = i1 - i0;
+    for (; n >= 8; n -= 8, yp += 8, qp += 8, zp += 8) {
+      double yv[8];
+      double2 qv[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        yv[u] = yp[u];
+        qv[u] = qp[u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) step(zp + u, yv[u], qv[u]);
+    }
+    for (; n > 0; --n, ++yp, ++qp, ++zp) step(zp, *yp, *qp);
+  };
+  double rm1 = 0.0, rm2 = 0.0, um1 = 0.0;
+  auto factor = [&](int i0, int i1) {
+    auto step = [&](double2* p, double as) {
+      const double d = fma(-um1 * um1, rm1, fma(-c2, rm2, as));
+      const double r = fmin(fmax(rcp64(d), -rtiny), rtiny);
+      const double u = fma(-c * rm1, um1, b);
+      *p = make_double2(r, u);
+      rm2 = rm1;
+      rm1 = r;
+      um1 = u;
+    };
+    const double* zp = z + r0 + i0;
+    double2* p = ru + r0 + i0;
+    int n = i1 - i0;
+    for (; n >= 8; n -= 8, zp += 8, p += 8) {
+      double av[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) av[u] = zp[u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) step(p + u, av[u]);
+    }
+    for (; n > 0; --n, ++zp, ++p) step(p, *zp);
+  };
+  const int nch = (max(kt, kb) + CH - 1) / CH;
+  for (int ch = 0; ch <= nch; ++ch) {
+    if (wv == 0 && ch < nch) {
+      if (lane < 2) factor(ch * CH, min(rows, ch * CH + CH));
+    } else if (wv == 1 && ch > 0) {
+      const int i = (ch - 1) * CH + (lane & (CH - 1));
+      const bool lower = lane >= CH;
+      if (i < (lower ? kb : kt)) {
+        const int row = lower ? kt + 2 + i : i;
+        const double2 q = ru[row];
+        lm[row] = make_double2(q.y * q.x, c * q.x);
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (lane < 2) forward((ch - 1) * CH, min(rows, ch * CH));
+    }
+    __syncthreads();
+  }
+  for (int it = 0; it < 2; ++it) {
+    // the middle pair, by every thread: the state of both sides from their last two rows
+    double xk, xk1;
+    {
+      auto side = [&](int n, int e0) {
+        SideZ q{};
+        if (n >= 1) {
+          const double2 p = ru[e0 + n - 1], w = lm[e0 + n - 1];
+          q.s.r1 = p.x;
+          q.s.u1 = p.y;
+          q.l1 = w.x;
+          q.m1 = w.y;
+          q.z1 = z[e0 + n - 1];
+        }
+        if (n >= 2) {
+          q.s.r2 = ru[e0 + n - 2].x;
+          q.m2 = lm[e0 + n - 2].y;
+          q.z2 = z[e0 + n - 2];
+        }
+        return q;
+      };
+      const SideZ zt = side(kt, 0), zb = side(kb, kt + 2);
+      middle_solve(zt.s, zb.s, zt, zb, ap[kt], ap[kt + 1], y[kt], y[kt + 1], b, c, sigma, tiny, xk, xk1);
+    }
+    __syncthreads();
+    for (int t = tid; t < N; t += NT)
+      if (t < kt || t > kt + 1) z[t] *= ru[t].x;  // z / d
+    __syncthreads();
+    if (tid < 2) {
+      // back substitution of a side toward its outer end
+      double x1 = bot ? xk1 : xk, x2 = bot ? xk : xk1;
+      auto step = [&](double* yp, double w, double2 q) {
+        const double xi = fma(-q.y, x2, fma(-q.x, x1, w));
+        *yp = xi;
+        x2 = x1;
+        x1 = xi;
+      };
+      int n = rows;
+      double* yp = y + r0 + n - 8;
+      const double* wp = z + r0 + n - 8;
+      const double2* qp = lm + r0 + n - 8;
+      for (; n >= 8; n -= 8, yp -= 8, wp -= 8, qp -= 8) {
+        double w8[8];
+        double2 qv[8];
+#pragma unroll
+        for (int u = 7; u >= 0; --u) {
+          w8[u] = wp[u];
+          qv[u] = qp[u];
+        }
+#pragma unroll
+        for (int u = 7; u >= 0; --u) step(yp + u, w8[u], qv[u]);
+      }
+      for (; n > 0; --n) step(y + r0 + n - 1, z[r0 + n - 1], lm[r0 + n - 1]);
+      if (tid == 0) {
+        y[kt] = xk;
+        y[kt + 1] = xk1;
+      }
+    }
+    __syncthreads();
+    double nrm[1] = {0.0};
+    for (int t = tid; t < N; t += NT) {
+      const double x = y[side_pos(t, N, kt)];
+      nrm[0] = fma(x, x, nrm[0]);
+    }
+    block_sum<1>(nrm, red);
+    const double sc = 1.0 / sqrt(nrm[0]);
+    for (int t = tid; t < N; t += NT) y[t] *= sc;
+    __syncthreads();
+    if (it == 0) {
+      z1 = z2 = lm1 = mm1 = mm2 = 0.0;
+      if (tid < 2) forward(0, rows);
+      __syncthreads();
+    }
+  }
+}
+
+// One eigenpair per workgroup: the multisection bracket of the eigenvalue down to 1e-9 relative (4 to 6 rounds of
+// 128 counts), then two inverse-iteration solves at its middle.  A round of counts is 11 us at N = 513, so:
+//   - the eigenvalue itself is found first.  Warm and moved by less than 1e-4 in the last SCF iteration: one wave
+//     refines the previous orbital (band_wave.h, 5 us a solve) and confirms its index with one count.  Else one
+//     or two rounds over 2 Ha about the last value (cold: two or three from the bottom of the spectrum) leave
+//     a bracket of ISOLATED at most whose neighbours' are APART intervals away, so that the solves at
+//     its middle converge at once, and the refinement runs inside it;
+//   - the rounds then follow without counting: a shift has more than j eigenvalues below it exactly if it lies
+//     above the j-th.  Where the refinement does not confirm the pair, they count as before.
+//   - The two solves: twisted_inverse_iteration.
+// The bracket, its middle and the solves are those of counting every round, so the orbitals are the same to the
+// bit; solving in parallel there too is as fast and as accurate, but moves the orbitals of nearly degenerate
+// pairs by their own rounding, 1e-13 over the gap.
+// Bound by the dependent chain of one pair: 55..75 us, of which the two solves 30.  A launch at N = 513: 3 systems
+// 69 us (91 with every round counted and the four phases of the solves in sequence), 64 systems x 5 pairs
+// 99 us (120), 601 systems 309 us (364).
+// ISOLATED: a round over 2 Ha leaves intervals of 2 / 127, the first bracket that a second one would not pay for.
+// APART: the first solve then shrinks the neighbours' parts by 1 / 9 or more; at 1 one pair in ten took 6 solves or
+// ended at a neighbour, and the launch waits for the slowest (batch of 64: 144 us).
+constexpr double ISOLATED = 1.6e-2;
+constexpr int APART = 4;
 __global__ __launch_bounds__(NT) void k_eigen(EigArgs e) {
   extern __shared__ double smem[];
   const int pair = e.pairs[blockIdx.x];  // (system << 8) | eigen index; -1 past the last pair
@@ -1036,146 +1324,140 @@ __global__ __launch_bounds__(NT) void k_eigen(EigArgs e) {
   const int N = e.N;
   double* a = smem;         // N    diagonal T_ii + v_i
   double* y = a + N;        // N    inverse-iteration vector
-  double* F = y + N;        // 4N   LDL^T factors and forward-solve values
-  double* red = F + 4 * N;  // 16
-  __shared__ double sh_lo, sh_hi;
-  __shared__ int sh_first[NWAVE];
+  double* F = y + N;        // wave_doubles(N)
+  double* red = F + wave_doubles(N);  // 16
+  double* ap = red + 16;    // N    the diagonal in the order of side_pos
+  __shared__ double sh_rho;
+  __shared__ int sh_first[3][NWAVE], sh_ok;
   const double* pot = e.pot + (size_t)s * N;
+  double* v = e.vec + ((size_t)s * e.K + j) * N;
+  const int kt = (N - 2) / 2, kb = N - 2 - kt;
   double amin = 1e300, amax = -1e300, aabs = 0.0;
   for (int t = tid; t < N; t += NT) {
-    const double v = e.Td + pot[t];
-    a[t] = v;
-    amin = fmin(amin, v);
-    amax = fmax(amax, v);
-    aabs = fmax(aabs, fabs(v));
+    const double d = e.Td + pot[t];
+    a[t] = d;
+    ap[side_pos(t, N, kt)] = d;
+    amin = fmin(amin, d);
+    amax = fmax(amax, d);
+    aabs = fmax(aabs, fabs(d));
   }
   const double off = 2.0 * (fabs(e.Tb) + fabs(e.Tc));
-  const double gl = -block_max(-amin, red) - off;
-  const double gu = block_max(amax, red) + off;
+  Bracket br;
+  br.gl = -block_max(-amin, red) - off;
+  br.gu = block_max(amax, red) + off;
   const double hnorm = block_max(aabs, red) + off;
   // Cold start: the wanted states are the lowest few, so the first bracket is the bottom 40 Ha
   // of the Gershgorin interval (a miss widens it to the top bound after one round).
-  double lo = gl, hi = fmin(gu, gl + 40.0);
+  br.lo = br.gl;
+  br.hi = fmin(br.gu, br.gl + 40.0);
   const bool warm = e.st && e.st[4 * s + 2] && e.eig_prev;
+  const double moved = warm ? fabs(e.eig_delta[(size_t)s * e.K + j]) : 0.0;
   if (warm) {
     const double p = e.eig_prev[(size_t)s * e.K + j];
-    const double w = 3.0 * fabs(e.eig_delta[(size_t)s * e.K + j]) + 1e-9 * fmax(1.0, fabs(p));
-    lo = fmax(gl, p - w);
-    hi = fmin(gu, p + w);
-    if (!(hi > lo)) {
-      lo = gl;
-      hi = gu;
+    const double w = 3.0 * moved + 1e-9 * fmax(1.0, fabs(p));
+    br.lo = fmax(br.gl, p - w);
+    br.hi = fmin(br.gu, p + w);
+    if (!(br.hi > br.lo)) {
+      br.lo = br.gl;
+      br.hi = br.gu;
     }
   }
-  int nrounds = 0;
-  // Multisection: NS shifts per round (both ends included) until the bracket of the j-th
-  // eigenvalue is 1e-9 relative; two inverse-iteration solves and the Rayleigh quotient then
-  // give the eigenpair to ~1e-13.  For N >= 4 each shift is counted by a pair of lanes, the even
-  // lane eliminating the top rows 0..kt-1 and the odd lane the bottom rows N-1..kt+2 (half the
-  // recurrence each), joined through the 2x2 block of rows kt, kt+1.
-  const bool two = N >= 4;
-  const int kt = (N - 2) / 2, kb = N - 2 - kt;
-  const int NS = two ? NT / 2 : NT, me = two ? tid >> 1 : tid;
-  for (int round = 0; round < 80; ++round) {
-    const double mid = 0.5 * (lo + hi);
-    const double tol = 1e-9 * fmax(1.0, fabs(mid)) + 64.0 * EPS * hnorm;
-    if (hi - lo <= tol) break;
-    ++nrounds;
-    const double step = (hi - lo) / (double)(NS - 1);
-    const double sig = me == NS - 1 ? hi : fma((double)me, step, lo);
-    int cnt;
-    if (two) {
-      const bool bot = tid & 1;
-      const Side h = sturm_side(bot ? a + N - 1 : a, bot ? -1 : 1, bot ? kb : kt, e.Tb, e.Tc, sig);
-      const Side o{__shfl_xor(h.r1, 1, 64), __shfl_xor(h.r2, 1, 64), __shfl_xor(h.u1, 1, 64), __shfl_xor(h.neg, 1, 64)};
-      cnt = bot ? sturm_join(o, h, a[kt], a[kt + 1], e.Tb, e.Tc, sig) : sturm_join(h, o, a[kt], a[kt + 1], e.Tb, e.Tc, sig);
-    } else {
-      cnt = sturm_count(a, N, e.Tb, e.Tc, sig);
-    }
-    const unsigned long long m = __ballot(cnt > j);
-    if ((tid & 63) == 0) sh_first[tid >> 6] = m ? (((__ffsll((long long)m) - 1) + (tid & ~63)) >> (two ? 1 : 0)) : NS;
+  // the eigenvalue by wave 0 (sh_rho), true if found
+  auto refine = [&](double slo, double shi, bool check) {
     __syncthreads();
-    int first = NS;
-#pragma unroll
-    for (int q = 0; q < NWAVE; ++q) first = min(first, sh_first[q]);
-    if (tid == 0) {
-      // the eigenvalue lies outside the bracket: the next one is the adjacent interval 256 times
-      // as wide (clipped to the Gershgorin bounds), so a missed warm start costs about one round
-      const double wide = 256.0 * (hi - lo);
-      if (first == 0) {
-        sh_hi = lo;
-        sh_lo = fmax(gl, lo - wide);
-        if (!(sh_lo < lo)) sh_lo = lo > gl ? gl : lo;
-      } else if (first == NS) {
-        sh_lo = hi;
-        sh_hi = fmin(gu, hi + wide);
-        if (!(sh_hi > hi)) sh_hi = hi < gu ? gu : hi;
-      } else {
-        sh_lo = first - 1 == 0 ? lo : fma((double)(first - 1), step, lo);
-        sh_hi = first == NS - 1 ? hi : fma((double)first, step, lo);
+    if (tid < 64) {
+      double rho = 0.0;
+      const bool ok = refine_eigenvalue(a, y, F, N, e.Tb, e.Tc, hnorm, j, slo, shi, check, &rho);
+      if (tid == 0) {
+        sh_ok = ok;
+        sh_rho = rho;
       }
     }
     __syncthreads();
-    const double nlo = sh_lo, nhi = sh_hi;
+    return sh_ok != 0;
+  };
+  // One round of counts: each shift by a pair of lanes, the even lane eliminating the top rows 0..kt-1 and
+  // the odd lane the bottom rows N-1..kt+2 (half the recurrence each), joined through the 2x2 block of rows
+  // kt, kt+1.  Returns the first shift with more than j eigenvalues below it; apart: the intervals between the
+  // j-th eigenvalue's and those of its neighbours.
+  constexpr int NS = NT / 2;
+  const int me = tid >> 1;
+  const bool bot = tid & 1;
+  int nrounds = 0;
+  int apart = 0;
+  auto count = [&](const Bracket& q, double st) {
+    ++nrounds;
+    const double sig = q.shift(me, NS, st);
+    const Side h = sturm_side(bot ? ap + kt + 2 : ap, 1, bot ? kb : kt, e.Tb, e.Tc, sig);
+    const Side o{__shfl_xor(h.r1, 1, 64), __shfl_xor(h.r2, 1, 64), __shfl_xor(h.u1, 1, 64), __shfl_xor(h.neg, 1, 64)};
+    const int cnt = bot ? sturm_join(o, h, a[kt], a[kt + 1], e.Tb, e.Tc, sig)
+                        : sturm_join(h, o, a[kt], a[kt + 1], e.Tb, e.Tc, sig);
+    // first shifts above the eigenvalues j - 1, j and j + 1
+    int first[3];
     __syncthreads();
-    if (nlo == lo && nhi == hi) break;  // no progress possible (rounding floor)
-    lo = nlo;
-    hi = nhi;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const unsigned long long m = __ballot(cnt > j - 1 + k);
+      if ((tid & 63) == 0) sh_first[k][tid >> 6] = m ? (((__ffsll((long long)m) - 1) + (tid & ~63)) >> 1) : NS;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      first[k] = NS;
+#pragma unroll
+      for (int w = 0; w < NWAVE; ++w) first[k] = min(first[k], sh_first[k][w]);
+    }
+    apart = min(j == 0 ? NS : first[1] - first[0], first[2] - first[1]);
+    return first[1];
+  };
+  // ---- the eigenvalue ----
+  bool known = false;
+  if (warm && moved < 1e-4) {
+    for (int t = tid; t < N; t += NT) y[t] = v[t];
+    known = refine(br.gl, br.gu, true);
   }
-  const double sigma = 0.5 * (lo + hi);
+  if (!known) {
+    Bracket q = br;
+    if (warm) {
+      const double mid = 0.5 * (br.lo + br.hi), w = fmax(0.5 * (br.hi - br.lo), 1.0);
+      q.lo = fmax(br.gl, mid - w);
+      q.hi = fmin(br.gu, mid + w);
+    }
+    for (int round = 0; round < 4; ++round) {
+      const double st = q.step(NS);
+      const int first = count(q, st);
+      if (!q.narrow(first, NS, st) || first == 0 || first == NS) continue;
+      if (apart < APART || q.hi - q.lo > ISOLATED * fmax(1.0, 0.5 * fabs(q.lo + q.hi))) continue;
+      for (int t = tid; t < N; t += NT) y[t] = warm ? v[t] + 1e-3 * start_value(t, j) : start_value(t, j);
+      known = refine(q.lo, q.hi, false);
+      break;
+    }
+  }
+  // ---- the bracket ----
+  for (int round = 0; round < 80 && !br.small(hnorm); ++round) {
+    const double st = br.step(NS);
+    int first;
+    if (known) {
+      const double rho = sh_rho, f = (rho - br.lo) / st;
+      first = f < 0.0 ? 0 : f > (double)NS ? NS : (int)f;
+      while (first > 0 && br.shift(first - 1, NS, st) > rho) --first;
+      while (first < NS && !(br.shift(first, NS, st) > rho)) ++first;
+    } else {
+      first = count(br, st);
+    }
+    if (!br.narrow(first, NS, st)) break;
+  }
+  const double sigma = 0.5 * (br.lo + br.hi);
   if (e.stats && tid == 0) {
     atomicAdd(&e.stats[0], (unsigned long long)nrounds);
     atomicAdd(&e.stats[1], 1ull);
   }
-  // inverse iteration: one LDL^T factorisation, two solves, normalised in between
-  double* v = e.vec + ((size_t)s * e.K + j) * N;
-  for (int t = tid; t < N; t += NT) y[t] = warm ? v[t] + 1e-3 * start_value(t, j) : start_value(t, j);
   __syncthreads();
-  // For N >= 4 lanes 0 and 1 of wave 0 solve the top and bottom halves (twisted at rows kt, kt+1):
-  // factorisation and forward solve of each side, the middle pair, then each side's back
-  // substitution outward.  F rows of the bottom side are stored at their own row indices.
-  Side fs{};
-  for (int it = 0; it < 2; ++it) {
-    if (two) {
-      if (tid < 2) {
-        const bool bot = tid == 1;
-        const int st = bot ? -1 : 1, rows = bot ? kb : kt;
-        double* Fs = bot ? F + 4 * (N - 1) : F;
-        double* ys = bot ? y + N - 1 : y;
-        const SideZ z = it == 0 ? ldlt_side_factor_forward(bot ? a + N - 1 : a, ys, st, rows, e.Tb, e.Tc, sigma,
-                                                           EPS * hnorm, Fs)
-                                : ldlt_side_forward(ys, st, rows, Fs);
-        if (it == 0) fs = z.s;
-        const Side os{__shfl_xor(fs.r1, 1, 64), __shfl_xor(fs.r2, 1, 64), __shfl_xor(fs.u1, 1, 64), 0};
-        const SideZ oz{os, __shfl_xor(z.l1, 1, 64), __shfl_xor(z.m1, 1, 64), __shfl_xor(z.m2, 1, 64),
-                       __shfl_xor(z.z1, 1, 64), __shfl_xor(z.z2, 1, 64)};
-        double xk, xk1;
-        if (bot)
-          middle_solve(os, fs, oz, z, a[kt], a[kt + 1], y[kt], y[kt + 1], e.Tb, e.Tc, sigma, EPS * hnorm, xk, xk1);
-        else
-          middle_solve(fs, os, z, oz, a[kt], a[kt + 1], y[kt], y[kt + 1], e.Tb, e.Tc, sigma, EPS * hnorm, xk, xk1);
-        ldlt_side_backward(Fs, st, rows, bot ? xk1 : xk, bot ? xk : xk1, ys);
-        if (tid == 0) {
-          y[kt] = xk;
-          y[kt + 1] = xk1;
-        }
-      }
-    } else if (tid == 0) {
-      if (it == 0)
-        ldlt_factor_forward(a, y, N, e.Tb, e.Tc, sigma, EPS * hnorm, F);
-      else
-        ldlt_forward(y, N, F);
-      ldlt_backward(F, N, y);
-    }
-    __syncthreads();
-    double nrm[1] = {0.0};
-    for (int t = tid; t < N; t += NT) nrm[0] = fma(y[t], y[t], nrm[0]);
-    block_sum<1>(nrm, red);
-    const double sc = 1.0 / sqrt(nrm[0]);
-    for (int t = tid; t < N; t += NT) y[t] *= sc;
-    __syncthreads();
-  }
-  for (int t = tid; t < N; t += NT) v[t] = y[t];
+  for (int t = tid; t < N; t += NT)
+    y[side_pos(t, N, kt)] = warm ? v[t] + 1e-3 * start_value(t, j) : start_value(t, j);
+  __syncthreads();
+  twisted_inverse_iteration(ap, y, F, red, N, kt, e.Tb, e.Tc, sigma, EPS * hnorm);
+  for (int t = tid; t < N; t += NT) v[t] = y[side_pos(t, N, kt)];
   if (tid == 0) e.eig[(size_t)s * e.K + j] = sigma;
 }
 
@@ -1808,7 +2090,7 @@ size_t gmlp_lds_bytes(const Dev1& a) {
   return ((size_t)a.N + 2 * (size_t)(a.nlay - 1) * a.hmax + NT + 2 * (size_t)a.hmax) * 8;
 }
 
-size_t eigen_lds_bytes(int N) { return (size_t)(6 * N + 16) * 8; }
+size_t eigen_lds_bytes(int N) { return (3 * (size_t)N + wave_doubles(N) + 16) * 8; }
 
 void kinetic(double dx, double* Td, double* Tb, double* Tc) {
   // T = -1/2 L / dx^2 with L = (-1/12, 4/3, -5/2, 4/3, -1/12)
