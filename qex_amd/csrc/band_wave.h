@@ -45,6 +45,16 @@ __device__ __forceinline__ Sym2 inverse(Sym2 d) {
   const double r = rcp_clamped(fma(d.p, d.s, -(d.q * d.q)));
   return {d.s * r, -d.q * r, d.p * r};
 }
+// D x = z by elimination with row pivoting: the last block of a singular A - sigma keeps its regular direction (the
+// determinant's rounding would scale it)
+__device__ __forceinline__ Vec2 solve(Sym2 d, Vec2 z) {
+  const bool sw = fabs(d.p) < fabs(d.q);
+  const double a = sw ? d.q : d.p, b = sw ? d.s : d.q, c = sw ? d.p : d.q, e = sw ? d.q : d.s;
+  const double za = sw ? z.y : z.x, zb = sw ? z.x : z.y;
+  const double r = rcp_clamped(a), l = c * r;
+  const double y = fma(-l, za, zb) * rcp_clamped(fma(-l, b, e));
+  return {fma(-b, y, za) * r, y};
+}
 // negative eigenvalues of the block: signs of p and of det / p
 __device__ __forceinline__ int negatives(Sym2 d) {
   const int a = sign_bit(d.p);
@@ -139,7 +149,7 @@ __device__ __forceinline__ int wave_solve(const double* a, double* y, int N, dou
     const bool stays = (p & (2 * h - 1)) == 2 * h - 1;      // its neighbours are
     const Sym2 I = inverse(D);
     const Mat2 W = mul(I, E);
-    const Vec2 v = SOLVE ? mul(I, Zr) : Vec2{0.0, 0.0};
+    const Vec2 v = SOLVE ? solve(D, Zr) : Vec2{0.0, 0.0};
     if (mine) {
       neg += negatives(D);
       if (SOLVE) {
@@ -176,7 +186,7 @@ __device__ __forceinline__ int wave_solve(const double* a, double* y, int N, dou
   for (int bit = 0; bit < 6; ++bit) total += __popcll(__ballot((neg >> bit) & 1)) << bit;
   if (!SOLVE) return total;
   // back through the levels: x_e = v_e - W_e x_(e-h) - (E_r D_e^-1)^T x_r, r = e + h
-  Vec2 x = mul(inverse(D), Zr);  // (lane 63)
+  Vec2 x = solve(D, Zr);  // (lane 63)
 #pragma unroll
   for (int t = 5; t >= 0; --t) {
     const int h = 1 << t;

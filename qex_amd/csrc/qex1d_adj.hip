@@ -9,8 +9,7 @@
 //   energy           nob += c (-v_KS + v_H(n_out) + v_xc(n_out) + v_ext), thetabar += c dF(n_out)/dtheta,
 //                    c = dE_k dx (the eigenvalue sum and -dx v_KS.n_out cancel at fixed n_out)
 //   k_adj_eig        vbar = sum_j occ_j (2/dx) psi_j * y_j with y_j = -(H - eps_j)^-1 Q (nob psi_j)
-//                    (Q projects out the occupied orbitals; a banded LU with partial pivoting in
-//                    LDS, then Q again) minus the pairs of occupied orbitals with unequal occupations
+//                    (Q projects out the occupied orbitals) minus the pairs of occupied orbitals with unequal occupations
 //   Hartree + XC     nbar += dx U vbar + H_F vbar, thetabar += d(vbar . grad F)/dtheta, F = sum e(n) n
 // The MLP terms come from reverse mode over the network's forward and forward-tangent passes, one
 // wavefront per point with one lane per hidden unit; each wavefront accumulates its parameter
@@ -27,6 +26,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "band_wave.h"
 #include "prof.h"
 #include "qex.h"
 
@@ -61,6 +61,19 @@ __device__ double bsum(double x, double* red) {
   __syncthreads();
   double s = 0.0;
   for (int q = 0; q < (int)(blockDim.x >> 6); ++q) s += red[q];
+  __syncthreads();
+  return s;
+}
+
+__device__ double bmax(double x, double* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  __syncthreads();
+  if (l == 0) red[w] = x;
+  __syncthreads();
+  double s = 0.0;
+  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) s = fmax(s, red[q]);
   __syncthreads();
   return s;
 }
@@ -605,8 +618,92 @@ __global__ void k_adj_scales(Adj a, int k, double* cs, double* ones) {
   ones[s] = 1.0;
 }
 
-// eigen adjoint, one workgroup per system.  LDS: H diagonal, r, y, vbar and the rows of U of the
-// banded LU factorisation (row i holds columns i .. i + 4).
+// Fallback of k_adj_eig, one thread: y <- (H - ej)^-1 y by Gaussian elimination with partial pivoting (bandwidth 2,
+// fill to 4).  The three active rows (columns i .. i + 4) are in registers; each finished row of U (5 entries)
+// goes to R and its right-hand side to y, then the back substitution.  Pivots below tiny become +-tiny.
+__device__ __attribute__((noinline)) void pivoted_solve(const double* hd, double* y, double* R, int N, double Tb, double Tc,
+                                                        double ej, double tiny) {
+  auto band = [&](int row, int col) -> double {  // entry of H - eps_j (zero outside the matrix)
+    if (row >= N || col < 0 || col >= N) return 0.0;
+    const int d = col - row;
+    return d == 0 ? hd[row] - ej : (d == 1 || d == -1) ? Tb : (d == 2 || d == -2) ? Tc : 0.0;
+  };
+  double r0[5], r1[5], r2[5];
+  for (int c = 0; c < 5; ++c) {
+    r0[c] = band(0, c);
+    r1[c] = band(1, c);
+    r2[c] = band(2, c);
+  }
+  double y0 = y[0], y1 = N > 1 ? y[1] : 0.0, y2 = N > 2 ? y[2] : 0.0;
+  for (int i = 0; i < N; ++i) {
+    // pivot among the (existing) rows i, i+1, i+2 in column i
+    int pr = 0;
+    double best = fabs(r0[0]);
+    if (i + 1 < N && fabs(r1[0]) > best) {
+      best = fabs(r1[0]);
+      pr = 1;
+    }
+    if (i + 2 < N && fabs(r2[0]) > best) pr = 2;
+    if (pr == 1) {
+      for (int c = 0; c < 5; ++c) {
+        const double t1 = r0[c];
+        r0[c] = r1[c];
+        r1[c] = t1;
+      }
+      const double ty = y0;
+      y0 = y1;
+      y1 = ty;
+    } else if (pr == 2) {
+      for (int c = 0; c < 5; ++c) {
+        const double t1 = r0[c];
+        r0[c] = r2[c];
+        r2[c] = t1;
+      }
+      const double ty = y0;
+      y0 = y2;
+      y2 = ty;
+    }
+    if (fabs(r0[0]) < tiny) r0[0] = r0[0] < 0.0 ? -tiny : tiny;
+    const double ip = 1.0 / r0[0];
+    const double l1 = r1[0] * ip, l2 = r2[0] * ip;
+    for (int c = 1; c < 5; ++c) {
+      r1[c] = fma(-l1, r0[c], r1[c]);
+      r2[c] = fma(-l2, r0[c], r2[c]);
+    }
+    y1 = fma(-l1, y0, y1);
+    y2 = fma(-l2, y0, y2);
+    for (int c = 0; c < 5; ++c) R[(size_t)i * 5 + c] = r0[c];
+    y[i] = y0;
+    // advance: rows i+1, i+2 shift one column left; row i+3 enters
+    for (int c = 0; c < 4; ++c) {
+      r0[c] = r1[c + 1];
+      r1[c] = r2[c + 1];
+    }
+    r0[4] = 0.0;
+    r1[4] = 0.0;
+    for (int c = 0; c < 5; ++c) r2[c] = band(i + 3, i + 1 + c);
+    y0 = y1;
+    y1 = y2;
+    y2 = i + 3 < N ? y[i + 3] : 0.0;
+  }
+  for (int i = N - 1; i >= 0; --i) {
+    double v = y[i];
+    for (int c = 1; c < 5 && i + c < N; ++c) v = fma(-R[(size_t)i * 5 + c], y[i + c], v);
+    y[i] = v / R[(size_t)i * 5];
+  }
+}
+
+// eigen adjoint, one workgroup per system.
+//
+// Bound by the dependent chain of the banded solves.  One thread eliminating with partial pivoting takes 0.7 us a
+// row; the substructured solve of one wave (band_wave.h) takes 5 us at N = 513 but does not pivot, so each solution
+// is refined on its residual inside the complement of the occupied orbitals until that is at the rounding of
+// (H - eps_j) x, and a system where SOLVES of them do not get there goes to the pivoted elimination.
+// One occupied orbital: N = 513 (32 systems) 386 -> 22 us a launch, N = 257 190 -> 15 us; one solve is at rounding
+// there, so most of what is left is latency of the projections and loads.
+// LDS: H diagonal, r, y, vbar, x, w and the factors of the wave (the rows of U of the pivoted elimination).
+constexpr int SOLVES = 5;
+size_t adj_eig_lds(int N) { return ((size_t)6 * N + qexband::wave_doubles(N)) * 8; }
 __global__ __launch_bounds__(NT) void k_adj_eig(Adj a, int k, double Td, double Tb, double Tc) {
   extern __shared__ double sm[];
   __shared__ double red[NT / 64];
@@ -616,132 +713,88 @@ __global__ __launch_bounds__(NT) void k_adj_eig(Adj a, int k, double Td, double 
   double* r = hd + N;    // N
   double* y = r + N;     // N
   double* vb = y + N;    // N
-  double* R = vb + N;    // N x 5 rows of U
+  double* x = vb + N;    // N
+  double* w = x + N;     // N
+  double* F = w + N;     // factors
   const int ne = a.ne[s], nocc = (ne + 1) / 2;
   const double* vxc = a.vxc + ((size_t)s * T + k) * N;
   const double* vh = a.vh + ((size_t)s * T + k) * N;
   const double* ve = a.vext + (size_t)s * N;
   const double* psi = a.orb + ((size_t)s * T + k) * a.K * N;
   const double* nob = a.nob + (size_t)s * N;
+  double hmax = 0.0;
   for (int t = threadIdx.x; t < N; t += NT) {
-    hd[t] = Td + ve[t] + vh[t] + vxc[t];
+    const double h = Td + ve[t] + vh[t] + vxc[t];
+    hd[t] = h;
+    hmax = fmax(hmax, fabs(h));
     vb[t] = 0.0;
   }
-  __syncthreads();
+  hmax = bmax(hmax, red);
+  // (H p)_t of a vector in memory or LDS
+  auto apply = [&](const double* p, int t) {
+    double hx = hd[t] * p[t];
+    if (t >= 1) hx = fma(Tb, p[t - 1], hx);
+    if (t + 1 < N) hx = fma(Tb, p[t + 1], hx);
+    if (t >= 2) hx = fma(Tc, p[t - 2], hx);
+    if (t + 2 < N) hx = fma(Tc, p[t + 2], hx);
+    return hx;
+  };
   // eigenvalues as Rayleigh quotients of the stored orbitals
   for (int j = 0; j < nocc; ++j) {
     const double* pj = psi + (size_t)j * N;
     double q = 0.0;
-    for (int t = threadIdx.x; t < N; t += NT) {
-      double hx = hd[t] * pj[t];
-      if (t >= 1) hx = fma(Tb, pj[t - 1], hx);
-      if (t + 1 < N) hx = fma(Tb, pj[t + 1], hx);
-      if (t >= 2) hx = fma(Tc, pj[t - 2], hx);
-      if (t + 2 < N) hx = fma(Tc, pj[t + 2], hx);
-      q = fma(pj[t], hx, q);
-    }
+    for (int t = threadIdx.x; t < N; t += NT) q = fma(pj[t], apply(pj, t), q);
     q = bsum(q, red);
     if (threadIdx.x == 0) eps[j] = q;
   }
   __syncthreads();
-  __shared__ double hmax;
-  if (threadIdx.x == 0) {
-    double hn = 0.0;
-    for (int t = 0; t < N; ++t) hn = fmax(hn, fabs(hd[t]));
-    hmax = hn;
-  }
-  __syncthreads();
-  // zero pivots are replaced by +-eps |H| (the solution's component along psi_j is projected out)
-  const double tiny = 2.220446049250313e-16 * (hmax + 2.0 * fabs(Tb) + 2.0 * fabs(Tc));
-  for (int j = 0; j < nocc; ++j) {
-    const double* pj = psi + (size_t)j * N;
-    const double oj = occupation(ne, j);
-    for (int t = threadIdx.x; t < N; t += NT) r[t] = nob[t] * pj[t];
-    __syncthreads();
-    // rhs = Q r
-    for (int t = threadIdx.x; t < N; t += NT) y[t] = r[t];
-    __syncthreads();
+  const double hnorm = hmax + 2.0 * fabs(Tb) + 2.0 * fabs(Tc), rounding = 2.220446049250313e-16 * hnorm;
+  // v <- Q v, the occupied orbitals projected out one after another
+  auto project = [&](double* v) {
     for (int b = 0; b < nocc; ++b) {
       const double* pb = psi + (size_t)b * N;
       double d = 0.0;
-      for (int t = threadIdx.x; t < N; t += NT) d = fma(pb[t], r[t], d);
+      for (int t = threadIdx.x; t < N; t += NT) d = fma(pb[t], v[t], d);
       d = bsum(d, red);
-      for (int t = threadIdx.x; t < N; t += NT) y[t] = fma(-d, pb[t], y[t]);
-      __syncthreads();
+      for (int t = threadIdx.x; t < N; t += NT) v[t] = fma(-d, pb[t], v[t]);
     }
-    // (H - eps_j) x = y by Gaussian elimination with partial pivoting (bandwidth 2, fill to 4):
-    // one lane keeps the three active rows (columns i .. i + 4) in registers, stores each finished
-    // row of U (5 entries) and its right-hand side in LDS, then back-substitutes.
-    const double ej = eps[j];
-    if (threadIdx.x == 0) {
-      auto band = [&](int row, int col) -> double {  // entry of H - eps_j (zero outside the matrix)
-        if (row >= N || col < 0 || col >= N) return 0.0;
-        const int d = col - row;
-        return d == 0 ? hd[row] - ej : (d == 1 || d == -1) ? Tb : (d == 2 || d == -2) ? Tc : 0.0;
-      };
-      double r0[5], r1[5], r2[5];
-      for (int c = 0; c < 5; ++c) {
-        r0[c] = band(0, c);
-        r1[c] = band(1, c);
-        r2[c] = band(2, c);
+  };
+  for (int j = 0; j < nocc; ++j) {
+    const double* pj = psi + (size_t)j * N;
+    const double oj = occupation(ne, j), ej = eps[j];
+    // rhs = Q r
+    for (int t = threadIdx.x; t < N; t += NT) {
+      const double v = nob[t] * pj[t];
+      r[t] = v;
+      y[t] = v;
+      x[t] = 0.0;
+    }
+    project(y);
+    for (int t = threadIdx.x; t < N; t += NT) w[t] = y[t];
+    bool solved = false;
+    for (int it = 0; it < SOLVES && !solved; ++it) {
+      __syncthreads();
+      if (threadIdx.x < 64) qexband::wave_solve<true>(hd, w, N, Tb, Tc, ej, F);
+      __syncthreads();
+      project(w);
+      double xx = 0.0, rr = 0.0;
+      for (int t = threadIdx.x; t < N; t += NT) {
+        x[t] += w[t];
+        xx = fma(x[t], x[t], xx);
       }
-      double y0 = y[0], y1 = N > 1 ? y[1] : 0.0, y2 = N > 2 ? y[2] : 0.0;
-      for (int i = 0; i < N; ++i) {
-        // pivot among the (existing) rows i, i+1, i+2 in column i
-        int pr = 0;
-        double best = fabs(r0[0]);
-        if (i + 1 < N && fabs(r1[0]) > best) {
-          best = fabs(r1[0]);
-          pr = 1;
-        }
-        if (i + 2 < N && fabs(r2[0]) > best) pr = 2;
-        if (pr == 1) {
-          for (int c = 0; c < 5; ++c) {
-            const double t1 = r0[c];
-            r0[c] = r1[c];
-            r1[c] = t1;
-          }
-          const double ty = y0;
-          y0 = y1;
-          y1 = ty;
-        } else if (pr == 2) {
-          for (int c = 0; c < 5; ++c) {
-            const double t1 = r0[c];
-            r0[c] = r2[c];
-            r2[c] = t1;
-          }
-          const double ty = y0;
-          y0 = y2;
-          y2 = ty;
-        }
-        if (fabs(r0[0]) < tiny) r0[0] = r0[0] < 0.0 ? -tiny : tiny;
-        const double ip = 1.0 / r0[0];
-        const double l1 = r1[0] * ip, l2 = r2[0] * ip;
-        for (int c = 1; c < 5; ++c) {
-          r1[c] = fma(-l1, r0[c], r1[c]);
-          r2[c] = fma(-l2, r0[c], r2[c]);
-        }
-        y1 = fma(-l1, y0, y1);
-        y2 = fma(-l2, y0, y2);
-        for (int c = 0; c < 5; ++c) R[(size_t)i * 5 + c] = r0[c];
-        y[i] = y0;
-        // advance: rows i+1, i+2 shift one column left; row i+3 enters
-        for (int c = 0; c < 4; ++c) {
-          r0[c] = r1[c + 1];
-          r1[c] = r2[c + 1];
-        }
-        r0[4] = 0.0;
-        r1[4] = 0.0;
-        for (int c = 0; c < 5; ++c) r2[c] = band(i + 3, i + 1 + c);
-        y0 = y1;
-        y1 = y2;
-        y2 = i + 3 < N ? y[i + 3] : 0.0;
-      }
-      for (int i = N - 1; i >= 0; --i) {
-        double v = y[i];
-        for (int c = 1; c < 5 && i + c < N; ++c) v = fma(-R[(size_t)i * 5 + c], y[i + c], v);
-        y[i] = v / R[(size_t)i * 5];
-      }
+      __syncthreads();
+      for (int t = threadIdx.x; t < N; t += NT) w[t] = fma(ej, x[t], y[t]) - apply(x, t);
+      project(w);
+      for (int t = threadIdx.x; t < N; t += NT) rr = fma(w[t], w[t], rr);
+      rr = bsum(rr, red);
+      xx = bsum(xx, red);
+      solved = rr <= 16.0 * rounding * rounding * xx;
+    }
+    if (!solved) {
+      // (the solution's component along psi_j is projected out)
+      for (int t = threadIdx.x; t < N; t += NT) x[t] = y[t];
+      __syncthreads();
+      if (threadIdx.x == 0) pivoted_solve(hd, x, F, N, Tb, Tc, ej, rounding);
     }
     __syncthreads();
     // x <- Q x; y_j = -x - sum over occupied b with occ_b != occ_j of psi_b (psi_b . r) / (eps_b - eps_j)
@@ -749,19 +802,18 @@ __global__ __launch_bounds__(NT) void k_adj_eig(Adj a, int k, double Td, double 
       const double* pb = psi + (size_t)b * N;
       double d = 0.0, dr = 0.0;
       for (int t = threadIdx.x; t < N; t += NT) {
-        d = fma(pb[t], y[t], d);
+        d = fma(pb[t], x[t], d);
         dr = fma(pb[t], r[t], dr);
       }
       d = bsum(d, red);
       dr = bsum(dr, red);
       const double ob = occupation(ne, b);
       const double extra = (b != j && ob != oj) ? dr / (eps[b] - ej) : 0.0;
-      // y holds x; the final y_j = -(Q x) - sum extra psi_b  ->  accumulate as x - d psi_b + extra psi_b, negated below
-      for (int t = threadIdx.x; t < N; t += NT) y[t] = fma(extra - d, pb[t], y[t]);
-      __syncthreads();
+      // the final y_j = -(Q x) - sum extra psi_b  ->  accumulate as x - d psi_b + extra psi_b, negated below
+      for (int t = threadIdx.x; t < N; t += NT) x[t] = fma(extra - d, pb[t], x[t]);
     }
     const double sc = -oj * 2.0 / a.dx;
-    for (int t = threadIdx.x; t < N; t += NT) vb[t] = fma(sc * pj[t], y[t], vb[t]);
+    for (int t = threadIdx.x; t < N; t += NT) vb[t] = fma(sc * pj[t], x[t], vb[t]);
     __syncthreads();
   }
   for (int t = threadIdx.x; t < N; t += NT) a.vbar[(size_t)s * N + t] = vb[t];
@@ -951,7 +1003,7 @@ int qex1d_kohn_sham_vjp(const qex1d_problem* p, const qex1d_inputs* in, const qe
   const int HL = a.NL == 2 ? a.H2 : a.H1;
   const size_t mlp_lds = (2 * (size_t)a.W * a.H1 + a.H1 + (a.NL == 2 ? 2 * (size_t)a.H1 * a.H2 + a.H2 : 0) + HL +
                           (size_t)(NT / 64) * 6 * 64) * 8;
-  const size_t eig_lds = (size_t)(4 + 5) * a.N * 8;
+  const size_t eig_lds = adj_eig_lds(a.N);
   const bool glob = p->xc_kind == QEX1D_XC_GLOBAL_MLP;
   const size_t gmlp_lds = (2 * (size_t)a.N + 2 * (NT / 64) * 64 + 12 * 64 + 8) * 8;
   if ((!glob && mlp_lds > 150 * 1024) || eig_lds > 150 * 1024)

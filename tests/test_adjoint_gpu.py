@@ -72,6 +72,30 @@ def test_device_gradient_matches_oracle(mods, act, sizes, m):
     np.testing.assert_allclose(g, go, rtol=0, atol=1e-6 * scale)
 
 
+@pytest.mark.parametrize("N,ne", [(33, 1), (65, 7), (319, 4), (320, 7), (321, 4), (513, 7), (1024, 4)])
+def test_gradient_over_grid_sizes_matches_oracle(mods, N, ne):
+    """The orbital response at the edges of the substructured solve's rows per lane, up to four occupied orbitals
+    (single and double occupations): 1e-6 of the largest entry, as for the other gradients."""
+    engine, train, _, _ = mods
+    grids = np.linspace(-12.8, 12.8, N)
+    dx = float(grids[1] - grids[0])
+    z = {1: [1.0], 4: [1.0, 1.0, 2.0], 7: [3.0, 1.0, 3.0]}[ne]
+    loc = np.array([-0.4, 1.3, 2.1])[: len(z)]
+    params = _params(6, [5, 8, 8, 1])
+    n0 = O.gaussian_initial_density(grids, loc, np.array(z), ne, weighted=True)
+    prob = _problem(mods, grids, [(loc, np.array(z), ne)], params, "tanh", 5, 3, 0.4, 0.9, 1)
+    tn = 0.9 * n0
+    loss, g, res = train.value_and_grad(prob, n0[None], train.c3_loss, np.array([-1.0]), tn[None], dx)
+    xc = O.LocalMLP([w for w, _ in params], [b for _, b in params], "tanh", 5, 2.0)
+    fw = A.forward_trajectory(loc, np.array(z), ne, 3, grids, xc, O.exponential_coulomb, n0, 0.4, 0.9, 1)
+    dE = np.zeros(3)
+    dn = np.zeros((3, N))
+    dE[-1] = 2 * (fw["energies"][-1] + 1.0)
+    dn[-1] = 2 * 1e-2 * dx * (fw["densities"][-1] - tn)
+    go = A.backward(fw, dE, dn)
+    np.testing.assert_allclose(g.cpu().numpy(), go, rtol=0, atol=1e-6 * np.abs(go).max())
+
+
 def test_device_gradient_matches_finite_differences(mods):
     engine, train, _, _ = mods
     grids = np.linspace(-12.8, 12.8, 257)
