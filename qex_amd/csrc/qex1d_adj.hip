@@ -11,10 +11,9 @@
 //   k_adj_eig        vbar = sum_j occ_j (2/dx) psi_j * y_j with y_j = -(H - eps_j)^-1 Q (nob psi_j)
 //                    (Q projects out the occupied orbitals) minus the pairs of occupied orbitals with unequal occupations
 //   Hartree + XC     nbar += dx U vbar + H_F vbar, thetabar += d(vbar . grad F)/dtheta, F = sum e(n) n
-// The MLP terms come from reverse mode over the network's forward and forward-tangent passes, one
-// wavefront per point with one lane per hidden unit; each wavefront accumulates its parameter
-// partials in registers, the waves of a workgroup combine them in LDS in a fixed order and add the
-// sum to the workgroup's own slot, and the slots are summed in a fixed order.
+// The MLP terms come from reverse mode over the network's forward and forward-tangent passes on tiles of
+// points (FP64 matrix instructions); each workgroup accumulates its parameter partials in registers and
+// adds them to its own slot, and the slots are summed in a fixed order.
 // A GLOBAL_MLP functional (amplitude encoded: E_xc = dx f(n), v_xc = dx grad f) takes the same
 // steps with F = f in the energy and F = dx f in the potential, through k_adj_gmlp (one workgroup
 // per system); under reflection its functional sees the unflipped densities (the forward flips only
@@ -33,9 +32,8 @@
 namespace {
 
 constexpr int NT = 256;
-constexpr int ADJ_SLOTS = 1024;  // wavefronts of the MLP adjoint launch
-constexpr int ADJ_WG = ADJ_SLOTS / (NT / 64);  // its workgroups = parameter-partial slots
-constexpr int HMAX = 64;        // hidden width (one lane per unit)
+constexpr int ADJ_WG = 256;     // workgroups of the MLP adjoint launch = parameter-partial slots
+constexpr int HMAX = 64;        // hidden width
 constexpr int WMAXW = QEX1D_MAX_MLP_WINDOW;
 thread_local char g_erra[512] = "";
 
@@ -258,191 +256,322 @@ __global__ __launch_bounds__(NT) void k_toeplitz(int N, double dx, const double*
   out[(size_t)s * N + i] = dx * acc;
 }
 
+typedef double d4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// sum over the 16 lanes of a DPP row, in every lane of it
+template <int ROT>
+__device__ __forceinline__ double row_rotated(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x120 + ROT, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x120 + ROT, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double x) {
+  x += row_rotated<8>(x);
+  x += row_rotated<4>(x);
+  x += row_rotated<2>(x);
+  return x + row_rotated<1>(x);
+}
+
 // MLP second-order adjoint.  Per point p = (s, i): x = window(xin[s])_i / norm, tangent
-// xt = window(tin[s])_i / norm (zero without tin), fbar = sf[s] * F1[s][i], fdbar = F2 ? F2[s][i] : 0.
+// xt = window(tin[s])_i / norm, fbar = sf[s] * F1[s][i], fdbar = F2[s][i].
 // Outputs per point: xbar (dPhi/dx), f, fdot; parameter gradient of Phi = fbar f + fdbar fdot
-// accumulated into the wavefront's slot.
-template <int NL>
-__global__ __launch_bounds__(NT, 1) void k_adj_mlp(Adj a, const double* xin, const double* tin, const double* F1,
-                                                   const double* sf, const double* F2) {
+// added to the workgroup's slot.  TAN = false: without tangents (Phi = fbar f, no tin, F2 and fdot).
+//
+// Every product is a tile of FP64 matrix instructions.  A group of 4 waves takes 32 rows: 16 points and their
+// tangents, or (TAN = false) 32 points; wave w owns the units 16 w .. 16 w + 15 of each layer, so a weight
+// fragment serves both row blocks, and value and tangent of a unit meet in one lane.  The partial sums of dW1
+// and dW2 stay in registers over all tiles of a group; weights, activations and adjoints are in LDS
+// (stride 66: the operand reads of a product along a row touch all banks once).
+// A workgroup holds two groups (two waves a SIMD), and there are at most as many workgroups as CUs, since each adds its
+// parameter partials to memory once per launch.
+// One point per wave with one lane per unit (weights from LDS for every multiply, 0.25 flop a byte) took 255 us for
+// 32 x 513 points of a 17-64-64-1 network; as matrix products 68 us with tangents and 54 without, of which 14
+// and 7 are the matrix instructions at peak: bound by the barriers between the phases and the activations.
+// MFMA operand layout (16x16x4, one wave): lane l supplies A[l%16][l/16] and B[l/16][l%16]; it receives
+// D[4v + l/16][l%16] in element v.
+constexpr int AG = 2;              // groups of a workgroup
+constexpr int ANT = AG * 256;      // its threads
+constexpr int AS = 66;             // LDS row stride (doubles)
+constexpr int AROWS = 32;          // rows of a tile
+constexpr int AW1 = (WMAXW + 3) / 4 * 4;  // rows of W1 in LDS
+constexpr int AKQ = HMAX / 4;      // k steps of a hidden layer
+constexpr int AXL = (AW1 + 7) / 8;  // window entries a thread fetches
+constexpr int ATILE = 3 * AROWS * AS + 4 * AROWS + AROWS;  // LDS of a group (doubles)
+constexpr size_t ADJ_MLP_LDS = (size_t)(AW1 * AS + HMAX * AS + AG * ATILE) * 8;
+static_assert(ADJ_MLP_LDS <= 160 * 1024, "LDS of a CU");
+// (the parameter partials take the place of the tiles at the end)
+static_assert(WMAXW * HMAX + HMAX * HMAX + 3 * HMAX + 1 <= AW1 * AS + AG * ATILE, "parameters fit in LDS");
+template <int NL, bool TAN>
+__global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const double* tin, const double* F1,
+                                                 const double* sf, const double* F2) {
   extern __shared__ double sm[];
-  const int W = a.W, H1 = a.H1, H2 = a.H2, HL = NL == 2 ? H2 : H1;
-  // weights in LDS
-  double* sW1 = sm;                       // W x H1
-  double* sb1 = sW1 + W * H1;             // H1
-  double* sW2 = sb1 + H1;                 // H1 x H2 (NL == 2)
-  double* sb2 = sW2 + (NL == 2 ? H1 * H2 : 0);
-  double* sW3 = sb2 + (NL == 2 ? H2 : 0);  // HL
-  double* sW1t = sW3 + HL;                 // H1 x W (transposed W1)
-  double* sW2t = sW1t + W * H1;            // H2 x H1 (transposed W2, NL == 2)
-  double* wbuf = sW2t + (NL == 2 ? H1 * H2 : 0);  // per wave: 6 x 64
-  for (int t = threadIdx.x; t < W * H1; t += NT) {
-    sW1[t] = a.mlp[a.w1 + t];
-    sW1t[(t % H1) * W + t / H1] = a.mlp[a.w1 + t];
+  constexpr int PTS = TAN ? 16 : 32;  // points of a tile
+  const int tid = threadIdx.x, grp = tid >> 8, t = tid & 255, wv = t >> 6, l = t & 63, lr = l & 15, lk = l >> 4;
+  const int W = a.W, H1 = a.H1, H2 = a.H2, HL = NL == 2 ? H2 : H1, N = a.N, h = W / 2;
+  double* sW1 = sm;                      // W1, row o at o * AS, rows to a multiple of 4 and all columns zero filled
+  double* sW2 = sW1 + AW1 * AS;          // W2 (NL == 2), zero filled
+  double* sX = sW2 + (NL == 2 ? HMAX * AS : 0) + grp * ATILE;  // window and tangent window
+  double* sA = sX + AROWS * AS;          // activations of layer 1, then its adjoints
+  double* sZ = sA + AROWS * AS;          // adjoints of layer 2
+  double* sY = sZ + AROWS * AS;          // output partials of the 4 waves
+  double* sF = sY + 4 * AROWS;           // fbar, fdbar
+  for (int q = tid; q < AW1 * HMAX; q += ANT) {
+    const int o = q / HMAX, u = q % HMAX;
+    sW1[o * AS + u] = o < W && u < H1 ? a.mlp[a.w1 + o * H1 + u] : 0.0;
   }
-  for (int t = threadIdx.x; t < H1; t += NT) sb1[t] = a.mlp[a.b1 + t];
-  if (NL == 2) {
-    for (int t = threadIdx.x; t < H1 * H2; t += NT) {
-      sW2[t] = a.mlp[a.w2 + t];
-      sW2t[(t % H2) * H1 + t / H2] = a.mlp[a.w2 + t];
+  const int col = wv * 16 + lr;
+  if constexpr (NL == 2)
+    for (int q = tid; q < HMAX * HMAX; q += ANT) {
+      const int k = q / HMAX, u = q % HMAX;
+      sW2[k * AS + u] = k < H1 && u < H2 ? a.mlp[a.w2 + k * H2 + u] : 0.0;
     }
-    for (int t = threadIdx.x; t < H2; t += NT) sb2[t] = a.mlp[a.b2 + t];
-  }
-  for (int t = threadIdx.x; t < HL; t += NT) sW3[t] = a.mlp[a.w3 + t];
-  __syncthreads();
-  const double b3 = a.mlp[a.b3];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int slot = blockIdx.x * (NT / 64) + wv;
-  double* sx = wbuf + wv * 6 * 64;  // window
-  double* sxt = sx + 64;            // tangent window
-  double* sa = sxt + 64;            // a1 / zb (reused)
-  double* sat = sa + 64;            // at1 / zdb
-  double* sz = sat + 64;            // zb1
-  const int h = W / 2, N = a.N;
-  const double inorm = 1.0 / a.norm;
-  // parameter partials of this lane (column `lane` of each weight matrix)
-  double gW1[WMAXW], gW2[HMAX];
+  const double b1 = col < H1 ? a.mlp[a.b1 + col] : 0.0, b2 = NL == 2 && col < H2 ? a.mlp[a.b2 + col] : 0.0;
+  const double w3 = col < HL ? a.mlp[a.w3 + col] : 0.0, b3 = a.mlp[a.b3];
+  const d4_t zero = {0.0, 0.0, 0.0, 0.0};
+  constexpr int RB1 = (WMAXW + 15) / 16;
+  d4_t gW1[RB1], gW2[NL == 2 ? 4 : 1];
 #pragma unroll
-  for (int o = 0; o < WMAXW; ++o) gW1[o] = 0.0;
+  for (int rb = 0; rb < RB1; ++rb) gW1[rb] = zero;
 #pragma unroll
-  for (int v = 0; v < HMAX; ++v) gW2[v] = 0.0;
+  for (int rb = 0; rb < (NL == 2 ? 4 : 1); ++rb) gW2[rb] = zero;
   double gb1 = 0.0, gb2 = 0.0, gW3 = 0.0, gb3 = 0.0;
-  const long npts = (long)a.B * N;
-  for (long p = slot; p < npts; p += ADJ_SLOTS) {
-    const int s = (int)(p / N), i = (int)(p % N);
-    const double* xs = xin + (size_t)s * N;
-    if (lane < W) {
-      const int j = i + lane - h;
-      sx[lane] = (j >= 0 && j < N) ? xs[j] * inorm : 0.0;
-      sxt[lane] = (tin && j >= 0 && j < N) ? tin[(size_t)s * N + j] * inorm : 0.0;
-    }
-    __builtin_amdgcn_wave_barrier();
-    const double fbar = sf[s] * F1[(size_t)s * N + i];
-    const double fdbar = F2 ? F2[(size_t)s * N + i] : 0.0;
-    // layer 1 (lane u)
-    double z1 = 0.0, zt1 = 0.0, a1 = 0.0, d11 = 0.0, d21 = 0.0, at1 = 0.0;
-    if (lane < H1) {
-      z1 = sb1[lane];
-      for (int o = 0; o < W; ++o) {
-        z1 = fma(sx[o], sW1[o * H1 + lane], z1);
-        zt1 = fma(sxt[o], sW1[o * H1 + lane], zt1);
-      }
-      act3(a.act, z1, &a1, &d11, &d21);
-      at1 = d11 * zt1;
-    }
-    double aL = a1, atL = at1, d1L = d11, d2L = d21, ztL = zt1;
-    double zt2 = 0.0, a2 = 0.0, d12 = 0.0, d22 = 0.0, at2 = 0.0;
-    if (NL == 2) {
-      if (lane < H1) {
-        sa[lane] = a1;
-        sat[lane] = at1;
-      }
-      __builtin_amdgcn_wave_barrier();
-      if (lane < H2) {
-        double z2 = sb2[lane];
-        for (int v = 0; v < H1; ++v) {
-          z2 = fma(sa[v], sW2[v * H2 + lane], z2);
-          zt2 = fma(sat[v], sW2[v * H2 + lane], zt2);
-        }
-        act3(a.act, z2, &a2, &d12, &d22);
-        at2 = d12 * zt2;
-      }
-      aL = a2;
-      atL = at2;
-      d1L = d12;
-      d2L = d22;
-      ztL = zt2;
-    }
-    const double w3 = lane < HL ? sW3[lane] : 0.0;
-    // raw output y and tangent yd, then the output transform f = g(y), fd = g'(y) yd
-    const double y = wsum(aL * w3) + b3;
-    const double yd = wsum(atL * w3);
-    double g1, g2;
-    const double f = out3(a.mlpout, y, &g1, &g2);
-    const double fd = g1 * yd;
-    // reverse through the transform: ybar = fbar g' + fdbar g'' yd, ydbar = fdbar g'
-    const double ybar = fma(fbar, g1, fdbar * g2 * yd), ydbar = fdbar * g1;
-    // reverse: output layer
-    if (lane < HL) gW3 = fma(ybar, aL, fma(ydbar, atL, gW3));
-    if (lane == 0) gb3 += ybar;
-    const double hb = ybar * w3, hdb = ydbar * w3;
-    double zdb = hdb * d1L;
-    double zb = fma(hb, d1L, hdb * d2L * ztL);
-    if (lane >= HL) {
-      zdb = 0.0;
-      zb = 0.0;
-    }
-    double zb1 = zb, zdb1 = zdb;
-    if (NL == 2) {
-      // W2 column `lane` (unit u = lane of layer 2): += a1_v zb_u + at1_v zdb_u
+  const double inorm = 1.0 / a.norm;
+  const int npts = a.B * N, ntile = (npts + PTS - 1) / PTS;
+  // inputs of a tile: 8 threads a row
+  const int frow = t >> 3, fo = t & 7;
+  double nx[AXL], nf;
+  auto fetch = [&](int tile) {
+    const int p = tile * PTS + (TAN ? frow & 15 : frow);
+    const bool in = tile < ntile && p < npts;
+    const int s = in ? p / N : 0, i = p - s * N;
+    const double* src = (TAN && frow >= 16 ? tin : xin) + (size_t)s * N;
 #pragma unroll
-      for (int v = 0; v < HMAX; ++v)
-        if (v < H1) gW2[v] = fma(sa[v], zb, fma(sat[v], zdb, gW2[v]));
-      gb2 += zb;
-      __builtin_amdgcn_wave_barrier();
-      sa[lane] = zb;  // a1 / at1 no longer needed
-      sat[lane] = zdb;
-      __builtin_amdgcn_wave_barrier();
-      double hb1 = 0.0, hdb1 = 0.0;
-      if (lane < H1) {
-        for (int u = 0; u < H2; ++u) {
-          hb1 = fma(sa[u], sW2t[u * H1 + lane], hb1);
-          hdb1 = fma(sat[u], sW2t[u * H1 + lane], hdb1);
+    for (int q = 0; q < AXL; ++q) {
+      const int o = fo + 8 * q, x = i + o - h;
+      nx[q] = in && o < W && x >= 0 && x < N ? src[x] * inorm : 0.0;
+    }
+    nf = 0.0;
+    if (in && fo == 0) nf = TAN && frow >= 16 ? F2[p] : sf[s] * F1[p];
+  };
+  const int G = gridDim.x;
+  fetch(blockIdx.x + G * grp);
+  // (both groups run the rounds of the first one)
+  for (int round = 0; blockIdx.x + G * AG * round < ntile; ++round) {
+    const int tile = blockIdx.x + G * (AG * round + grp);
+#pragma unroll
+    for (int q = 0; q < AXL; ++q)
+      if (fo + 8 * q < AW1) sX[frow * AS + fo + 8 * q] = nx[q];
+    if (fo == 0) sF[frow] = nf;
+    __syncthreads();
+    fetch(tile + G * AG);
+    // ---- layer 1 ----
+    d4_t z0 = zero, z1 = zero;
+#pragma unroll
+    for (int q = 0; q < AW1 / 4; ++q)
+      if (4 * q < W) {
+        const int k = 4 * q + lk;
+        const double b = sW1[k * AS + col];
+        z0 = mfma64(sX[lr * AS + k], b, z0);
+        z1 = mfma64(sX[(16 + lr) * AS + k], b, z1);
+      }
+    // TAN: z0 the pre-activations and z1 their tangents; else both pre-activations
+    double aL[2][4], p1[2][4], q1[4], t1[4];  // activations, act' (block 1: unused with TAN), act'', tangents
+    auto activate = [&](double bias, d4_t y0, d4_t y1, double (&av)[2][4], double (&d1)[2][4], double (&d2)[4], double (&zt)[4]) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double e2;
+        act3(a.act, y0[v] + bias, &av[0][v], &d1[0][v], &e2);
+        if (TAN) {
+          d2[v] = e2;
+          zt[v] = y1[v];
+          av[1][v] = d1[0][v] * y1[v];
+        } else {
+          act3(a.act, y1[v] + bias, &av[1][v], &d1[1][v], &e2);
         }
       }
-      zdb1 = hdb1 * d11;
-      zb1 = fma(hb1, d11, hdb1 * d21 * zt1);
-      if (lane >= H1) {
-        zdb1 = 0.0;
-        zb1 = 0.0;
+    };
+    activate(b1, z0, z1, aL, p1, q1, t1);
+    double p2[2][4], q2[4], t2[4];
+    if constexpr (NL == 2) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        sA[(4 * v + lk) * AS + col] = col < H1 ? aL[0][v] : 0.0;
+        sA[(16 + 4 * v + lk) * AS + col] = col < H1 ? aL[1][v] : 0.0;
+      }
+      __syncthreads();
+      z0 = z1 = zero;
+#pragma unroll
+      for (int q = 0; q < AKQ; ++q)
+        if (4 * q < H1) {
+          const double b = sW2[(4 * q + lk) * AS + col];
+          z0 = mfma64(sA[lr * AS + 4 * q + lk], b, z0);
+          z1 = mfma64(sA[(16 + lr) * AS + 4 * q + lk], b, z1);
+        }
+      activate(b2, z0, z1, aL, p2, q2, t2);
+    }
+    // ---- output: the units of a wave in one DPP row, the waves through LDS ----
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double y = row_sum(aL[rb][v] * w3);
+        if (lr == 0) sY[wv * AROWS + rb * 16 + 4 * v + lk] = y;
+      }
+    __syncthreads();
+    // adjoints of the last hidden layer: zb[0] of the values, zb[1] of the tangents (else of the points 16 .. 31)
+    double zb[2][4];
+    const double(&pl)[2][4] = NL == 2 ? p2 : p1;
+    const double(&ql)[4] = NL == 2 ? q2 : q1;
+    const double(&tl)[4] = NL == 2 ? t2 : t1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = 4 * v + lk;
+      auto raw = [&](int row) { return (sY[row] + sY[AROWS + row]) + (sY[2 * AROWS + row] + sY[3 * AROWS + row]); };
+      double g1, g2;
+      if (TAN) {
+        const int p = tile * PTS + r;
+        const double fbar = sF[r], fdbar = sF[16 + r], yd = raw(16 + r);
+        const double f = out3(a.mlpout, raw(r) + b3, &g1, &g2);
+        // reverse through the transform: ybar = fbar g' + fdbar g'' yd, ydbar = fdbar g'
+        const double ybar = fma(fbar, g1, fdbar * g2 * yd), ydbar = fdbar * g1;
+        if (wv == 0 && lr == 0) {
+          if (tile < ntile && p < npts) {
+            a.fv[p] = f;
+            a.fdv[p] = g1 * yd;
+          }
+          gb3 += ybar;
+        }
+        gW3 = fma(ybar, aL[0][v], fma(ydbar, aL[1][v], gW3));
+        const double hb = ybar * w3, hdb = ydbar * w3;
+        zb[0][v] = fma(hb, pl[0][v], hdb * ql[v] * tl[v]);
+        zb[1][v] = hdb * pl[0][v];
+      } else {
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          const int row = rb * 16 + r, p = tile * PTS + row;
+          const double f = out3(a.mlpout, raw(row) + b3, &g1, &g2);
+          const double ybar = sF[row] * g1;
+          if (wv == 0 && lr == 0) {
+            if (tile < ntile && p < npts) a.fv[p] = f;
+            gb3 += ybar;
+          }
+          gW3 = fma(ybar, aL[rb][v], gW3);
+          zb[rb][v] = ybar * w3 * pl[rb][v];
+        }
       }
     }
-    // W1 column `lane`: += x_o zb1 + xt_o zdb1
+    if constexpr (NL == 2) {
 #pragma unroll
-    for (int o = 0; o < WMAXW; ++o)
-      if (o < W) gW1[o] = fma(sx[o], zb1, fma(sxt[o], zdb1, gW1[o]));
-    gb1 += zb1;
-    sz[lane] = zb1;
-    __builtin_amdgcn_wave_barrier();
-    if (lane < W) {
-      double xb = 0.0;
-      for (int u = 0; u < H1; ++u) xb = fma(sz[u], sW1t[u * W + lane], xb);
-      a.xbar[(size_t)p * W + lane] = xb;
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sZ[(rb * 16 + 4 * v + lk) * AS + col] = zb[rb][v];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) gb2 += TAN ? zb[0][v] : zb[0][v] + zb[1][v];
+      __syncthreads();
+      // dW2 += a1^T zb (rows of values and tangents in one sum); adjoints of a1 = zb W2^T
+#pragma unroll
+      for (int q = 0; q < AROWS / 4; ++q) {
+        const double b = sZ[(4 * q + lk) * AS + col];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+          if (16 * rb < H1) gW2[rb] = mfma64(sA[(4 * q + lk) * AS + rb * 16 + lr], b, gW2[rb]);
+      }
+      z0 = z1 = zero;
+#pragma unroll
+      for (int q = 0; q < AKQ; ++q)
+        if (4 * q < H2) {
+          const double b = sW2[col * AS + 4 * q + lk];
+          z0 = mfma64(sZ[lr * AS + 4 * q + lk], b, z0);
+          z1 = mfma64(sZ[(16 + lr) * AS + 4 * q + lk], b, z1);
+        }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (TAN) {
+          zb[0][v] = fma(z0[v], p1[0][v], z1[v] * q1[v] * t1[v]);
+          zb[1][v] = z1[v] * p1[0][v];
+        } else {
+          zb[0][v] = z0[v] * p1[0][v];
+          zb[1][v] = z1[v] * p1[1][v];
+        }
+      }
+      __syncthreads();  // every wave has read the activations
     }
-    if (lane == 0) {
-      a.fv[p] = f;
-      a.fdv[p] = fd;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sA[(rb * 16 + 4 * v + lk) * AS + col] = col < H1 ? zb[rb][v] : 0.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) gb1 += TAN ? zb[0][v] : zb[0][v] + zb[1][v];
+    __syncthreads();
+    // dW1 += x^T zb; window cotangents = zb W1^T
+#pragma unroll
+    for (int q = 0; q < AROWS / 4; ++q) {
+      const double b = sA[(4 * q + lk) * AS + col];
+#pragma unroll
+      for (int rb = 0; rb < RB1; ++rb)
+        if (16 * rb < W) gW1[rb] = mfma64(sX[(4 * q + lk) * AS + rb * 16 + lr], b, gW1[rb]);
     }
-    __builtin_amdgcn_wave_barrier();
+    if (wv * 16 < W) {
+      z0 = z1 = zero;
+#pragma unroll
+      for (int q = 0; q < AKQ; ++q)
+        if (4 * q < H1) {
+          const double b = col < W ? sW1[col * AS + 4 * q + lk] : 0.0;
+          z0 = mfma64(sA[lr * AS + 4 * q + lk], b, z0);
+          if (!TAN) z1 = mfma64(sA[(16 + lr) * AS + 4 * q + lk], b, z1);
+        }
+#pragma unroll
+      for (int rb = 0; rb < (TAN ? 1 : 2); ++rb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int p = tile * PTS + rb * 16 + 4 * v + lk;
+          if (col < W && tile < ntile && p < npts) a.xbar[(size_t)p * W + col] = rb ? z1[v] : z0[v];
+        }
+    }
+    __syncthreads();
   }
-  // the workgroup's waves add their partials into LDS one after another (the weights are no longer
-  // needed, and their area holds the P parameters), then the sum goes to the workgroup's slot (slots
-  // are owned: no races; a fixed order)
-  __syncthreads();
+  // the groups add their partials into LDS one after another, then the sum goes to the
+  // workgroup's slot (slots are owned: no races; a fixed order)
+  auto over_rows = [&](double x) {
+    x += __shfl_xor(x, 16, 64);
+    return x + __shfl_xor(x, 32, 64);
+  };
+  gb1 = over_rows(gb1);
+  gb2 = over_rows(gb2);
+  gW3 = over_rows(gW3);
+  gb3 = over_rows(gb3);
   double* r = sm;
-  for (int t = threadIdx.x; t < a.P; t += NT) r[t] = 0.0;
-  __syncthreads();
-  for (int w = 0; w < NT / 64; ++w) {
-    if (wv == w) {
-      if (lane < H1) {
+  for (int g = 0; g < AG; ++g) {
+    if (grp == g) {
+      auto put = [&](int at, double x) { r[at] = g == 0 ? x : r[at] + x; };
 #pragma unroll
-        for (int o = 0; o < WMAXW; ++o)
-          if (o < W) r[a.w1 + o * H1 + lane] += gW1[o];
-        r[a.b1 + lane] += gb1;
-      }
-      if (NL == 2 && lane < H2) {
+      for (int rb = 0; rb < RB1; ++rb)
 #pragma unroll
-        for (int v = 0; v < HMAX; ++v)
-          if (v < H1) r[a.w2 + v * H2 + lane] += gW2[v];
-        r[a.b2 + lane] += gb2;
+        for (int v = 0; v < 4; ++v) {
+          const int o = rb * 16 + 4 * v + lk;
+          if (o < W && col < H1) put(a.w1 + o * H1 + col, gW1[rb][v]);
+        }
+      if constexpr (NL == 2) {
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int k = rb * 16 + 4 * v + lk;
+            if (k < H1 && col < H2) put(a.w2 + k * H2 + col, gW2[rb][v]);
+          }
+        if (lk == 0 && col < H2) put(a.b2 + col, gb2);
       }
-      if (lane < HL) r[a.w3 + lane] += gW3;
-      if (lane == 0) r[a.b3] += gb3;
+      if (lk == 0 && col < H1) put(a.b1 + col, gb1);
+      if (lk == 0 && col < HL) put(a.w3 + col, gW3);
+      if (t == 0) put(a.b3, gb3);
     }
     __syncthreads();
   }
   double* g = a.thp + (size_t)blockIdx.x * a.P;
-  for (int t = threadIdx.x; t < a.P; t += NT) g[t] += r[t];
+  for (int q = tid; q < a.P; q += ANT) g[q] += r[q];
 }
 
 // Global-network second-order adjoint (GLOBAL_MLP: f(n) = g(MLP(n / norm)), one scalar per
@@ -1001,25 +1130,28 @@ int qex1d_kohn_sham_vjp(const qex1d_problem* p, const qex1d_inputs* in, const qe
   const double s2 = -0.5 / (a.dx * a.dx);
   const double Td = s2 * -2.5, Tb = s2 * (4.0 / 3.0), Tc = s2 * (-1.0 / 12.0);
   const int HL = a.NL == 2 ? a.H2 : a.H1;
-  const size_t mlp_lds = (2 * (size_t)a.W * a.H1 + a.H1 + (a.NL == 2 ? 2 * (size_t)a.H1 * a.H2 + a.H2 : 0) + HL +
-                          (size_t)(NT / 64) * 6 * 64) * 8;
   const size_t eig_lds = adj_eig_lds(a.N);
   const bool glob = p->xc_kind == QEX1D_XC_GLOBAL_MLP;
   const size_t gmlp_lds = (2 * (size_t)a.N + 2 * (NT / 64) * 64 + 12 * 64 + 8) * 8;
-  if ((!glob && mlp_lds > 150 * 1024) || eig_lds > 150 * 1024)
-    return faila(QEX_E_UNSUPPORTED, "problem too large for LDS");
   if (eig_lds > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)k_adj_eig, hipFuncAttributeMaxDynamicSharedMemorySize, (int)eig_lds);
-  if (!glob && mlp_lds > 64 * 1024) {
-    (void)hipFuncSetAttribute((const void*)k_adj_mlp<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlp_lds);
-    (void)hipFuncSetAttribute((const void*)k_adj_mlp<2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlp_lds);
+  if (!glob) {
+    const void* fns[4] = {(const void*)k_adj_mlp<1, false>, (const void*)k_adj_mlp<1, true>,
+                          (const void*)k_adj_mlp<2, false>, (const void*)k_adj_mlp<2, true>};
+    for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ADJ_MLP_LDS);
   }
   auto mlp = [&](const double* xin, const double* tin, const double* F1, const double* sf, const double* F2) {
     qexprof::Scope ps(qexprof::K_ADJ_MLP, st);
-    if (a.NL == 2)
-      hipLaunchKernelGGL(k_adj_mlp<2>, dim3(ADJ_WG), dim3(NT), mlp_lds, st, a, xin, tin, F1, sf, F2);
+    const long tiles = ((long)a.B * a.N + (tin ? 15 : 31)) / (tin ? 16 : 32);
+    const dim3 grid((unsigned)(tiles < ADJ_WG ? tiles : ADJ_WG)), block(ANT);
+    if (a.NL == 2 && tin)
+      hipLaunchKernelGGL((k_adj_mlp<2, true>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
+    else if (a.NL == 2)
+      hipLaunchKernelGGL((k_adj_mlp<2, false>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
+    else if (tin)
+      hipLaunchKernelGGL((k_adj_mlp<1, true>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
     else
-      hipLaunchKernelGGL(k_adj_mlp<1>, dim3(ADJ_WG), dim3(NT), mlp_lds, st, a, xin, tin, F1, sf, F2);
+      hipLaunchKernelGGL((k_adj_mlp<1, false>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
   };
   // the global network: one workgroup per system (at most ADJ_WG, each then taking several in turn)
   const unsigned gG = (unsigned)(a.B < ADJ_WG ? a.B : ADJ_WG);

@@ -96,6 +96,37 @@ def test_gradient_over_grid_sizes_matches_oracle(mods, N, ne):
     np.testing.assert_allclose(g.cpu().numpy(), go, rtol=0, atol=1e-6 * np.abs(go).max())
 
 
+@pytest.mark.parametrize("N,act,sizes,out", [(65, "silu", [33, 64, 64, 1], "linear"), (66, "tanh", [1, 1, 1], "linear"),
+                                             (63, "gelu", [17, 15, 17, 1], "negativity"), (80, "softplus", [3, 64, 1], "negativity"),
+                                             (97, "sigmoid", [15, 33, 63, 1], "linear"), (64, "silu", [17, 48, 5, 1], "linear")])
+def test_gradient_over_network_sizes_matches_oracle(mods, N, act, sizes, out):
+    """Windows, widths and point counts at the edges of the network adjoint's tiles (16 units, 4 k steps, 16
+    and 32 points), both output transforms: 1e-6 of the largest entry, as for the other gradients."""
+    engine, train, utils, xcm = mods
+    grids = np.linspace(-6.4, 6.4, N)
+    dx = float(grids[1] - grids[0])
+    systems = _systems()
+    params = _params(9, sizes)
+    f = xcm.LocalMLPXC(params, window=sizes[0], activation=act, norm=2.0, output=out)
+    n0 = np.stack([O.gaussian_initial_density(grids, l, z, ne, weighted=True) for l, z, ne in systems])
+    prob = engine.Problem1D(grids, [s[0] for s in systems], [s[1] for s in systems], [s[2] for s in systems],
+                            utils.exponential_coulomb, f, 2, alpha=0.4, alpha_decay=0.9, num_mixing_iterations=1,
+                            loop="scan", want_orbitals=True)
+    tn = 0.9 * n0
+    tE = np.array([-1.2, -2.5, -4.0])
+    loss, g, res = train.value_and_grad(prob, n0, train.c3_loss, tE, tn, dx)
+    xc = O.LocalMLP([w for w, _ in params], [b for _, b in params], act, sizes[0], 2.0, out)
+    go = 0.0
+    for s, (loc, z, ne) in enumerate(systems):
+        fw = A.forward_trajectory(loc, z, ne, 2, grids, xc, O.exponential_coulomb, n0[s], 0.4, 0.9, 1)
+        dE = np.zeros(2)
+        dn = np.zeros((2, N))
+        dE[-1] = 2 * (fw["energies"][-1] - tE[s]) / 3
+        dn[-1] = 2 * 1e-2 * dx * (fw["densities"][-1] - tn[s]) / 3
+        go = go + A.backward(fw, dE, dn)
+    np.testing.assert_allclose(g.cpu().numpy(), go, rtol=0, atol=1e-6 * np.abs(go).max())
+
+
 def test_device_gradient_matches_finite_differences(mods):
     engine, train, _, _ = mods
     grids = np.linspace(-12.8, 12.8, 257)
