@@ -82,6 +82,25 @@ def test_xc_evaluate_matches_oracle(name):
         _close(vxc[b], O.xc_potential(ref, n[b], DX))
 
 
+@pytest.mark.parametrize("sizes", [[1, 1, 1], [33, 64, 1], [17, 64, 64, 1], [9, 15, 17, 1], [33, 64, 64, 64, 1],
+                                   [3, 5, 63, 33, 1], [33, 64, 64, 64, 64, 1], [7, 16, 8, 49, 12, 1]])
+@pytest.mark.parametrize("npts", [5, 16, 131])
+def test_matrix_core_network_sizes(sizes, npts):
+    """One to four hidden layers, windows, widths and point counts at the edges of the 16-point tiles and of
+    the 8-row k steps, more systems than waves: the bar of this file."""
+    rng = np.random.default_rng(sum(sizes) + npts)
+    W = [rng.standard_normal((a, b)) / np.sqrt(a) for a, b in zip(sizes[:-1], sizes[1:])]
+    b = [0.1 * rng.standard_normal(k) for k in sizes[1:]]
+    n = rng.uniform(0.0, 1.0, (40, npts))
+    eps, exc, vxc = (t.cpu().numpy() for t in engine.xc_evaluate(
+        xc.LocalMLPXC(list(zip(W, b)), window=sizes[0], activation="silu", norm=2.0), n, DX))
+    ref = O.LocalMLP(W, b, "silu", sizes[0], 2.0)
+    for k in range(len(n)):
+        _close(eps[k], O.xc_energy_density_out(ref, n[k]))
+        _close(exc[k], O.xc_energy(ref, n[k], DX))
+        _close(vxc[k], O.xc_potential(ref, n[k], DX))
+
+
 @pytest.mark.parametrize("name", ["lda", "mlp_mfma", "mlp_lpp8", "power_global", "global_mlp"])
 def test_xc_potential_is_derivative_of_device_energy(name):
     f, _ = _cases()[name]
