@@ -786,10 +786,12 @@ __device__ double mlp_v_unsym(const Dev1& a, int s, int i) {
   return v + acc / a.norm;
 }
 
-// Global MLP on the whole density, one workgroup per system: f(n_in) with the input gradient
+// Global MLP on the whole density, two workgroups per system: f(n_in) with the input gradient
 // (potential dx df/dn into mlp_e) and f at the pending output density; scalars in
 // mlp_eout[2 s] (f(n_in)) and mlp_eout[2 s + 1] (f(n_out)).  Layer activations and derivatives
 // in LDS, hmax doubles per layer (HB).
+// Bound by the latency of the weights' loads (133 KB a system at N = 257, from L2): 16 in flight a thread, in the order
+// of the sums, and the two evaluations side by side: 52 -> 15 us a launch for 5 systems (257-64-64-1).
 __device__ double gmlp_forward(const Dev1& a, const double* x, double* acts, double* dzs, double* part, double* red) {
   const int N = a.N, tid = threadIdx.x, HB = a.hmax;
   const int H1 = a.widths[1];
@@ -798,6 +800,7 @@ __device__ double gmlp_forward(const Dev1& a, const double* x, double* acts, dou
     const int G = NT / H1, u = tid % H1, g = tid / H1;
     double acc = 0.0;
     if (g < G)
+#pragma unroll 16
       for (int i = g; i < N; i += G) acc = fma(x[i], a.mlp[a.woff[0] + (size_t)i * H1 + u], acc);
     part[tid] = acc;
     __syncthreads();
@@ -812,6 +815,7 @@ __device__ double gmlp_forward(const Dev1& a, const double* x, double* acts, dou
     // wide first layer: every thread takes units tid, tid + NT, ... over the whole input
     for (int u = tid; u < H1; u += NT) {
       double z = a.mlp[a.boff[0] + u];
+#pragma unroll 16
       for (int i = 0; i < N; ++i) z = fma(x[i], a.mlp[a.woff[0] + (size_t)i * H1 + u], z);
       double dz;
       acts[u] = act_fwd(a.act, z, &dz);
@@ -825,6 +829,7 @@ __device__ double gmlp_forward(const Dev1& a, const double* x, double* acts, dou
     const double* prev = acts + (l - 1) * HB;
     for (int u = tid; u < fo; u += NT) {
       double z = a.mlp[a.boff[l] + u];
+#pragma unroll 16
       for (int v = 0; v < fi; ++v) z = fma(prev[v], a.mlp[a.woff[l] + v * fo + u], z);
       double dz;
       acts[l * HB + u] = act_fwd(a.act, z, &dz);
@@ -845,8 +850,9 @@ __global__ __launch_bounds__(NT) void k_gmlp(Dev1 a, int k_launch) {
   __shared__ double red[NWAVE * 8];
   const int s = blockIdx.x, N = a.N, tid = threadIdx.x, HB = a.hmax;
   const int k = iter_of(a, s, k_launch);
-  const bool doPot = k >= 0 && k < a.T && a.st[4 * s + 0] == 0;
-  const bool doE = a.st[4 * s + 1] >= 0 && a.st[4 * s + 1] < a.T;
+  // the potential and the deferred energy have a workgroup each
+  const bool doPot = blockIdx.y == 0 && k >= 0 && k < a.T && a.st[4 * s + 0] == 0;
+  const bool doE = blockIdx.y == 1 && a.st[4 * s + 1] >= 0 && a.st[4 * s + 1] < a.T;
   double* x = smem;                       // N
   double* acts = x + N;                   // (nlay - 1) x HB
   double* dzs = acts + (a.nlay - 1) * HB;  // (nlay - 1) x HB
@@ -867,9 +873,11 @@ __global__ __launch_bounds__(NT) void k_gmlp(Dev1 a, int k_launch) {
     __syncthreads();
     for (int l = L - 1; l >= 1; --l) {
       const int fi = a.widths[l], fo = a.widths[l + 1];
+      const double* Wl = a.mlp + a.woff[l];
       for (int v = tid; v < fi; v += NT) {
         double g = 0.0;
-        for (int u = 0; u < fo; ++u) g = fma(a.mlp[a.woff[l] + v * fo + u], cur[u], g);
+#pragma unroll 16
+        for (int u = 0; u < fo; ++u) g = fma(Wl[v * fo + u], cur[u], g);
         nxt[v] = g * dzs[(l - 1) * HB + v];
       }
       __syncthreads();
@@ -880,8 +888,10 @@ __global__ __launch_bounds__(NT) void k_gmlp(Dev1 a, int k_launch) {
     // v_i = dx df/dn_i = dx / norm sum_u W1[i][u] delta_u
     const int H1 = a.widths[1];
     for (int i = tid; i < N; i += NT) {
+      const double* W0 = a.mlp + a.woff[0] + (size_t)i * H1;
       double g = 0.0;
-      for (int u = 0; u < H1; ++u) g = fma(a.mlp[a.woff[0] + (size_t)i * H1 + u], cur[u], g);
+#pragma unroll 16
+      for (int u = 0; u < H1; ++u) g = fma(W0[u], cur[u], g);
       a.mlp_e[(size_t)s * N + i] = a.dx * in * g;
     }
     if (tid == 0) a.mlp_eout[2 * s] = f;
@@ -2401,7 +2411,7 @@ void launch_network(const Plan1d& P, int k, hipStream_t stream) {
   }
   if (a.xc == QEX1D_XC_GLOBAL_MLP) {
     Scope ps(qexprof::K_MLP, stream);
-    hipLaunchKernelGGL(k_gmlp, dim3(a.B), dim3(NT), P.lds_gmlp, stream, a, k);
+    hipLaunchKernelGGL(k_gmlp, dim3(a.B, 2), dim3(NT), P.lds_gmlp, stream, a, k);
   }
 }
 

@@ -581,6 +581,8 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
 // blockIdx.x + gridDim.x, ... in order, so each slot is written by one workgroup in a fixed order.
 // Hidden widths <= 64: unit u of a layer is lane u of a wave; the input layer's sums over the N
 // grid points are split over the 4 waves and combined in a fixed order.
+// Bound by the latency of the weights' loads and of the partials' updates: 16 in flight a thread, 44 -> 26 us a launch
+// for 5 systems (257-64-64-1).
 template <int NL>
 __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const double* tin, const double* sf,
                                                  double fd, const double* A2, double* dst) {
@@ -609,6 +611,7 @@ __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const
     {
       double acc = 0.0, accd = 0.0;
       if (u < H1)
+#pragma unroll 16
         for (int i = q; i < N; i += NW) {
           const double w = W1[(size_t)i * H1 + u];
           acc = fma(x[i], w, acc);
@@ -635,6 +638,7 @@ __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const
     __syncthreads();
     if (NL == 2 && t < H2) {
       double z = a.mlp[a.b2 + t], zd = 0.0;
+#pragma unroll 16
       for (int v = 0; v < H1; ++v) {
         const double w = W2[v * H2 + t];
         z = fma(h1[v], w, z);
@@ -652,6 +656,7 @@ __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const
     const double* hl = NL == 2 ? h2 : h1;
     if (t == 0) {
       double y = a.mlp[a.b3], yd = 0.0;
+#pragma unroll 16
       for (int v = 0; v < HL; ++v) {
         y = fma(hl[v], W3[v], y);
         yd = fma(hl[64 + v], W3[v], yd);
@@ -678,12 +683,21 @@ __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const
     if (NL == 2) {
       // W2 (H1 x H2): lane u = row, waves over the columns
       if (u < H1)
-        for (int v = q; v < H2; v += NW)
-          g[a.w2 + u * H2 + v] += h1[u] * h2[320 + v] + h1[64 + u] * h2[256 + v];
+      {
+        double w[HMAX / NW];
+#pragma unroll
+        for (int e = 0; e < HMAX / NW; ++e) w[e] = q + e * NW < H2 ? g[a.w2 + u * H2 + q + e * NW] : 0.0;
+#pragma unroll
+        for (int e = 0; e < HMAX / NW; ++e) {
+          const int v = q + e * NW;
+          if (v < H2) g[a.w2 + u * H2 + v] = w[e] + (h1[u] * h2[320 + v] + h1[64 + u] * h2[256 + v]);
+        }
+      }
       if (t < H2) g[a.b2 + t] += h2[320 + t];
       __syncthreads();
       if (t < H1) {
         double hb = 0.0, hdb = 0.0;
+#pragma unroll 16
         for (int v = 0; v < H2; ++v) {
           const double w = W2[t * H2 + v];
           hb = fma(w, h2[320 + v], hb);
@@ -697,10 +711,20 @@ __global__ __launch_bounds__(NT) void k_adj_gmlp(Adj a, const double* xin, const
     }
     // layer 1: W1 (N x H1), b1, and the input cotangent
     if (u < H1)
-      for (int i = q; i < N; i += NW) g[a.w1 + (size_t)i * H1 + u] += x[i] * h1[320 + u] + xd[i] * h1[256 + u];
+      for (int i0 = q; i0 < N; i0 += 16 * NW) {  // (16 loads in flight)
+        double w[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) w[e] = i0 + e * NW < N ? g[a.w1 + (size_t)(i0 + e * NW) * H1 + u] : 0.0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int i = i0 + e * NW;
+          if (i < N) g[a.w1 + (size_t)i * H1 + u] = w[e] + (x[i] * h1[320 + u] + xd[i] * h1[256 + u]);
+        }
+      }
     if (t < H1) g[a.b1 + t] += h1[320 + t];
     for (int i = t; i < N; i += NT) {
       double xb = 0.0;
+#pragma unroll 16
       for (int v = 0; v < H1; ++v) xb = fma(W1[(size_t)i * H1 + v], h1[320 + v], xb);
       double r = xb * in;
       if (A2) r += A2[(size_t)s * N + i];
