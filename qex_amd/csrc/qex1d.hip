@@ -493,8 +493,8 @@ __global__ __launch_bounds__(NT) void k_mlp(Dev1 a, int k_launch) {
 // weights (LDS, copied once) and nothing else: no barriers, and one wave's activations run beside another's
 // matrix instructions.  The potential's tiles and the deferred energy's are separate items.
 // A workgroup of 4 waves per 48-point tile, with barriers between the layers and the weights read from L2 in the
-// k loops, took 366 us for 601 x 513 points of a 17-64-64-1 network (61 for 64 x 513, 50 for 32 x 513); now
-// 323, 60 and 40.  The matrix instructions alone are 132 us of the 323 and the activations' FP64 about as much:
+// k loops, took 366 us for 601 x 401 points of a 17-64-64-1 network (61 for 64 x 513, 50 for 32 x 513); now
+// 323, 60 and 40.  The matrix instructions alone are 104 us of the 323 and the activations' FP64 about as much:
 // the two share the FP64 units, so they add up.
 // MFMA operand layout (16x16x4, one wave): lane l supplies A[l%16][l/16] and B[l/16][l%16];
 // it receives D[4v + l/16][l%16] in element v.
@@ -508,7 +508,7 @@ constexpr int MLP_CB = MLP_HMAX / 16;  // column blocks
 constexpr int MLP_K = 8;       // k of a loop iteration
 constexpr int MLP_TILE = MLP_P * MLP_S + MLP_P;  // LDS of a wave (doubles)
 // waves of a workgroup: one workgroup a CU, as many waves as the weights leave LDS for, at most 2 a SIMD (at 3 the
-// activations spill: 345 us instead of 333 for 601 x 513 points)
+// activations spill: 345 us instead of 333 for 601 x 401 points)
 constexpr int mlp_waves(int hidden) { return hidden <= 3 ? 8 : 4; }
 
 __device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
@@ -1362,9 +1362,9 @@ __device__ __forceinline__ void twisted_inverse_iteration(const double* ap, doub
 // The bracket, its middle and the solves are those of counting every round, so the orbitals are the same to the
 // bit; solving in parallel there too is as fast and as accurate, but moves the orbitals of nearly degenerate
 // pairs by their own rounding, 1e-13 over the gap.
-// Bound by the dependent chain of one pair: 55..75 us, of which the two solves 30.  A launch at N = 513: 3 systems
-// 69 us (91 with every round counted and the four phases of the solves in sequence), 64 systems x 5 pairs
-// 99 us (120), 601 systems 309 us (364).
+// Bound by the dependent chain of one pair: 55..75 us, of which the two solves 30.  A launch at N = 513: one system
+// 69 us (91 with every round counted and the four phases of the solves in sequence), 64 systems of up to 5 pairs
+// 99 us (120); 601 systems at N = 401 309 us (364).
 // ISOLATED: a round over 2 Ha leaves intervals of 2 / 127, the first bracket that a second one would not pay for.
 // APART: the first solve then shrinks the neighbours' parts by 1 / 9 or more; at 1 one pair in ten took 6 solves or
 // ended at a neighbour, and the launch waits for the slowest (batch of 64: 144 us).

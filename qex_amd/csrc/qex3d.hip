@@ -1672,7 +1672,7 @@ __global__ __launch_bounds__(NT) void k_coulomb(int n, int npair, const double* 
 // step and receives C[4v + l/16][l%16] in element v).  Operands in LDS or global memory (glob / lds
 // below), row-major or, with T, transposed.  The matrices are at most 96 wide and come from L2, so the
 // time is load latency: GEMM_U steps' operands are in flight together, read from clamped addresses
-// and zeroed past K instead of behind branches (n = 80, one workgroup: see k_scf_fock).
+// and zeroed past K instead of behind branches (n = 80, one workgroup: see k_scf_step).
 typedef const __attribute__((address_space(1))) double* gptr_t;
 typedef const __attribute__((address_space(3))) double* lptr_t;
 template <class P>
