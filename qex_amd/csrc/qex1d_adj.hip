@@ -25,6 +25,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "band_wave.h"
 #include "prof.h"
 #include "qex.h"
@@ -288,7 +290,7 @@ __device__ __forceinline__ double row_sum(double x) {
 // A workgroup holds two groups (two waves a SIMD), and there are at most as many workgroups as CUs, since each adds its
 // parameter partials to memory once per launch.
 // One point per wave with one lane per unit (weights from LDS for every multiply, 0.25 flop a byte) took 255 us for
-// 32 x 513 points of a 17-64-64-1 network; as matrix products 68 us with tangents and 54 without, of which 14
+// 32 x 513 points of a 17-64-64-1 network; as matrix products 64 us with tangents and 52 without, of which 14
 // and 7 are the matrix instructions at peak: bound by the barriers between the phases and the activations.
 // MFMA operand layout (16x16x4, one wave): lane l supplies A[l%16][l/16] and B[l/16][l%16]; it receives
 // D[4v + l/16][l%16] in element v.
@@ -318,16 +320,24 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
   double* sZ = sA + AROWS * AS;          // adjoints of layer 2
   double* sY = sZ + AROWS * AS;          // output partials of the 4 waves
   double* sF = sY + 4 * AROWS;           // fbar, fdbar
-  for (int q = tid; q < AW1 * HMAX; q += ANT) {
-    const int o = q / HMAX, u = q % HMAX;
-    sW1[o * AS + u] = o < W && u < H1 ? a.mlp[a.w1 + o * H1 + u] : 0.0;
-  }
-  const int col = wv * 16 + lr;
-  if constexpr (NL == 2)
-    for (int q = tid; q < HMAX * HMAX; q += ANT) {
-      const int k = q / HMAX, u = q % HMAX;
-      sW2[k * AS + u] = k < H1 && u < H2 ? a.mlp[a.w2 + k * H2 + u] : 0.0;
+  // weights into LDS, a thread's loads in flight together
+  auto copy = [&](double* dst, int w, int rows, int cols, auto padded) {
+    constexpr int total = decltype(padded)::value, M = (total * HMAX + ANT - 1) / ANT;
+    double v[M];
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      const int q = tid + e * ANT, r = q / HMAX, u = q % HMAX;
+      v[e] = r < rows && u < cols ? a.mlp[w + r * cols + u] : 0.0;
     }
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      const int q = tid + e * ANT;
+      if (q < total * HMAX) dst[q / HMAX * AS + q % HMAX] = v[e];
+    }
+  };
+  copy(sW1, a.w1, W, H1, std::integral_constant<int, AW1>{});
+  const int col = wv * 16 + lr;
+  if constexpr (NL == 2) copy(sW2, a.w2, H1, H2, std::integral_constant<int, HMAX>{});
   const double b1 = col < H1 ? a.mlp[a.b1 + col] : 0.0, b2 = NL == 2 && col < H2 ? a.mlp[a.b2 + col] : 0.0;
   const double w3 = col < HL ? a.mlp[a.w3 + col] : 0.0, b3 = a.mlp[a.b3];
   const d4_t zero = {0.0, 0.0, 0.0, 0.0};
@@ -369,9 +379,8 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
     fetch(tile + G * AG);
     // ---- layer 1 ----
     d4_t z0 = zero, z1 = zero;
-#pragma unroll
-    for (int q = 0; q < AW1 / 4; ++q)
-      if (4 * q < W) {
+#pragma unroll 1
+    for (int q = 0; 4 * q < W; ++q) {
         const int k = 4 * q + lk;
         const double b = sW1[k * AS + col];
         z0 = mfma64(sX[lr * AS + k], b, z0);
@@ -403,9 +412,8 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
       }
       __syncthreads();
       z0 = z1 = zero;
-#pragma unroll
-      for (int q = 0; q < AKQ; ++q)
-        if (4 * q < H1) {
+#pragma unroll 4
+      for (int q = 0; 4 * q < H1; ++q) {
           const double b = sW2[(4 * q + lk) * AS + col];
           z0 = mfma64(sA[lr * AS + 4 * q + lk], b, z0);
           z1 = mfma64(sA[(16 + lr) * AS + 4 * q + lk], b, z1);
@@ -472,7 +480,7 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
       for (int v = 0; v < 4; ++v) gb2 += TAN ? zb[0][v] : zb[0][v] + zb[1][v];
       __syncthreads();
       // dW2 += a1^T zb (rows of values and tangents in one sum); adjoints of a1 = zb W2^T
-#pragma unroll
+#pragma unroll 2
       for (int q = 0; q < AROWS / 4; ++q) {
         const double b = sZ[(4 * q + lk) * AS + col];
 #pragma unroll
@@ -480,9 +488,8 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
           if (16 * rb < H1) gW2[rb] = mfma64(sA[(4 * q + lk) * AS + rb * 16 + lr], b, gW2[rb]);
       }
       z0 = z1 = zero;
-#pragma unroll
-      for (int q = 0; q < AKQ; ++q)
-        if (4 * q < H2) {
+#pragma unroll 4
+      for (int q = 0; 4 * q < H2; ++q) {
           const double b = sW2[col * AS + 4 * q + lk];
           z0 = mfma64(sZ[lr * AS + 4 * q + lk], b, z0);
           z1 = mfma64(sZ[(16 + lr) * AS + 4 * q + lk], b, z1);
@@ -507,7 +514,7 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
     for (int v = 0; v < 4; ++v) gb1 += TAN ? zb[0][v] : zb[0][v] + zb[1][v];
     __syncthreads();
     // dW1 += x^T zb; window cotangents = zb W1^T
-#pragma unroll
+#pragma unroll 2
     for (int q = 0; q < AROWS / 4; ++q) {
       const double b = sA[(4 * q + lk) * AS + col];
 #pragma unroll
@@ -516,9 +523,8 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
     }
     if (wv * 16 < W) {
       z0 = z1 = zero;
-#pragma unroll
-      for (int q = 0; q < AKQ; ++q)
-        if (4 * q < H1) {
+#pragma unroll 4
+      for (int q = 0; 4 * q < H1; ++q) {
           const double b = col < W ? sW1[col * AS + 4 * q + lk] : 0.0;
           z0 = mfma64(sA[lr * AS + 4 * q + lk], b, z0);
           if (!TAN) z1 = mfma64(sA[(16 + lr) * AS + 4 * q + lk], b, z1);
@@ -571,7 +577,14 @@ __global__ __launch_bounds__(ANT) void k_adj_mlp(Adj a, const double* xin, const
     __syncthreads();
   }
   double* g = a.thp + (size_t)blockIdx.x * a.P;
-  for (int q = tid; q < a.P; q += ANT) g[q] += r[q];
+  for (int q0 = tid; q0 < a.P; q0 += 8 * ANT) {  // (8 loads in flight)
+    double v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = q0 + e * ANT < a.P ? g[q0 + e * ANT] : 0.0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (q0 + e * ANT < a.P) g[q0 + e * ANT] = v[e] + r[q0 + e * ANT];
+  }
 }
 
 // Global-network second-order adjoint (GLOBAL_MLP: f(n) = g(MLP(n / norm)), one scalar per
