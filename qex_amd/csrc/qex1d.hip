@@ -488,287 +488,242 @@ __global__ __launch_bounds__(NT) void k_mlp(Dev1 a, int k_launch) {
 
 // --------------------------------------------------------------------------------------------
 // k_mlp_mfma: the same windowed MLP on FP64 matrix cores (v_mfma_f64_16x16x4f64) for hidden
-// widths <= 64 and <= 4 hidden layers.  A wave takes 16 consecutive points of the flattened [B][N] grid through the
-// whole network, forward and backward, in its own LDS tile, so the waves of a workgroup share the
-// weights (LDS, copied once) and nothing else: no barriers, and one wave's activations run beside another's
-// matrix instructions.  The potential's tiles and the deferred energy's are separate items.
-// A workgroup of 4 waves per 48-point tile, with barriers between the layers and the weights read from L2 in the
-// k loops, took 366 us for 601 x 401 points of a 17-64-64-1 network (61 for 64 x 513, 50 for 32 x 513); now
-// 323, 60 and 40.  The matrix instructions alone are 104 us of the 323 and the activations' FP64 about as much:
-// the two share the FP64 units, so they add up.
+// widths <= 64 and <= 4 hidden layers.  A workgroup takes MP = 48 consecutive points of the
+// flattened [B][N] grid; each layer is a 48 x H tile GEMM (3 row blocks), wave w owning output
+// columns 16w..16w+15, written back in place into the one activation tile once every wave has
+// read it (25 KB of LDS, so three workgroups share a CU: the 64 x 513 points of a c2 batch are
+// 684 tiles, one round on 256 CUs with at most 144 points per CU).  Activation derivatives stay
+// in registers for the backward GEMMs (W^T).
 // MFMA operand layout (16x16x4, one wave): lane l supplies A[l%16][l/16] and B[l/16][l%16];
 // it receives D[4v + l/16][l%16] in element v.
 // --------------------------------------------------------------------------------------------
 typedef double d4_t __attribute__((ext_vector_type(4)));
-constexpr int MLP_P = 16;      // points of a wave's tile
+constexpr int MP = 48;         // points per workgroup (3 MFMA row blocks)
+constexpr int MLP_RB = MP / 16;  // row blocks of 16 points
 constexpr int MLP_HMAX = 64;   // widest hidden layer on the MFMA path
 constexpr int MLP_LH = 4;      // hidden layers on the MFMA path
-constexpr int MLP_S = 66;      // LDS row stride (doubles): a row block's operand reads touch all banks once
-constexpr int MLP_CB = MLP_HMAX / 16;  // column blocks
-constexpr int MLP_K = 8;       // k of a loop iteration
-constexpr int MLP_TILE = MLP_P * MLP_S + MLP_P;  // LDS of a wave (doubles)
-// waves of a workgroup: one workgroup a CU, as many waves as the weights leave LDS for, at most 2 a SIMD (at 3 the
-// activations spill: 345 us instead of 333 for 601 x 401 points)
-constexpr int mlp_waves(int hidden) { return hidden <= 3 ? 8 : 4; }
+constexpr int MLP_S = 65;      // LDS row stride (doubles) of the activation tiles
 
 __device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-__host__ __device__ constexpr int rup(int x, int m) { return (x + m - 1) / m * m; }
+__device__ __forceinline__ int rup(int x, int m) { return (x + m - 1) / m * m; }
 
-// the wave's own LDS writes are visible to its other lanes
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// acc[cb] = in[16 x K] . B[K x ncols], column block cb, B[k][col] = w[k * MLP_S + col] or, TRANS, w[col * MLP_S + k].
-// in and w are zero up to the next multiple of MLP_K of K; w also for columns past ncols (TRANS: these columns
-// of the result are not used).
-template <bool TRANS, int NB>
-__device__ __forceinline__ void tile_gemm_blocks(const double* in, int K, const double* w, int ncols, d4_t (&acc)[MLP_CB]) {
-  const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
-  const double* ap = in + lr * MLP_S + lk;
-  const double* bp = TRANS ? w + lk : w + lk * MLP_S + lr;
-  int at[NB];
+// acc[rb] (rows 16rb.., columns of this wave's block cb) = in[MP x K] . B[K x ncols], where
+// B[kk][col] = W[kk * ldw + col] (or W[col * ldw + kk] when trans); entries outside
+// kk < K, col < ncols are zero.  `in` is an LDS tile with row stride MLP_S, zero beyond K.
+__device__ __forceinline__ void tile_gemm(const double* in, int K, const double* W, int ldw, int ncols, bool trans,
+                                         int cb, d4_t (&acc)[MLP_RB]) {
+  const int l = threadIdx.x & 63;
 #pragma unroll
-  for (int cb = 0; cb < NB; ++cb) at[cb] = TRANS ? min(16 * cb + lr, ncols - 1) * MLP_S : 16 * cb;
-#pragma unroll 1
-  for (int k0 = 0; k0 < K; k0 += MLP_K) {
+  for (int rb = 0; rb < MLP_RB; ++rb) acc[rb] = (d4_t){0.0, 0.0, 0.0, 0.0};
+  const int col = cb * 16 + (l & 15);
+  const int kp = rup(K, 4);
+  for (int k0 = 0; k0 < kp; k0 += 4) {
+    const int kk = k0 + (l >> 4);
+    double bv = 0.0;
+    if (kk < K && col < ncols) bv = trans ? W[(size_t)col * ldw + kk] : W[(size_t)kk * ldw + col];
 #pragma unroll
-    for (int q = 0; q < MLP_K; q += 4) {
-      const double av = ap[q];
-#pragma unroll
-      for (int cb = 0; cb < NB; ++cb) acc[cb] = mfma64(av, bp[at[cb] + (TRANS ? q : q * MLP_S)], acc[cb]);
+    for (int rb = 0; rb < MLP_RB; ++rb) {
+      const double av = in[(rb * 16 + (l & 15)) * MLP_S + kk];
+      acc[rb] = mfma64(av, bv, acc[rb]);
     }
-    ap += MLP_K;
-    bp += TRANS ? MLP_K : MLP_K * MLP_S;
   }
 }
-template <bool TRANS>
-__device__ __forceinline__ void tile_gemm(const double* in, int K, const double* w, int ncols, d4_t (&acc)[MLP_CB]) {
-#pragma unroll
-  for (int cb = 0; cb < MLP_CB; ++cb) acc[cb] = (d4_t){0.0, 0.0, 0.0, 0.0};
-  if (ncols > 48)
-    tile_gemm_blocks<TRANS, 4>(in, K, w, ncols, acc);
-  else if (ncols > 32)
-    tile_gemm_blocks<TRANS, 3>(in, K, w, ncols, acc);
-  else if (ncols > 16)
-    tile_gemm_blocks<TRANS, 2>(in, K, w, ncols, acc);
-  else
-    tile_gemm_blocks<TRANS, 1>(in, K, w, ncols, acc);
-}
 
-// One hidden layer of the tile: x <- act(x W + b), in place; keeps act' in dz.
-__device__ __forceinline__ void mlp_hidden_fwd(const Dev1& a, int lh, const double* w, const double* bl, double* x, double (&dz)[MLP_CB][4]) {
-  const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+// One hidden layer of the tile MLP: nxt = act(cur W_lh + b_lh); keeps act' in dzl.
+__device__ __forceinline__ void mlp_hidden_fwd(const Dev1& a, int lh, const double* cur, double* nxt,
+                                               double (&dzl)[MLP_RB][4], int wv, int l) {
   const int fi = a.widths[lh], fo = a.widths[lh + 1];
-  double bias[MLP_CB];
+  const double* Wl = a.mlp + a.woff[lh];
+  const double* bl = a.mlp + a.boff[lh];
+  d4_t acc[MLP_RB];
+  tile_gemm(cur, fi, Wl, fo, fo, false, wv, acc);
+  const int col = wv * 16 + (l & 15);
+  const double bias = col < fo ? bl[col] : 0.0;
+  __syncthreads();  // every wave has read cur (nxt may be the same tile)
 #pragma unroll
-  for (int cb = 0; cb < MLP_CB; ++cb) bias[cb] = bl[16 * cb + lr];
-  d4_t acc[MLP_CB];
-  tile_gemm<false>(x, fi, w, fo, acc);
-  wave_sync();  // (the tile has been read)
-  // one column block an iteration, the blocks rotating through acc[0] and dz[MLP_CB - 1]: unrolled, the
-  // activations are 30 KB of instructions that every wave runs through once a tile, and fetching them took
-  // longer than running them
-#pragma unroll 1
-  for (int cb = 0; cb < MLP_CB; ++cb) {
-    double d[4];
-    if (16 * cb < fo) {
-      const int col = 16 * cb + lr;
+  for (int rb = 0; rb < MLP_RB; ++rb) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const double y = act_fwd(a.act, acc[0][v] + bias[0], &d[v]);
-        x[(4 * v + lk) * MLP_S + col] = col < fo ? y : 0.0;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int row = rb * 16 + 4 * v + (l >> 4);
+      double d;
+      const double y = act_fwd(a.act, acc[rb][v] + bias, &d);
+      nxt[row * MLP_S + col] = col < fo ? y : 0.0;
+      dzl[rb][v] = col < fo ? d : 0.0;
     }
-#pragma unroll
-    for (int c = 0; c + 1 < MLP_CB; ++c) {
-      acc[c] = acc[c + 1];
-      bias[c] = bias[c + 1];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) dz[c][v] = dz[c + 1][v];
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) dz[MLP_CB - 1][v] = d[v];
   }
-  wave_sync();
+  __syncthreads();
 }
 
-// Backward through hidden layer lh: x <- (x W_lh^T) * act'(z_{lh-1}), in place (dz: act' of lh - 1).
-__device__ __forceinline__ void mlp_hidden_bwd(const Dev1& a, int lh, const double* w, double* x, const double (&dz)[MLP_CB][4]) {
-  const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+// Backward through hidden layer lh: nxt = (cur W_lh^T) * act'(z_{lh-1}) (dzp holds act' of lh-1).
+__device__ __forceinline__ void mlp_hidden_bwd(const Dev1& a, int lh, const double* cur, double* nxt,
+                                               const double (&dzp)[MLP_RB][4], int wv, int l) {
   const int fi = a.widths[lh], fo = a.widths[lh + 1];
-  d4_t acc[MLP_CB];
-  tile_gemm<true>(x, fo, w, fi, acc);
-  wave_sync();
+  const double* Wl = a.mlp + a.woff[lh];
+  d4_t acc[MLP_RB];
+  tile_gemm(cur, fo, Wl, fo, fi, true, wv, acc);
+  const int col = wv * 16 + (l & 15);
+  __syncthreads();  // every wave has read cur (nxt may be the same tile)
 #pragma unroll
-  for (int cb = 0; cb < MLP_CB; ++cb)
-    if (16 * cb < fi)
+  for (int rb = 0; rb < MLP_RB; ++rb)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) x[(4 * v + lk) * MLP_S + 16 * cb + lr] = 16 * cb + lr < fi ? acc[cb][v] * dz[cb][v] : 0.0;
-  wave_sync();
+    for (int v = 0; v < 4; ++v) {
+      const int row = rb * 16 + 4 * v + (l >> 4);
+      nxt[row * MLP_S + col] = col < fi ? acc[rb][v] * dzp[rb][v] : 0.0;
+    }
+  __syncthreads();
 }
 
 // Gradient at the last hidden layer's pre-activations: cot_row * w_out[col] * act'.
-__device__ __forceinline__ void mlp_out_grad(double* x, const double* cot, const double* wo, int fo, const double (&dz)[MLP_CB][4]) {
-  const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+__device__ __forceinline__ void mlp_out_grad(double* nxt, const double* cot, double wo, const double (&dzl)[MLP_RB][4],
+                                             int col, int l) {
 #pragma unroll
-  for (int cb = 0; cb < MLP_CB; ++cb)
-    if (16 * cb < fo) {
-      const int col = 16 * cb + lr;
-      const double w = col < fo ? wo[col] : 0.0;
+  for (int rb = 0; rb < MLP_RB; ++rb)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) x[(4 * v + lk) * MLP_S + col] = col < fo ? cot[4 * v + lk] * w * dz[cb][v] : 0.0;
+    for (int v = 0; v < 4; ++v) {
+      const int row = rb * 16 + 4 * v + (l >> 4);
+      nxt[row * MLP_S + col] = cot[row] * wo * dzl[rb][v];
     }
-  wave_sync();
 }
 
 template <int NH>
-__global__ __launch_bounds__(mlp_waves(NH) * 64) void k_mlp_mfma(Dev1 a, int k_launch) {
+__global__ __launch_bounds__(NT, NH <= 2 ? 3 : 2) void k_mlp_mfma(Dev1 a, int k_launch) {
   extern __shared__ double smem[];
-  constexpr int NTM = mlp_waves(NH) * 64;
-  const int tid = threadIdx.x, l = tid & 63, lr = l & 15, lk = l >> 4, wv = tid >> 6;
-  const int N = a.N, W = a.W, h = W / 2;
+  // one activation tile: each layer's GEMM keeps its result in registers until every wave has
+  // read the tile, then writes it back in place (34 KB of LDS: three workgroups per CU)
+  double* bufB = smem;                 // MP x MLP_S
+  double* cot = bufB + MP * MLP_S;     // MP cotangents
+  __shared__ int sh_any[2];
+  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
+  const int N = a.N, W = a.W, h = W / 2, L = a.nlay;
   const long total = (long)a.B * N;
-  const long tiles = (total + MLP_P - 1) / MLP_P;
+  const long g0 = (long)blockIdx.x * MP;
   const bool sym = a.reflect && xc_is_local(a.xc);
-  // ---- weights into LDS, rows to a multiple of MLP_K and all columns zero filled ----
-  const double* w[NH];
-  double* at = smem;
-#pragma unroll
-  for (int lh = 0; lh < NH; ++lh) {
-    w[lh] = at;
-    const int fi = a.widths[lh], fo = a.widths[lh + 1], rows = rup(fi, MLP_K);
-    const double* Wl = a.mlp + a.woff[lh];
-    // (8 loads in flight a thread)
-    for (int q0 = tid; q0 < rows * MLP_HMAX; q0 += 8 * NTM) {
-      double v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int q = q0 + e * NTM, r = q / MLP_HMAX, c = q % MLP_HMAX;
-        v[e] = r < fi && c < fo ? Wl[r * fo + c] : 0.0;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int q = q0 + e * NTM;
-        if (q < rows * MLP_HMAX) at[q / MLP_HMAX * MLP_S + q % MLP_HMAX] = v[e];
-      }
-    }
-    at += rows * MLP_S;
-  }
-  // biases of the hidden layers, then the output layer's weights
-  const double* vec = at;
-  for (int q = tid; q < (NH + 1) * MLP_HMAX; q += NTM) {
-    const int lh = q / MLP_HMAX, c = q % MLP_HMAX;
-    const int n = lh < NH ? a.widths[lh + 1] : a.widths[NH];
-    at[q] = c < n ? a.mlp[(lh < NH ? a.boff[lh] : a.woff[NH]) + c] : 0.0;
-  }
-  at += (NH + 1) * MLP_HMAX;
-  const double b_out = a.mlp[a.boff[NH]];
-  double* x = at + wv * MLP_TILE;      // the wave's tile
-  double* cot = x + MLP_P * MLP_S;     // cotangents of its points
+  if (tid < 2) sh_any[tid] = 0;
   __syncthreads();
-  const int hl = a.widths[NH], wp = rup(W, MLP_K);
-  const double* WL = vec + NH * MLP_HMAX;
-  // items: the tiles of the potential (forward and backward), then those of the deferred energy (forward)
-  for (long item = blockIdx.x + (long)gridDim.x * wv; item < 2 * tiles; item += (long)gridDim.x * mlp_waves(NH)) {
-    const bool pot = item < tiles;
-    const long g0 = (pot ? item : item - tiles) * MLP_P;
-    // ---- window inputs (x / norm), zero padded to a multiple of MLP_K columns ----
-    // 4 lanes per point: the system index and status are read once per point, and a lane's
+  if (tid < MP) {
+    const long g = g0 + tid;
+    if (g < total) {
+      const int s = (int)(g / N);
+      const int k = iter_of(a, s, k_launch);
+      if (k >= 0 && k < a.T && !a.st[4 * s + 0]) sh_any[0] = 1;
+      if (a.st[4 * s + 1] >= 0 && a.st[4 * s + 1] < a.T) sh_any[1] = 1;
+    }
+  }
+  __syncthreads();
+  const bool any_pot = sh_any[0] != 0, any_e = sh_any[1] != 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    if (pass == 0 && !any_pot) continue;
+    if (pass == 1 && !any_e) continue;
+    const bool backward = pass == 0;
+    // ---- window inputs (x / norm) into bufB, zero padded to a multiple of 4 columns ----
+    // 4 threads per point: the system index and status are read once per point, and a thread's
     // window loads are independent, so they are in flight together
-    {
-      const int p = l >> 2;
+    static_assert(MP * 4 <= NT, "4 threads per point");
+    const int wp = rup(W, 4);
+    if (tid < MP * 4) {
+      const int p = tid >> 2;
       const long g = g0 + p;
       const bool inb = g < total;
-      // (one 64-bit division a tile, of uniform operands)
-      int s = (int)(g0 / N), i = (int)(g0 - (long)s * N) + p;
-      while (i >= N) {
-        i -= N;
-        ++s;
-      }
-      if (!inb) s = i = 0;
+      const int s = inb ? (int)(g / N) : 0, i = inb ? (int)(g % N) : 0;
       const int k = iter_of(a, s, k_launch);
-      const int ke = a.st[4 * s + 1];
-      const bool act = inb && (pot ? (k >= 0 && k < a.T && !a.st[4 * s + 0]) : (ke >= 0 && ke < a.T));
-      if (!__any(act)) continue;
-      const double* src = !act ? nullptr : pot ? input_density(a, s, k) : a.o_xc + (size_t)s * N;
+      const bool act =
+          inb && (pass == 0 ? (k >= 0 && k < a.T && !a.st[4 * s + 0]) : (a.st[4 * s + 1] >= 0 && a.st[4 * s + 1] < a.T));
+      const double* src = !act ? nullptr : pass == 0 ? input_density(a, s, k) : a.o_xc + (size_t)s * N;
       int lo = 0, hi = -1;
-      if (pot && sym && act) {
+      if (pass == 0 && sym && act) {
         lo = a.win[2 * s];
         hi = a.win[2 * s + 1];
       }
 #pragma unroll 4
-      for (int o = l & 3; o < wp; o += 4) {
+      for (int o = tid & 3; o < wp; o += 4) {
         const int j = i + o - h;
-        double v = 0.0;
+        double x = 0.0;
         if (act && o < W && j >= 0 && j < N) {
-          v = src[j];
-          if (pot && sym) v = 0.5 * (v + src[mirror(j, lo, hi)]);
-          v /= a.norm;
+          x = src[j];
+          if (pass == 0 && sym) x = 0.5 * (x + src[mirror(j, lo, hi)]);
+          x /= a.norm;
         }
-        if (o == h) cot[p] = act ? v * a.norm : 0.0;  // the point's own density (cotangent of e)
-        x[p * MLP_S + o] = v;
+        if (o == h) cot[p] = act ? x * a.norm : 0.0;  // the point's own density (cotangent of e)
+        bufB[p * MLP_S + o] = x;
       }
-      wave_sync();
     }
+    __syncthreads();
     // ---- hidden layers (one named register array of activation derivatives per layer) ----
-    double dz0[MLP_CB][4], dz1[MLP_CB][4], dz2[MLP_CB][4], dz3[MLP_CB][4];
-    mlp_hidden_fwd(a, 0, w[0], vec + 0 * MLP_HMAX, x, dz0);
-    if constexpr (NH > 1) mlp_hidden_fwd(a, 1, w[1], vec + 1 * MLP_HMAX, x, dz1);
-    if constexpr (NH > 2) mlp_hidden_fwd(a, 2, w[2], vec + 2 * MLP_HMAX, x, dz2);
-    if constexpr (NH > 3) mlp_hidden_fwd(a, 3, w[3], vec + 3 * MLP_HMAX, x, dz3);
+    // NH (compile time) = L - 1 hidden layers; only the arrays in use stay live
+    double dz0[MLP_RB][4], dz1[NH > 1 ? MLP_RB : 1][4], dz2[NH > 2 ? MLP_RB : 1][4], dz3[NH > 3 ? MLP_RB : 1][4];
+    double* cur = bufB;
+    double* nxt = bufB;
+    auto swap_bufs = [&]() {};
+    if constexpr (NH > 0) { mlp_hidden_fwd(a, 0, cur, nxt, dz0, wv, l); swap_bufs(); }
+    if constexpr (NH > 1) { mlp_hidden_fwd(a, 1, cur, nxt, dz1, wv, l); swap_bufs(); }
+    if constexpr (NH > 2) { mlp_hidden_fwd(a, 2, cur, nxt, dz2, wv, l); swap_bufs(); }
+    if constexpr (NH > 3) { mlp_hidden_fwd(a, 3, cur, nxt, dz3, wv, l); swap_bufs(); }
     // ---- output layer (fan_out 1): 4 lanes per point ----
+    const int hl = a.widths[L - 1];
+    const double* WL = a.mlp + a.woff[L - 1];
     {
-      const int p = l >> 2, q = l & 3;
+      const int p = tid >> 2, q = tid & 3;
       double part = 0.0;
-#pragma unroll 4
-      for (int u = q; u < hl; u += 4) part = fma(x[p * MLP_S + u], WL[u], part);
+      if (p < MP)
+        for (int u = q; u < hl; u += 4) part = fma(cur[p * MLP_S + u], WL[u], part);
       part += __shfl_xor(part, 1, 64);
       part += __shfl_xor(part, 2, 64);
       const long g = g0 + p;
-      if (q == 0) {
+      if (q == 0 && p < MP) {
         double de;
-        const double e = out_transform(a.mlpout, part + b_out, &de);
-        if (g < total) (pot ? a.mlp_e : a.mlp_eout)[g] = e;
-        cot[p] *= de;  // cotangent of the raw output
-      }
-      wave_sync();
-    }
-    if (!pot) continue;
-    // ---- backward: g_{NH} = cot * w_out * act'(z_{NH}), g_{l-1} = (g_l W_l^T) * act'(z_{l-1}) ----
-    if constexpr (NH == 1) mlp_out_grad(x, cot, WL, hl, dz0);
-    if constexpr (NH == 2) mlp_out_grad(x, cot, WL, hl, dz1);
-    if constexpr (NH == 3) mlp_out_grad(x, cot, WL, hl, dz2);
-    if constexpr (NH == 4) mlp_out_grad(x, cot, WL, hl, dz3);
-    if constexpr (NH > 3) mlp_hidden_bwd(a, 3, w[3], x, dz2);
-    if constexpr (NH > 2) mlp_hidden_bwd(a, 2, w[2], x, dz1);
-    if constexpr (NH > 1) mlp_hidden_bwd(a, 1, w[1], x, dz0);
-    // gX = g_0 W_0^T (window columns)
-    d4_t acc[MLP_CB];
-    tile_gemm<true>(x, a.widths[1], w[0], W, acc);
-#pragma unroll
-    for (int cb = 0; cb < MLP_CB; ++cb)
-      if (16 * cb < W) {
-        const int col = 16 * cb + lr;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const long g = g0 + 4 * v + lk;
-          if (col < W && g < total) a.mlp_G[g * W + col] = acc[cb][v];
+        const double e = out_transform(a.mlpout, part + a.mlp[a.boff[L - 1]], &de);
+        if (g < total) {
+          if (pass == 0)
+            a.mlp_e[g] = e;
+          else
+            a.mlp_eout[g] = e;
         }
+        if (pass == 0) cot[p] *= de;  // cotangent of the raw output (read after the next barrier)
       }
-    wave_sync();  // (the tile and its cotangents have been read)
+    }
+    if (!backward) {
+      __syncthreads();
+      continue;
+    }
+    // ---- backward: g_{L-2} = cot * w_out * act'(z_{L-2}) ----
+    __syncthreads();
+    {
+      const int col = wv * 16 + (l & 15);
+      const double wo = col < hl ? WL[col] : 0.0;
+      if constexpr (NH == 1) mlp_out_grad(nxt, cot, wo, dz0, col, l);
+      if constexpr (NH == 2) mlp_out_grad(nxt, cot, wo, dz1, col, l);
+      if constexpr (NH == 3) mlp_out_grad(nxt, cot, wo, dz2, col, l);
+      if constexpr (NH == 4) mlp_out_grad(nxt, cot, wo, dz3, col, l);
+    }
+    __syncthreads();
+    swap_bufs();
+    // g_{l-1} = (g_l W_l^T) * act'(z_{l-1}), l = L-2 .. 1
+    if constexpr (NH > 3) { mlp_hidden_bwd(a, 3, cur, nxt, dz2, wv, l); swap_bufs(); }
+    if constexpr (NH > 2) { mlp_hidden_bwd(a, 2, cur, nxt, dz1, wv, l); swap_bufs(); }
+    if constexpr (NH > 1) { mlp_hidden_bwd(a, 1, cur, nxt, dz0, wv, l); swap_bufs(); }
+    // gX = g_0 W_0^T  (window columns): waves 0..ceil(W/16)-1
+    {
+      const int f1 = a.widths[1];
+      const double* W0 = a.mlp + a.woff[0];
+      if (wv * 16 < W) {
+        d4_t acc[MLP_RB];
+        tile_gemm(cur, f1, W0, f1, W, true, wv, acc);
+        const int col = wv * 16 + (l & 15);
+#pragma unroll
+        for (int rb = 0; rb < MLP_RB; ++rb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int row = rb * 16 + 4 * v + (l >> 4);
+            const long g = g0 + row;
+            if (col < W && g < total) a.mlp_G[g * W + col] = acc[rb][v];
+          }
+      }
+    }
+    __syncthreads();
   }
-}
-
-// LDS of a workgroup: the weights and biases, and a tile per wave
-size_t mlp_mfma_lds(const Dev1& a) {
-  size_t rows = 0;
-  for (int lh = 0; lh < a.nlay - 1; ++lh) rows += rup(a.widths[lh], MLP_K);
-  return (rows * MLP_S + (size_t)a.nlay * MLP_HMAX + (size_t)mlp_waves(a.nlay - 1) * MLP_TILE) * 8;
 }
 
 // --------------------------------------------------------------------------------------------
@@ -2141,7 +2096,6 @@ size_t mlp_lds_bytes(const Dev1& a, int lpp) {
   return ((size_t)a.N + 2 * P * stride + (size_t)(a.nlay - 1) * P * stride) * 8;
 }
 constexpr size_t LDS_MAX = 160 * 1024;
-constexpr int NCU = 256;  // CUs of an MI355X
 size_t gmlp_lds_bytes(const Dev1& a) {
   return ((size_t)a.N + 2 * (size_t)(a.nlay - 1) * a.hmax + NT + 2 * (size_t)a.hmax) * 8;
 }
@@ -2362,20 +2316,17 @@ void fill_network(const qex1d_problem* p, Dev1& a) {
 // Launch shapes and LDS of the network kernels and of the potential kernel's grid.
 int plan_network(Plan1d* P) {
   const Dev1& a = P->a;
-  bool mlp_mfma = a.xc == QEX1D_XC_LOCAL_MLP && a.nlay - 1 <= MLP_LH && a.W <= MLP_HMAX;
+  bool mlp_mfma = a.xc == QEX1D_XC_LOCAL_MLP && a.nlay - 1 <= MLP_LH && a.W <= MLP_S - 1;
   for (int l = 1; l < a.nlay && mlp_mfma; ++l) mlp_mfma = a.widths[l] <= MLP_HMAX;
-  mlp_mfma = mlp_mfma && mlp_mfma_lds(a) <= LDS_MAX;
   P->mlp_mfma = mlp_mfma;
   // the generic path: 8 lanes per point (32 points per workgroup) when their activations fit in
   // LDS, else 64 lanes per point (4 points)
   P->mlp_lpp = mlp_lds_bytes(a, 8) <= LDS_MAX ? 8 : 64;
-  P->lds_mlp = a.xc != QEX1D_XC_LOCAL_MLP ? 0 : mlp_mfma ? mlp_mfma_lds(a) : mlp_lds_bytes(a, P->mlp_lpp);
+  P->lds_mlp = a.xc != QEX1D_XC_LOCAL_MLP ? 0 : mlp_mfma ? (size_t)(MP * MLP_S + MP) * 8 : mlp_lds_bytes(a, P->mlp_lpp);
   if (P->lds_mlp > LDS_MAX) return fail(QEX_E_UNSUPPORTED, "MLP too wide for LDS (%zu bytes)", P->lds_mlp);
   P->lds_gmlp = a.xc != QEX1D_XC_GLOBAL_MLP ? 0 : gmlp_lds_bytes(a);
   if (P->lds_gmlp > LDS_MAX) return fail(QEX_E_UNSUPPORTED, "global MLP too wide for LDS (%zu bytes)", P->lds_gmlp);
-  // one workgroup a CU; the items go to the workgroups in turn, so few of them spread over the CUs
-  const long items = 2 * (((long)a.B * a.N + MLP_P - 1) / MLP_P);
-  P->gmlp_mfma = dim3((unsigned)(items < NCU ? items : NCU));
+  P->gmlp_mfma = dim3((unsigned)(((long)a.B * a.N + MP - 1) / MP));
   P->gpot = dim3(a.nTiles, a.B);
   P->gmlp = dim3((a.N + NT / P->mlp_lpp - 1) / (NT / P->mlp_lpp), a.B);
   const void* mlp_fn = P->mlp_lpp == 8 ? (const void*)k_mlp<8> : (const void*)k_mlp<64>;
@@ -2398,10 +2349,10 @@ void launch_network(const Plan1d& P, int k, hipStream_t stream) {
     Scope ps(qexprof::K_MLP, stream);
     if (P.mlp_mfma) {
       switch (a.nlay - 1) {
-        case 1: hipLaunchKernelGGL(k_mlp_mfma<1>, P.gmlp_mfma, dim3(mlp_waves(1) * 64), P.lds_mlp, stream, a, k); break;
-        case 2: hipLaunchKernelGGL(k_mlp_mfma<2>, P.gmlp_mfma, dim3(mlp_waves(2) * 64), P.lds_mlp, stream, a, k); break;
-        case 3: hipLaunchKernelGGL(k_mlp_mfma<3>, P.gmlp_mfma, dim3(mlp_waves(3) * 64), P.lds_mlp, stream, a, k); break;
-        default: hipLaunchKernelGGL(k_mlp_mfma<4>, P.gmlp_mfma, dim3(mlp_waves(4) * 64), P.lds_mlp, stream, a, k); break;
+        case 1: hipLaunchKernelGGL(k_mlp_mfma<1>, P.gmlp_mfma, dim3(NT), P.lds_mlp, stream, a, k); break;
+        case 2: hipLaunchKernelGGL(k_mlp_mfma<2>, P.gmlp_mfma, dim3(NT), P.lds_mlp, stream, a, k); break;
+        case 3: hipLaunchKernelGGL(k_mlp_mfma<3>, P.gmlp_mfma, dim3(NT), P.lds_mlp, stream, a, k); break;
+        default: hipLaunchKernelGGL(k_mlp_mfma<4>, P.gmlp_mfma, dim3(NT), P.lds_mlp, stream, a, k); break;
       }
     } else if (P.mlp_lpp == 8) {
       hipLaunchKernelGGL(k_mlp<8>, P.gmlp, dim3(NT), P.lds_mlp, stream, a, k);
