@@ -25,6 +25,7 @@
 #include "qex.h"
 #include "prof.h"
 #include "symeig.h"
+#include "symeig_lds.h"
 
 namespace {
 
@@ -1742,6 +1743,7 @@ struct Scf3 {
   int prec, x32blk;   // grid precision; workgroups of the FP32 grid kernels for this molecule
   // state (workspace)
   double *Fd, *D, *C, *mo, *J, *K, *Vxc, *vpart, *spart, *rho, *tmp2;
+  double *F, *Cp, *tmp1;  // (FP32 grid path)
   double *diisF, *diisE, *diisB;  // [space][n*n], [space][n*n], [(space+1)^2]
   double* scal;                    // [0] e_tot, [1] e_last, [2] nelec, [3] exc (LDA), [4] gnorm, [5] exc (network)
   int* ist;                        // [0] frozen, [1] cycles done, [2] diis count, [3] diis head, [4] converged
@@ -1925,7 +1927,7 @@ __device__ __forceinline__ void diis_solve(int m, const double* b, int M, const 
 //     used, whose first n_occ columns equal the cycle's bit for bit.
 __global__ __launch_bounds__(NT_EIG) void k_scf_step(const Scf3* __restrict__ ss, int ecycle, int fcycle, int full) {
   const Scf3 s = ss[blockIdx.x];
-  if (s.ist[0] && !full) return;
+  if (s.prec == QEX3D_PRECISION_FP32_GRID || (s.ist[0] && !full)) return;
   extern __shared__ __attribute__((aligned(16))) double sm[];
   __shared__ qexeig::Smem sh;
   __shared__ double red[QEX3D_MAX_DIIS][NW_EIG];
@@ -2116,6 +2118,215 @@ __global__ __launch_bounds__(NT_EIG) void k_scf_step(const Scf3* __restrict__ ss
   lds_gemm(n, n, nocc, rows(Z), rows(Z), [&](int r, int c, double x) { s.D[r * n + c] = 2.0 * x; });
 }
 
+// ---- the same step for the molecules of the FP32 grid path, as three kernels ----
+// FP32 rounding in V multiplies a rounding change of the orbitals to 1e-8 of the density matrix (symeig_lds.h), so
+// these molecules keep these kernels' order of operations, and with it their results; k_scf_step takes the others.
+__device__ __forceinline__ bool fp32_grid(const Scf3& s) { return s.prec == QEX3D_PRECISION_FP32_GRID; }
+
+// Fock + CDIIS (one workgroup of NT_SCF threads).  cycle < 0: plain F = H + Veff (no DIIS).
+constexpr int NT_SCF = 1024;
+constexpr int NW_SCF = NT_SCF / 64;
+__global__ __launch_bounds__(NT_SCF) void k_scf_fock(const Scf3* __restrict__ ss, int cycle) {
+  const Scf3 s = ss[blockIdx.x];
+  if (!fp32_grid(s) || s.ist[0]) return;
+  __shared__ double redm[QEX3D_MAX_DIIS][NW_SCF];
+  const int n = s.n, nn = n * n;
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+    s.F[t] = s.H[t] + s.J[t] + s.Vxc[t];
+  }
+  __syncthreads();
+  if (cycle < 1 || s.diis_space < 1) {
+    for (int t = threadIdx.x; t < nn; t += NT_SCF) s.Fd[t] = s.F[t];
+    __syncthreads();
+    return;
+  }
+  // error e = F D S - S D F
+  mfma_gemm(n, n, n, glob(s.F, n, 1), glob(s.D, 1, n), s.tmp1, n, 1.0);     // FD
+  mfma_gemm(n, n, n, glob(s.tmp1, n, 1), glob(s.S, 1, n), s.tmp2, n, 1.0);  // FDS
+  // S D F = (F D S)^T for symmetric F, D, S
+  const int cnt = s.ist[2], head = s.ist[3];
+  const int slot = head;
+  double* Fi = s.diisF + (size_t)slot * nn;
+  double* Ei = s.diisE + (size_t)slot * nn;
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+    const int i = t / n, j = t % n;
+    Ei[t] = s.tmp2[i * n + j] - s.tmp2[j * n + i];
+    Fi[t] = s.F[t];
+  }
+  __syncthreads();
+  const int m = cnt + 1 < s.diis_space ? cnt + 1 : s.diis_space;
+  // B (stored by slot) row/column of the new vector: the m dot products in one pass
+  const int M = s.diis_space;
+  {
+    double d[QEX3D_MAX_DIIS];
+#pragma unroll
+    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) d[q] = 0.0;
+    for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+      const double e = Ei[t];
+#pragma unroll
+      for (int q = 0; q < QEX3D_MAX_DIIS; ++q)
+        if (q < m) d[q] = fma(e, s.diisE[(size_t)q * nn + t], d[q]);
+    }
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < QEX3D_MAX_DIIS; ++q) {
+      const double x = wsum(d[q]);
+      if (l == 0) redm[q][w] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x < m) {
+      const int q = threadIdx.x;
+      double v = 0.0;
+      for (int k = 0; k < NW_SCF; ++k) v += redm[q][k];
+      s.diisB[slot * M + q] = v;
+      s.diisB[q * M + slot] = v;
+    }
+    __syncthreads();
+  }
+  // solve [0 -1; -1 B] [l; c] = [-1; 0] in the chronological order of the stored vectors
+  __shared__ double Bm[(QEX3D_MAX_DIIS + 1) * (QEX3D_MAX_DIIS + 2)];
+  __shared__ double coef[QEX3D_MAX_DIIS + 1];
+  __shared__ int order[QEX3D_MAX_DIIS];
+  if (threadIdx.x == 0) {
+    const int oldest = m < M ? 0 : (slot + 1) % M;
+    for (int q = 0; q < m; ++q) order[q] = (oldest + q) % M;
+    const int dim = m + 1, ld = m + 2;
+    for (int r = 0; r < dim; ++r)
+      for (int c = 0; c < dim; ++c) {
+        double v;
+        if (r == 0 && c == 0)
+          v = 0.0;
+        else if (r == 0 || c == 0)
+          v = -1.0;
+        else
+          v = s.diisB[order[r - 1] * M + order[c - 1]];
+        Bm[r * ld + c] = v;
+      }
+    for (int r = 0; r < dim; ++r) Bm[r * ld + dim] = r == 0 ? -1.0 : 0.0;
+    // Gaussian elimination with partial pivoting
+    for (int c = 0; c < dim; ++c) {
+      int pr = c;
+      for (int r = c + 1; r < dim; ++r)
+        if (fabs(Bm[r * ld + c]) > fabs(Bm[pr * ld + c])) pr = r;
+      if (pr != c)
+        for (int k = 0; k <= dim; ++k) {
+          const double t = Bm[c * ld + k];
+          Bm[c * ld + k] = Bm[pr * ld + k];
+          Bm[pr * ld + k] = t;
+        }
+      const double pv = Bm[c * ld + c];
+      for (int r = c + 1; r < dim; ++r) {
+        const double f = Bm[r * ld + c] / pv;
+        for (int k = c; k <= dim; ++k) Bm[r * ld + k] -= f * Bm[c * ld + k];
+      }
+    }
+    for (int r = dim - 1; r >= 0; --r) {
+      double v = Bm[r * ld + dim];
+      for (int k = r + 1; k < dim; ++k) v -= Bm[r * ld + k] * coef[k];
+      coef[r] = v / Bm[r * ld + r];
+    }
+    s.ist[2] = m;
+    s.ist[3] = (slot + 1) % M;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+    double f = 0.0;
+    for (int q = 0; q < m; ++q) f = fma(coef[q + 1], s.diisF[(size_t)order[q] * nn + t], f);
+    s.Fd[t] = f;
+  }
+  __syncthreads();
+}
+
+// generalized eigh of Fd: Fp = X^T Fd X (symmetrised), Fp = Z diag(e) Z^T in LDS, C = X Z,
+// D = 2 C_occ C_occ^T.  One workgroup of NT_SCF threads.
+// full = 0 (the SCF cycles): only the orbitals the cycle uses (the n_occ + 2 lowest; C's other
+// columns zero, their energies unrefined); full = 1 (after the last cycle, every molecule, frozen or
+// not): the whole solve, whose first n_occ + 2 columns equal the cycles' bit for bit.
+__global__ __launch_bounds__(NT_SCF) void k_scf_eigh(const Scf3* __restrict__ ss, int full) {
+  const Scf3 s = ss[blockIdx.x];
+  if (!fp32_grid(s) || (s.ist[0] && !full)) return;
+  extern __shared__ __attribute__((aligned(16))) double sm[];
+  __shared__ qexeig_lds::Smem sh;
+  const int n = s.n, nn = n * n, S = n + 1;
+  double* A = sm;
+  double* Z = A + (size_t)n * S;
+  mfma_gemm(n, n, n, glob(s.Fd, n, 1), glob(s.X, 1, n), s.tmp1, n, 1.0);  // Fd X
+  mfma_gemm(n, n, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), A, S, 1.0);      // X^T Fd X (into LDS)
+  for (int t = threadIdx.x; t < nn; t += blockDim.x) {
+    const int i = t / n, j = t % n;
+    if (i < j) {
+      const double v = 0.5 * (A[i * S + j] + A[j * S + i]);
+      A[i * S + j] = v;
+      A[j * S + i] = v;
+    }
+  }
+  __syncthreads();
+  qexeig_lds::symeig(n, A, Z, S, s.mo, s.eigf, sh, full ? n : s.nocc + 2);
+  mfma_gemm(n, n, n, glob(s.X, n, 1), lds(Z, 1, S), s.C, n, 1.0);  // C = X Z
+  mfma_gemm(n, n, s.nocc, glob(s.C, n, 1), glob(s.C, n, 1), s.D, n, 2.0);  // D = 2 C_occ C_occ^T
+}
+
+// Energies and convergence (one workgroup of NT_SCF threads).
+__global__ __launch_bounds__(NT_SCF) void k_scf_energy(const Scf3* __restrict__ ss, int cycle) {
+  const Scf3 s = ss[blockIdx.x];
+  if (!fp32_grid(s) || s.ist[0]) return;
+  __shared__ double red[NW_SCF];
+  const int n = s.n, nn = n * n, nocc = s.nocc;
+  double e1 = 0.0, e2 = 0.0;
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+    e1 = fma(s.D[t], s.H[t], e1);
+    e2 = fma(s.D[t], 0.5 * s.J[t], e2);
+  }
+  e1 = bsum(e1, red);
+  e2 = bsum(e2, red);
+  const double etot = e1 + e2 + (has_point_exc(s.method) ? s.scal[3] : s.method == QEX3D_RKS_NN_GLOBAL ? s.scal[5] : 0.0) +
+                      s.enuc;
+  if (cycle < 0) {
+    if (threadIdx.x == 0) {
+      s.scal[0] = etot;
+      s.e_hist[0] = etot;
+    }
+    return;
+  }
+  // orbital gradient norm with the new Fock matrix: |C_vir^T F C_occ|^2 via the S^-1 projector
+  // = tr(Co^T F X X^T F Co) - |Co^T F Co|^2, times 4 (the factor 2 of pyscf's get_grad)
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) {
+    s.F[t] = s.H[t] + s.J[t] + s.Vxc[t];
+  }
+  __syncthreads();
+  mfma_gemm(n, nocc, n, glob(s.F, n, 1), glob(s.C, 1, n), s.tmp1, n, 1.0);    // tmp1 = F C_occ   (n x nocc)
+  mfma_gemm(n, nocc, n, glob(s.X, 1, n), glob(s.tmp1, 1, n), s.tmp2, n, 1.0);  // tmp2 = X^T F C_occ
+  mfma_gemm(nocc, nocc, n, glob(s.C, 1, n), glob(s.tmp1, 1, n), s.Cp, n, 1.0); // Cp = C_occ^T F C_occ
+  double a = 0.0, b = 0.0;
+  for (int t = threadIdx.x; t < n * nocc; t += NT_SCF) {
+    const double v = s.tmp2[(t / nocc) * n + t % nocc];
+    a = fma(v, v, a);
+  }
+  for (int t = threadIdx.x; t < nocc * nocc; t += NT_SCF) {
+    const double v = s.Cp[(t / nocc) * n + t % nocc];
+    b = fma(v, v, b);
+  }
+  a = bsum(a, red);
+  b = bsum(b, red);
+  if (threadIdx.x == 0) {
+    const double g2 = fmax(0.0, 4.0 * (a - b));
+    const int nvir = n - s.nocc;
+    const double gnorm = sqrt(g2) / sqrt((double)(nvir > 0 ? nvir * s.nocc : 1));
+    const double elast = s.scal[0];
+    s.scal[1] = elast;
+    s.scal[0] = etot;
+    s.scal[4] = gnorm;
+    s.e_hist[cycle + 1] = etot;
+    s.ist[1] = cycle + 1;
+    if (fabs(etot - elast) < s.conv_tol && gnorm < sqrt(s.conv_tol)) {
+      s.ist[0] = 1;
+      s.ist[4] = 1;
+    } else if (cycle + 1 >= s.max_cycle) {
+      s.ist[0] = 1;  // out of cycles: frozen, not converged (a batch runs to its longest member)
+    }
+  }
+}
+
 // batched generalized eigh F C = S C e, one workgroup per matrix (scratch: 8 n^2 doubles each)
 __global__ __launch_bounds__(NT_EIG) void k_gen_eigh(int n, const double* F, const double* Sm, double* mo, double* C,
                                                      double* scratch) {
@@ -2196,7 +2407,52 @@ constexpr int NT_ORTH = 256;
 __global__ __launch_bounds__(NT_ORTH) void k_scf_orthogonaliser(const Scf3* __restrict__ ss) {
   __shared__ qexeig::Smem sh;
   const Scf3 s = ss[blockIdx.x];
+  if (fp32_grid(s)) return;
   qexeig::by_size(s.n, [&](auto nc) { qexeig::inverse_cholesky<decltype(nc)::value>(s.n, s.S, s.X, sh); });
+}
+
+// Cholesky S = L L^T (in place, lower), then X = L^-T (upper): C = X V solves F C = S C e.
+__device__ void orthogonaliser(int n, const double* S, double* L, double* X) {
+  const int NT = blockDim.x;
+  for (int t = threadIdx.x; t < n * n; t += NT) L[t] = S[t];
+  __syncthreads();
+  for (int k = 0; k < n; ++k) {
+    if (threadIdx.x == 0) L[k * n + k] = sqrt(L[k * n + k]);
+    __syncthreads();
+    const double dkk = L[k * n + k];
+    for (int i = k + 1 + threadIdx.x; i < n; i += NT) L[i * n + k] /= dkk;
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < (n - k - 1) * (n - k - 1); idx += NT) {
+      const int i = k + 1 + idx / (n - k - 1), j = k + 1 + idx % (n - k - 1);
+      if (j <= i) L[i * n + j] -= L[i * n + k] * L[j * n + k];
+    }
+    __syncthreads();
+  }
+  for (int t = threadIdx.x; t < n * n; t += NT) {
+    const int i = t / n, j = t % n;
+    if (j > i) L[t] = 0.0;
+  }
+  __syncthreads();
+  // Linv (lower) column by column: Linv[:, c] solves L x = e_c; X = Linv^T
+  for (int c = threadIdx.x; c < n; c += NT) {
+    for (int i = 0; i < n; ++i) {
+      double s = i == c ? 1.0 : 0.0;
+      for (int k = c; k < i; ++k) s -= L[i * n + k] * X[c * n + k];  // X row c holds Linv[:, c]
+      X[c * n + i] = i < c ? 0.0 : s / L[i * n + i];
+    }
+  }
+  __syncthreads();
+}
+// the FP32 grid path's: LDS copies (2 n^2 doubles of dynamic LDS), X written out
+__global__ __launch_bounds__(NT_SCF) void k_scf_orthogonaliser_lds(const Scf3* __restrict__ ss) {
+  extern __shared__ __attribute__((aligned(16))) double sm[];
+  const Scf3 s = ss[blockIdx.x];
+  if (!fp32_grid(s)) return;
+  const int nn = s.n * s.n;
+  double* Ls = sm;
+  double* Xs = sm + nn;
+  orthogonaliser(s.n, s.S, Ls, Xs);
+  for (int t = threadIdx.x; t < nn; t += NT_SCF) s.X[t] = Xs[t];
 }
 
 // fill e_hist beyond the last cycle with the final energy (frozen state repeats); status out
@@ -2347,7 +2603,7 @@ __global__ __launch_bounds__(256) void k_coulomb_jsum_b(const Scf3* __restrict__
 }
 
 struct Lay3 {
-  size_t Fd, D, J, K, Vxc, vpart, spart, rho, tmp2, diisF, diisE, diisB, scal, ist;
+  size_t F, Fd, D, Cp, J, K, Vxc, vpart, spart, rho, tmp1, tmp2, diisF, diisE, diisB, scal, ist;
   size_t zpart, z1, dz1, wv, ex, eigf, jpart, total;
 };
 
@@ -2363,8 +2619,10 @@ Lay3 layout3(int n, long ng, int space, int h1 = 0) {
     off = al(off + b);
     return o;
   };
+  L.F = take(nn);
   L.Fd = take(nn);
   L.D = take(nn);
+  L.Cp = take(nn);
   L.J = take(nn);
   L.K = take(nn);
   L.Vxc = take(nn);
@@ -2372,6 +2630,7 @@ Lay3 layout3(int n, long ng, int space, int h1 = 0) {
   L.vpart = take(v64 > v32 ? v64 : v32);
   L.spart = take((size_t)nchunk * 16);
   L.rho = take((size_t)ng * 8);
+  L.tmp1 = take(nn);
   L.tmp2 = take(nn);
   L.diisF = take((size_t)space * nn);
   L.diisE = take((size_t)space * nn);
@@ -3337,7 +3596,10 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     s.x32blk = x32_blocks(ng);
     s.X = (double*)(w + L.total);
     s.status_out = outs[b].status;
+    s.F = (double*)(w + L.F);
     s.Fd = (double*)(w + L.Fd);
+    s.Cp = (double*)(w + L.Cp);
+    s.tmp1 = (double*)(w + L.tmp1);
     s.D = outs[b].dm;
     s.C = outs[b].mo_coeff;
     s.mo = outs[b].mo_energy;
@@ -3403,9 +3665,12 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
   if (off > need) return fail3(QEX_E_WORKSPACE, "internal layout exceeds workspace");
   const size_t lds_eigh = eigh_lds(nmax);
   constexpr size_t static_lds = sizeof(qexeig::Smem) + sizeof(double) * QEX3D_MAX_DIIS * (NW_EIG + 1) + 64;
+  static_assert(sizeof(qexeig_lds::Smem) <= static_lds, "LDS of the eigensolvers");
   if (lds_eigh + static_lds > 160 * 1024) return fail3(QEX_E_UNSUPPORTED, "nao too large for the LDS eigensolver");
-  if (lds_eigh > 64 * 1024)
+  if (lds_eigh > 64 * 1024) {
     (void)hipFuncSetAttribute((const void*)k_scf_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_eigh);
+    (void)hipFuncSetAttribute((const void*)k_scf_eigh, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_eigh);
+  }
   if (lds_nnl > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)k_nn_local_b, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_nnl);
   for (int b0 = 0; b0 < B; b0 += PUT_N) {
@@ -3468,23 +3733,55 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
     qexprof::Scope ps_(kind, st);
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(NT), 0, st, dss, args...);
   };
+  // one cycle's step of the molecules whose grid work is FP64, and of those on the FP32 grid path
+  const bool any_fp64 = any_grid || any_rhf;
   auto step = [&](int kind, int ecycle, int fcycle, int full) {
+    if (!any_fp64) return;
     qexprof::Scope ps_(kind, st);
     hipLaunchKernelGGL(k_scf_step, dim3(nb), dim3(NT_EIG), lds_eigh, st, dss, ecycle, fcycle, full);
+  };
+  auto fock32 = [&](int cycle) {
+    if (!any_x32) return;
+    qexprof::Scope ps_(qexprof::K_FOCK, st);
+    hipLaunchKernelGGL(k_scf_fock, dim3(nb), dim3(NT_SCF), 0, st, dss, cycle);
+  };
+  auto eigh32 = [&](int full) {
+    if (!any_x32) return;
+    qexprof::Scope ps_(qexprof::K_EIGH, st);
+    hipLaunchKernelGGL(k_scf_eigh, dim3(nb), dim3(NT_SCF), lds_eigh, st, dss, full);
+  };
+  auto energy32 = [&](int cycle) {
+    if (!any_x32) return;
+    qexprof::Scope ps_(qexprof::K_ENERGY, st);
+    hipLaunchKernelGGL(k_scf_energy, dim3(nb), dim3(NT_SCF), 0, st, dss, cycle);
   };
   constexpr int NONE = -2;
   // core-Hamiltonian guess: F = H (k_scf_init zeroes J, K, Vxc and D with a kernel, not a memset)
   per_mol(qexprof::K_OTHER, k_scf_init);
-  {
+  if (any_fp64) {
     qexprof::Scope ps_(qexprof::K_OTHER, st);
     hipLaunchKernelGGL(k_scf_orthogonaliser, dim3(nb), dim3(NT_ORTH), 0, st, dss);
   }
+  if (any_x32) {
+    qexprof::Scope ps_(qexprof::K_OTHER, st);
+    const size_t lds_o = (size_t)2 * nmax * nmax * 8;
+    if (lds_o > 64 * 1024)
+      (void)hipFuncSetAttribute((const void*)k_scf_orthogonaliser_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds_o);
+    hipLaunchKernelGGL(k_scf_orthogonaliser_lds, dim3(nb), dim3(NT_SCF), lds_o, st, dss);
+  }
   step(qexprof::K_EIGH, NONE, -1, 0);
+  fock32(-1);
+  eigh32(0);
   veff();
+  energy32(-1);
   int done = -1;  // the cycle whose energy the next step evaluates
   for (int c = 0; c < max_cycle; ++c) {
     step(qexprof::K_EIGH, done, c, 0);
+    fock32(c);
+    eigh32(0);
     veff();
+    energy32(c);
     done = c;
     if (sync_every > 0 && (c + 1) % sync_every == 0 && c + 1 < max_cycle) {
       // optional host check: stop enqueueing cycles once every molecule is frozen
@@ -3500,6 +3797,7 @@ static int scf_run(int B, const qex3d_scf_problem* ps, const qex3d_scf_inputs* i
   }
   if (done != NONE) step(qexprof::K_ENERGY, done, NONE, 0);
   step(qexprof::K_EIGH, NONE, NONE, 1);  // all orbitals and orbital energies of the final Fock matrix
+  eigh32(1);
   per_mol(qexprof::K_OTHER, k_scf_finish);
   return launch_status(name);
 }

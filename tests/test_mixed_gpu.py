@@ -145,3 +145,23 @@ def test_fp32_grid_argument_checks(qtd):
     mf = _solver(qtd, mol, "fp16")
     with pytest.raises(ValueError, match="precision"):
         mf.kernel()
+
+
+def test_fp32_grid_chains_keep_their_density_matrices(qtd):
+    """Chains whose FP32-grid result depends on the last bits of the orbitals: V's FP32 sums multiply a rounding
+    change of 1e-14 to several 1e-9 of the density matrix.  The path's order of operations is fixed,
+    so its results are too: 1e-9 relative (2-norm), the bound of an FP64 result."""
+    import sys
+    sys.path.insert(0, GOLDEN)
+    try:
+        import make_fp32_grid_reference as ref
+    finally:
+        sys.path.remove(GOLDEN)
+    g = np.load(os.path.join(GOLDEN, "fp32_grid_chains.npz"))
+    print("fp32_grid: 5 displaced H16 chains", flush=True)
+    e, diag = ref.solve(qtd, g["z"], g["exps"], g["coefs"])
+    for k in range(len(e)):
+        d = np.linalg.norm(diag[k] - g["dm_diag"][k]) / np.linalg.norm(g["dm_diag"][k])
+        print(f"  chain {k}: |dE| {abs(e[k] - g['e_tot'][k]):.1e}, dm diagonal {d:.1e}", flush=True)
+        assert d <= 1e-9
+        assert abs(e[k] - g["e_tot"][k]) <= 1e-9 * abs(g["e_tot"][k])
