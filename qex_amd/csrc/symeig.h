@@ -215,8 +215,8 @@ __device__ __forceinline__ double ldl_solve(const double* d, const double* e, in
   }
   // row h, in both lanes (a side without rows contributes l = 0)
   const double l = ep * qi, el = ep * l, ly = l * y;
+  const double bh = FIRST ? start_entry(col, h) : scale * Y[h * S + col];  // (read before the exchange: one lane then writes it)
   const double elo = dpp_f64<0xB1>(el), lyo = dpp_f64<0xB1>(ly);
-  const double bh = FIRST ? start_entry(col, h) : scale * Y[h * S + col];
   const double qh = FIRST ? fmin(fmax(rcp_nr((d[h] - lam) - (bot ? elo + el : el + elo)), -rmax), rmax) : Dm[h * S + col];
   double x = (bh - (bot ? lyo + ly : ly + lyo)) * qh;
   double n0 = bot ? 0.0 : x * x;
@@ -259,6 +259,12 @@ __device__ __forceinline__ double rsqrt_nr(double d) {
   return fma(y, fma(-0.5 * d * y, y, 0.5), y);
 }
 
+// exponent of the power of two above |x| (0 for 0, infinities and NaN), where 2^-exponent is a normal number
+__device__ __forceinline__ int exponent(double x) {
+  const int ex = x > 0.0 ? __builtin_amdgcn_frexp_exp(x) : 0;
+  return min(max(ex, -1000), 1000);
+}
+
 // Householder tridiagonalisation of A (n x n in LDS, row stride S).  NC >= ceil(n / 8).
 // Thread (r, c) = (tid / 8, tid % 8) of 512 holds A[r + 64 i][c + 8 j] in registers: row sums cross 8
 // lanes (three DPP steps), and two waves per SIMD fill each other's dependency stalls (four waves of
@@ -267,8 +273,12 @@ __device__ __forceinline__ double rsqrt_nr(double d) {
 // and column q of A as it still is go to LDS together, and after the barrier every thread forms its part
 // of the updated column q, the next x, itself.  Row k of V (stride 8 NC, zero padded, over A's own LDS)
 // receives v_k; sh.d, sh.e, sh.tau the rest.
+// A is scaled by a power of two to a largest element of 1/2 .. 1, and a column whose squared norm below the subdiagonal is
+// under TAIL is taken as reduced: with both, the squares and tau = 2 / |v|^2 neither overflow nor underflow,
+// whatever A's norm and however weakly its blocks are coupled.  Returns the exponent: T is that of A / 2^ex.
+constexpr double TAIL = 1e-280;
 template <int NC>
-__device__ __forceinline__ void tridiagonalise(int n, double* A, int S, Smem& sh) {
+__device__ __forceinline__ int tridiagonalise(int n, double* A, int S, Smem& sh) {
   constexpr int NR = (NC + 7) / 8, SP = 8 * NC;
   const int tid = threadIdx.x, r = tid >> 3, c = tid & 7;
   double a[NR][NC];
@@ -291,8 +301,28 @@ __device__ __forceinline__ void tridiagonalise(int n, double* A, int S, Smem& sh
     const int row = r + 64 * i;
     xr[i] = row >= 1 && row < n ? A[row * S] : 0.0;
   }
-  if (tid == 0) sh.d[0] = a[0][0];
+  double amax = 0.0;
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) amax = fmax(amax, fabs(a[i][j]));
+  amax = wave_max(amax);
+  if ((tid & 63) == 0) sh.nv[tid >> 6] = amax;
   __syncthreads();  // A is in registers; its LDS takes V
+#pragma unroll
+  for (int k = 0; k < NT_MIN / 64; ++k) amax = fmax(amax, sh.nv[k]);
+  const int ex = exponent(amax);
+  const double scale = ldexp(1.0, -ex);
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    xr[i] *= scale;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) a[i][j] *= scale;
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j) xc[j] *= scale;
+  x0 *= scale;
+  if (tid == 0) sh.d[0] = a[0][0];
   static_for<0, NC>([&](auto block) {
     constexpr int jb = decltype(block)::value, ib = jb / 8;
 #pragma unroll 1
@@ -311,7 +341,7 @@ __device__ __forceinline__ void tridiagonalise(int n, double* A, int S, Smem& sh
         for (int j = jb + 1; j < NC; ++j) tail = fma(xc[j], xc[j], tail);
       }
       tail = group8_sum(tail);
-      const bool skip = !(tail > 0.0);
+      const bool skip = !(tail > TAIL);
       const double s2 = fma(x0, x0, tail), nx = s2 * rsqrt_nr(s2);
       const double alpha = x0 >= 0.0 ? -nx : nx;
       const double v0 = skip ? 0.0 : x0 - alpha;
@@ -382,6 +412,7 @@ __device__ __forceinline__ void tridiagonalise(int n, double* A, int S, Smem& sh
     for (int j = 0; j < NC; ++j)
       if (r + 64 * i == n - 1 && c + 8 * j == n - 1) sh.d[n - 1] = a[i][j];
   __syncthreads();
+  return ex;
 }
 
 // X = L^-T (upper triangle, row-major n x n) of the Cholesky factorisation S = L L^T, both in registers: thread
@@ -556,23 +587,23 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
     return;
   }
   // ---- 1. tridiagonalisation ----
+  int ex = 0;  // T and the eigenvalues below are those of A / 2^ex
   by_size(n, [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
-    tridiagonalise<NC>(n, A, S, sh);
+    ex = tridiagonalise<NC>(n, A, S, sh);
     // V to scratch: the pivots of phase 4 take its place
     for (int idx = tid; idx < (n - 2) * 8 * NC; idx += nt) f[idx] = A[idx];
   });
   // ---- 2. norm, scaling, unreduced blocks ----
-  double scale, unscale;  // powers of two
+  double scale;  // a power of two
   {
     double nrm = 0.0;  // every wave by itself
     for (int i = lane; i < n; i += 64)
       nrm = fmax(nrm, fabs(sh.d[i]) + (i > 0 ? fabs(sh.e[i - 1]) : 0.0) + (i < n - 1 ? fabs(sh.e[i]) : 0.0));
     nrm = wave_max(nrm);
-    int ex = nrm > 0.0 ? __builtin_amdgcn_frexp_exp(nrm) - 1 : 0;
-    ex = ex < -1000 ? -1000 : ex > 1000 ? 1000 : ex;
-    scale = ldexp(1.0, -ex);
-    unscale = ldexp(1.0, ex);
+    const int et = nrm > 0.0 ? exponent(nrm) - 1 : 0;
+    scale = ldexp(1.0, -et);
+    ex += et;
   }
   __syncthreads();
   if (wv < 2) {
@@ -735,7 +766,7 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
     num = group4_sum(num);
     den = group4_sum(den);
     if (c < n && q4 == 0) {
-      sh.rq[c] = (den > 0.0 ? num / den : sh.lam[c]) * unscale;  // no vector: the multisection value
+      sh.rq[c] = ldexp(den > 0.0 ? num / den : sh.lam[c], ex);  // no vector: the multisection value
       sh.nv[c] = den > 0.0 ? 1.0 / sqrt(den) : 0.0;
     }
   }

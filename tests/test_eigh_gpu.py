@@ -149,3 +149,33 @@ def test_register_patch_edges(geigh, n):
         w, v = geigh(As, np.broadcast_to(np.eye(n), As.shape).copy())
         for k in range(len(As)):
             _check(w[k].cpu().numpy() / f, v[k].cpu().numpy(), As[k] / f, np.eye(n))
+
+
+def test_extreme_norms_and_couplings(geigh):
+    """Matrices whose reduction meets squares outside the range of a double: rank-deficient with equal entries
+    (the reflectors' columns shrink by 1e-16 each), blocks coupled by 1e-140 .. 1e-200, and norms 1e-200 and 1e200.
+    Backward stability of n reflectors: 40 n eps."""
+    eps = np.finfo(float).eps
+    for n in (15, 18, 24, 39, 64, 72, 96):
+        ones = np.full((n, n), 0.3)
+        bip = np.zeros((n, n))
+        bip[: n // 2, n // 2:] = 1.0
+        bip += bip.T
+        rng = np.random.default_rng(n)
+        M = rng.standard_normal((n, n))
+        As, units = [ones, bip, M + M.T, M + M.T], [1.0, 1.0, 2.0**-665, 2.0**665]
+        for c in (1e-140, 1e-150, 1e-156, 1e-160, 1e-200):
+            B = np.tril(M).copy()
+            B[n // 2:, : n // 2] *= c
+            As.append(B + np.tril(B, -1).T)
+            units.append(1.0)
+        A = np.stack([a * u for a, u in zip(As, units)])
+        w, v = geigh(A, np.broadcast_to(np.eye(n), A.shape).copy())
+        for k, (a, u) in enumerate(zip(As, units)):
+            wk, Z = w[k].cpu().numpy() / u, v[k].cpu().numpy()
+            ref = np.linalg.eigvalsh(a)
+            norm = np.abs(ref).max()
+            tol = max(40 * n * eps, 1e-12) if k > 1 else 40 * n * eps  # (a random spectrum: eps over its smallest gap)
+            assert np.abs(wk - ref).max() <= tol * norm, (n, k)
+            assert np.abs(a @ Z - Z * wk).max() <= tol * norm, (n, k)
+            assert np.abs(Z.T @ Z - np.eye(n)).max() <= tol, (n, k)
