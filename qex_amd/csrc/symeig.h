@@ -22,6 +22,7 @@
 // back-transformation stays in four lanes' registers from the first reflector to the last.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <math.h>
 
 namespace qexeig {
 
@@ -773,8 +774,11 @@ __device__ __forceinline__ void symeig(int n, double* A, double* Z, int S, doubl
   __syncthreads();
   // ---- 5. sort ascending (rank; ties by slot), back-transform ----
   for (int i = tid; i < n; i += nt) {
+    // (a NaN ranks with the infinities: perm is a permutation whatever the input holds)
+    auto key = [&](int j) { return sh.rq[j] == sh.rq[j] ? sh.rq[j] : HUGE_VAL; };
+    const double ki = key(i);
     int r = 0;
-    for (int j = 0; j < n; ++j) r += (sh.rq[j] < sh.rq[i]) || (sh.rq[j] == sh.rq[i] && j < i);
+    for (int j = 0; j < n; ++j) r += key(j) < ki || (key(j) == ki && j < i);
     sh.perm[r] = i;
     w[r] = sh.rq[i];
   }

@@ -189,6 +189,7 @@ inline unsigned __builtin_amdgcn_alignbit(unsigned hi, unsigned lo, unsigned s) 
 inline int __double2hiint(double x) { return (int)(lanes::bits(x) >> 32); }
 inline int __double2loint(double x) { return (int)lanes::bits(x); }
 inline double __hiloint2double(int h, int l) { return lanes::value(((uint64_t)(uint32_t)h << 32) | (uint32_t)l); }
+inline long long __double_as_longlong(double x) { return (long long)lanes::bits(x); }
 inline int __popc(unsigned x) { return __builtin_popcount(x); }
 inline int __popcll(unsigned long long x) { return __builtin_popcountll(x); }
 inline int __ffsll(long long x) { return __builtin_ffsll(x); }

@@ -32,17 +32,17 @@ def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
-def _eigh(lib, A, nvec=1 << 30):
+def _eigh(lib, A, nvec=1 << 30, solver="host_symeig"):
     A = np.ascontiguousarray(A, dtype=np.float64)
     n = len(A)
-    w, Z = np.zeros(n), np.zeros((n, n))
-    lib.host_symeig(n, _p(A), nvec, _p(w), _p(Z))
-    return w, Z
+    w, Z, perm = np.zeros(n), np.zeros((n, n)), np.zeros(n, dtype=np.int32)
+    getattr(lib, solver)(n, _p(A), nvec, _p(w), _p(Z), _p(perm))
+    return w, Z, perm
 
 
 def _check_eigh(lib, A, tol, unit=1.0):
     """Eigenvalues, residual and orthogonality within tol of the norm; A given in units of `unit`."""
-    w, Z = _eigh(lib, A * unit)
+    w, Z, _ = _eigh(lib, A * unit)
     ref = np.linalg.eigvalsh(A)
     norm = max(np.abs(ref).max(), 1e-300)
     w = w / unit
@@ -96,3 +96,18 @@ def test_symeig_norms(lib, unit):
     """An ordinary matrix at the ends of the range of a double."""
     A = np.random.default_rng(8).standard_normal((20, 20))
     _check_eigh(lib, A + A.T, 1e-12, unit)
+
+
+@pytest.mark.parametrize("solver", ["host_symeig", "host_symeig_lds"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_symeig_slots_stay_a_permutation(lib, solver, value):
+    """A matrix with a NaN or infinite entry: no eigenvalues, but the columns' order still names every slot
+    once (a slot left out would be read from whatever the LDS held).  The order alone is looked at: symeig_lds.h's
+    numbers rely on a wave's lanes reading a row together before one of them changes it, which fibers do not."""
+    rng = np.random.default_rng(2)
+    for n, at in ((5, (1, 1)), (12, (7, 2)), (24, (0, 0))):
+        A = rng.standard_normal((n, n))
+        A = A + A.T
+        A[at] = A[at[::-1]] = value
+        perm = _eigh(lib, A, solver=solver)[2]
+        assert sorted(perm) == list(range(n))
