@@ -73,9 +73,18 @@ __device__ __forceinline__ Mat2 mul(Mat2 a, Mat2 b) {
   return {fma(a.xx, b.xx, a.xy * b.yx), fma(a.xx, b.xy, a.xy * b.yy), fma(a.yx, b.xx, a.yy * b.yx), fma(a.yx, b.xy, a.yy * b.yy)};
 }
 
+// What the lanes of a wave wrote to LDS before, all of them read after: the LDS executes one wave's accesses in
+// issue order, so only the compiler must be kept from moving them across this point.
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Every lane of the wave calls this.  a, y: LDS, N doubles each; F: LDS, wave_doubles(N) doubles.
 // SOLVE: y <- (A - sigma)^-1 y.  Returns the number of eigenvalues of A below sigma (the same in every lane).
-// The LDS contents written by the wave itself need no barrier before and after.
+// Each lane reads and writes only its own rows of y and F; lanes that go on to read others' rows call
+// wave_lds_order first.
 template <bool SOLVE>
 __device__ __forceinline__ int wave_solve(const double* a, double* y, int N, double b, double c, double sigma, double* F) {
   const int p = threadIdx.x & 63, m = wave_rows(N), k = m - 2, row0 = p * m;

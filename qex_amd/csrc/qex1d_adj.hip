@@ -784,81 +784,6 @@ __global__ void k_adj_scales(Adj a, int k, double* cs, double* ones) {
   ones[s] = 1.0;
 }
 
-// Fallback of k_adj_eig, one thread: y <- (H - ej)^-1 y by Gaussian elimination with partial pivoting (bandwidth 2,
-// fill to 4).  The three active rows (columns i .. i + 4) are in registers; each finished row of U (5 entries)
-// goes to R and its right-hand side to y, then the back substitution.  Pivots below tiny become +-tiny.
-__device__ __attribute__((noinline)) void pivoted_solve(const double* hd, double* y, double* R, int N, double Tb, double Tc,
-                                                        double ej, double tiny) {
-  auto band = [&](int row, int col) -> double {  // entry of H - eps_j (zero outside the matrix)
-    if (row >= N || col < 0 || col >= N) return 0.0;
-    const int d = col - row;
-    return d == 0 ? hd[row] - ej : (d == 1 || d == -1) ? Tb : (d == 2 || d == -2) ? Tc : 0.0;
-  };
-  double r0[5], r1[5], r2[5];
-  for (int c = 0; c < 5; ++c) {
-    r0[c] = band(0, c);
-    r1[c] = band(1, c);
-    r2[c] = band(2, c);
-  }
-  double y0 = y[0], y1 = N > 1 ? y[1] : 0.0, y2 = N > 2 ? y[2] : 0.0;
-  for (int i = 0; i < N; ++i) {
-    // pivot among the (existing) rows i, i+1, i+2 in column i
-    int pr = 0;
-    double best = fabs(r0[0]);
-    if (i + 1 < N && fabs(r1[0]) > best) {
-      best = fabs(r1[0]);
-      pr = 1;
-    }
-    if (i + 2 < N && fabs(r2[0]) > best) pr = 2;
-    if (pr == 1) {
-      for (int c = 0; c < 5; ++c) {
-        const double t1 = r0[c];
-        r0[c] = r1[c];
-        r1[c] = t1;
-      }
-      const double ty = y0;
-      y0 = y1;
-      y1 = ty;
-    } else if (pr == 2) {
-      for (int c = 0; c < 5; ++c) {
-        const double t1 = r0[c];
-        r0[c] = r2[c];
-        r2[c] = t1;
-      }
-      const double ty = y0;
-      y0 = y2;
-      y2 = ty;
-    }
-    if (fabs(r0[0]) < tiny) r0[0] = r0[0] < 0.0 ? -tiny : tiny;
-    const double ip = 1.0 / r0[0];
-    const double l1 = r1[0] * ip, l2 = r2[0] * ip;
-    for (int c = 1; c < 5; ++c) {
-      r1[c] = fma(-l1, r0[c], r1[c]);
-      r2[c] = fma(-l2, r0[c], r2[c]);
-    }
-    y1 = fma(-l1, y0, y1);
-    y2 = fma(-l2, y0, y2);
-    for (int c = 0; c < 5; ++c) R[(size_t)i * 5 + c] = r0[c];
-    y[i] = y0;
-    // advance: rows i+1, i+2 shift one column left; row i+3 enters
-    for (int c = 0; c < 4; ++c) {
-      r0[c] = r1[c + 1];
-      r1[c] = r2[c + 1];
-    }
-    r0[4] = 0.0;
-    r1[4] = 0.0;
-    for (int c = 0; c < 5; ++c) r2[c] = band(i + 3, i + 1 + c);
-    y0 = y1;
-    y1 = y2;
-    y2 = i + 3 < N ? y[i + 3] : 0.0;
-  }
-  for (int i = N - 1; i >= 0; --i) {
-    double v = y[i];
-    for (int c = 1; c < 5 && i + c < N; ++c) v = fma(-R[(size_t)i * 5 + c], y[i + c], v);
-    y[i] = v / R[(size_t)i * 5];
-  }
-}
-
 // eigen adjoint, one workgroup per system.
 //
 // Bound by the dependent chain of the banded solves.  One thread eliminating with partial pivoting takes 0.7 us a
@@ -960,7 +885,7 @@ __global__ __launch_bounds__(NT) void k_adj_eig(Adj a, int k, double Td, double 
       // (the solution's component along psi_j is projected out)
       for (int t = threadIdx.x; t < N; t += NT) x[t] = y[t];
       __syncthreads();
-      if (threadIdx.x == 0) pivoted_solve(hd, x, F, N, Tb, Tc, ej, rounding);
+      if (threadIdx.x == 0) qexband::pivoted_solve(hd, x, F, N, Tb, Tc, ej, rounding);
     }
     __syncthreads();
     // x <- Q x; y_j = -x - sum over occupied b with occ_b != occ_j of psi_b (psi_b . r) / (eps_b - eps_j)

@@ -3,46 +3,28 @@ workgroup a fiber, exchanges and barriers as on the device, hardware reciprocals
 LAPACK (CPU only)."""
 
 import ctypes
-import os
-import shutil
-import subprocess
 
 import numpy as np
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EPS = np.finfo(float).eps
-
-
-@pytest.fixture(scope="module")
-def lib(tmp_path_factory):
-    gxx = shutil.which("g++")
-    if not gxx:
-        pytest.skip("g++ not available")
-    so = str(tmp_path_factory.mktemp("lanes") / "lanes.so")
-    host = os.path.join(ROOT, "tests", "host")
-    subprocess.run([gxx, "-O2", "-march=native", "-ffp-contract=off", "-std=c++17", "-w", "-shared", "-fPIC",
-                    "-I", os.path.join(host, "lanes"),
-                    "-I", os.path.join(ROOT, "qex_amd", "csrc"), os.path.join(host, "lanes_harness.cpp"), "-o", so],
-                   check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
-    return ctypes.CDLL(so)
 
 
 def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
-def _eigh(lib, A, nvec=1 << 30, solver="host_symeig"):
+def _eigh(lanes_lib, A, nvec=1 << 30, solver="host_symeig"):
     A = np.ascontiguousarray(A, dtype=np.float64)
     n = len(A)
     w, Z, perm = np.zeros(n), np.zeros((n, n)), np.zeros(n, dtype=np.int32)
-    getattr(lib, solver)(n, _p(A), nvec, _p(w), _p(Z), _p(perm))
+    getattr(lanes_lib, solver)(n, _p(A), nvec, _p(w), _p(Z), _p(perm))
     return w, Z, perm
 
 
-def _check_eigh(lib, A, tol, unit=1.0):
+def _check_eigh(lanes_lib, A, tol, unit=1.0):
     """Eigenvalues, residual and orthogonality within tol of the norm; A given in units of `unit`."""
-    w, Z, _ = _eigh(lib, A * unit)
+    w, Z, _ = _eigh(lanes_lib, A * unit)
     ref = np.linalg.eigvalsh(A)
     norm = max(np.abs(ref).max(), 1e-300)
     w = w / unit
@@ -52,16 +34,16 @@ def _check_eigh(lib, A, tol, unit=1.0):
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 16, 17, 33, 64, 65, 96])
-def test_symeig_random(lib, n):
+def test_symeig_random(lanes_lib, n):
     """Sizes at the edges of the register patches and size classes.  The closest pair of such a matrix is
     1e-3 of the norm apart, where two inverse iterations leave eps / 1e-3 = 2e-13; 1e-12 with the sums over n."""
     A = np.random.default_rng(n).standard_normal((n, n))
-    _check_eigh(lib, A + A.T, 1e-12)
+    _check_eigh(lanes_lib, A + A.T, 1e-12)
 
 
 @pytest.mark.parametrize("n", [3, 13, 15, 16, 22, 26, 33, 41])
 @pytest.mark.parametrize("kind", ["ones", "pi", "bipartite"])
-def test_symeig_rank_deficient_with_equal_entries(lib, n, kind):
+def test_symeig_rank_deficient_with_equal_entries(lanes_lib, n, kind):
     """Reduction leaves a block of rounding errors that keeps the symmetry of the matrix, so its columns shrink by
     1e-16 a reflector, through every magnitude where a square or its reciprocal is no normal number.
     Backward stability of n reflectors: 40 n eps."""
@@ -71,11 +53,11 @@ def test_symeig_rank_deficient_with_equal_entries(lib, n, kind):
         A += A.T
     else:
         A = np.full((n, n), 0.3 if kind == "ones" else np.pi)
-    _check_eigh(lib, A, 40 * n * EPS)
+    _check_eigh(lanes_lib, A, 40 * n * EPS)
 
 
 @pytest.mark.parametrize("coupling", [1e-140, 1e-150, 1e-154, 1e-156, 1e-158, 1e-160, 1e-162, 1e-165, 1e-200])
-def test_symeig_weakly_coupled_blocks(lib, coupling):
+def test_symeig_weakly_coupled_blocks(lanes_lib, coupling):
     """Two blocks joined by entries whose squares are near or below the smallest double (well separated
     fragments): the spectrum of the blocks."""
     rng = np.random.default_rng(4)
@@ -83,24 +65,24 @@ def test_symeig_weakly_coupled_blocks(lib, coupling):
     A[:6, :6], A[6:, 6:] = rng.standard_normal((6, 6)), rng.standard_normal((6, 6))
     A[6:, :6] = coupling * rng.standard_normal((6, 6))
     A = np.tril(A) + np.tril(A, -1).T
-    _check_eigh(lib, A, 1e-13)
+    _check_eigh(lanes_lib, A, 1e-13)
     # as the smallest example: two coupled pairs
     B = np.diag([1.0, 2.0, 3.0, 4.0])
     B[0, 1] = B[1, 0] = B[2, 3] = B[3, 2] = 0.3
     B[0, 2] = B[2, 0] = B[1, 3] = B[3, 1] = coupling
-    _check_eigh(lib, B, 40 * 4 * EPS)
+    _check_eigh(lanes_lib, B, 40 * 4 * EPS)
 
 
 @pytest.mark.parametrize("unit", [2.0**-1000, 2.0**-665, 2.0**-530, 2.0**-515, 2.0**-100, 2.0**500, 2.0**515, 2.0**1000])
-def test_symeig_norms(lib, unit):
+def test_symeig_norms(lanes_lib, unit):
     """An ordinary matrix at the ends of the range of a double."""
     A = np.random.default_rng(8).standard_normal((20, 20))
-    _check_eigh(lib, A + A.T, 1e-12, unit)
+    _check_eigh(lanes_lib, A + A.T, 1e-12, unit)
 
 
 @pytest.mark.parametrize("solver", ["host_symeig", "host_symeig_lds"])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
-def test_symeig_slots_stay_a_permutation(lib, solver, value):
+def test_symeig_slots_stay_a_permutation(lanes_lib, solver, value):
     """A matrix with a NaN or infinite entry: no eigenvalues, but the columns' order still names every slot
     once (a slot left out would be read from whatever the LDS held).  The order alone is looked at: symeig_lds.h's
     numbers rely on a wave's lanes reading a row together before one of them changes it, which fibers do not."""
@@ -109,5 +91,5 @@ def test_symeig_slots_stay_a_permutation(lib, solver, value):
         A = rng.standard_normal((n, n))
         A = A + A.T
         A[at] = A[at[::-1]] = value
-        perm = _eigh(lib, A, solver=solver)[2]
+        perm = _eigh(lanes_lib, A, solver=solver)[2]
         assert sorted(perm) == list(range(n))
