@@ -52,15 +52,15 @@ __device__ __forceinline__ void inverse_step(const double* a, double* y, double*
   wave_lds_order();
 }
 
-// The j-th eigenvalue to 1e-12 by Rayleigh-quotient iteration on one wave (all 64 lanes) from the vector in
-// y, until the residual |A y - rho y| is 1e-8 (the quotient's error is its square over the gap).
-//   check: at most 3 solves, the first with y's own quotient as shift; the eigenvalue count just above rho
-//     must then be j + 1.
-//   else: [slo, shi] is known to hold the j-th eigenvalue and no other; the shift is its middle until the
-//     quotient lies inside.
-// false if that does not end with the j-th pair; the caller brackets the eigenvalue further.
-__device__ bool refine_eigenvalue(const double* a, double* y, double* F, int N, double b, double c, double hnorm, int j,
-                                  double slo, double shi, bool check, double* rho_out) {
+// An eigenvalue by Rayleigh-quotient iteration on one wave (all 64 lanes) from the vector in y, until the residual
+// |A y - rho y| is 1e-8; the quotient's error is the residual's square over the gap to the next eigenvalue.
+//   near: at most 3 solves, the first with y's own quotient as shift.  Of a pair closer than 2e-8 any mixture has
+//     such a residual, and another eigenvalue may be nearer: confirm_side has to say that it is the j-th.
+//   else: [slo, shi] is known to hold the j-th eigenvalue and no other, with the neighbours well away; the shift
+//     is its middle until the quotient lies inside.
+// false if that does not end; the caller brackets the eigenvalue further.
+__device__ bool refine_eigenvalue(const double* a, double* y, double* F, int N, double b, double c, double slo, double shi,
+                                  bool near, double* rho_out) {
   const int m = wave_rows(N), r0 = (threadIdx.x & 63) * m, r1 = min(N, r0 + m);
   auto hy = [&](int i) {
     double v = a[i] * y[i];
@@ -75,8 +75,8 @@ __device__ bool refine_eigenvalue(const double* a, double* y, double* F, int N, 
     for (int i = r0; i < r1; ++i) q = fma(y[i], hy(i), q);
     return wave_sum_same(q);
   };
-  double sigma = check ? quotient() : 0.5 * (slo + shi);
-  for (int it = 0; it < (check ? 3 : 6); ++it) {
+  double sigma = near ? quotient() : 0.5 * (slo + shi);
+  for (int it = 0; it < (near ? 3 : 6); ++it) {
     inverse_step(a, y, F, N, b, c, sigma);
     const double rho = quotient();
     if (rho >= slo && rho <= shi) {
@@ -87,13 +87,20 @@ __device__ bool refine_eigenvalue(const double* a, double* y, double* F, int N, 
       }
       if (wave_sum_same(r2) <= 1e-16 * fmax(1.0, rho * rho)) {
         *rho_out = rho;
-        const double tau = 1e-9 * fmax(1.0, fabs(rho)) + 64.0 * EPS * hnorm;
-        return !check || wave_solve<false>(a, y, N, b, c, rho + tau, F) == j + 1;
+        return true;
       }
       sigma = rho;
     }
   }
   return false;
+}
+
+// One side of "the j-th eigenvalue lies within tau of rho", by the number of eigenvalues below rho + tau (above)
+// or rho - tau; a wave.  tau is the quotient's error at a gap of 1e-5 and the rounding of a count.
+__device__ __forceinline__ bool confirm_side(const double* a, double* F, int N, double b, double c, double hnorm, int j,
+                                             double rho, bool above) {
+  const double tau = 1e-11 * fmax(1.0, fabs(rho)) + 64.0 * EPS * hnorm;
+  return wave_solve<false>(a, nullptr, N, b, c, above ? rho + tau : rho - tau, F) == j + (above ? 1 : 0);
 }
 
 // Multisection bracket of the j-th eigenvalue: NS shifts per round, both ends included; first = index of the

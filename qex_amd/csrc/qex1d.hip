@@ -41,6 +41,7 @@ int g_pool_n = 0, g_pool_used = 0;
 namespace {
 
 using qexband::Bracket;
+using qexband::confirm_side;
 using qexband::dpp_f64;
 using qexband::read_lane;
 using qexband::refine_eigenvalue;
@@ -1017,16 +1018,17 @@ __device__ __forceinline__ double start_value(int i, int j) {
 // One eigenpair per workgroup: the multisection bracket of the eigenvalue down to 1e-9 relative (4 to 6 rounds of
 // 128 counts), then two inverse-iteration solves at its middle.  A round of counts is 11 us at N = 513, so:
 //   - the eigenvalue itself is found first.  Warm and moved by less than 1e-4 in the last SCF iteration: one wave
-//     refines the previous orbital (band_wave.h, 5 us a solve) and confirms its index with one count.  Else one
-//     or two rounds over 2 Ha about the last value (cold: two or three from the bottom of the spectrum) leave
+//     refines the previous orbital (eigen1d.h, 5 us a solve), and two waves confirm its index by a count on each
+//     side of the value: a mixture of a pair closer than the refinement resolves is not taken.  Else one or two rounds over 2 Ha about the last value (cold: two or three from the bottom of the spectrum) leave
 //     a bracket of ISOLATED at most whose neighbours' are APART intervals away, so that the solves at
 //     its middle converge at once, and the refinement runs inside it;
 //   - the rounds then follow without counting: a shift has more than j eigenvalues below it exactly if it lies
 //     above the j-th.  Where the refinement does not confirm the pair, they count as before.
 //   - The two solves: twisted_inverse_iteration.
-// The bracket, its middle and the solves are those of counting every round, so the orbitals are the same to the
-// bit; solving in parallel there too is as fast and as accurate, but moves the orbitals of nearly degenerate
-// pairs by their own rounding, 1e-13 over the gap.
+// The bracket, its middle and the solves are those of counting every round, unless a shift falls within the
+// refinement's error (1e-11) of the eigenvalue: the densities of 589 .. 597 of 601 systems are the same bits as with
+// every round counted, the others' within 1.3e-12.  Solving in parallel there too is as fast and as accurate, but
+// moves the orbitals of nearly degenerate pairs by their own rounding, 1e-13 over the gap.
 // Bound by the dependent chain of one pair: 55..75 us, of which the two solves 30.  A launch at N = 513: one system
 // 69 us (91 with every round counted and the four phases of the solves in sequence), 64 systems of up to 5 pairs
 // 99 us (120); 601 systems at N = 401 309 us (364).
@@ -1048,7 +1050,7 @@ __global__ __launch_bounds__(NT) void k_eigen(EigArgs e) {
   double* red = F + wave_doubles(N);  // 16
   double* ap = red + 16;    // N    the diagonal in the order of side_pos
   __shared__ double sh_rho;
-  __shared__ int sh_first[3][NWAVE], sh_ok;
+  __shared__ int sh_first[3][NWAVE], sh_ok[2];
   const double* pot = e.pot + (size_t)s * N;
   double* v = e.vec + ((size_t)s * e.K + j) * N;
   const int kt = (N - 2) / 2, kb = N - 2 - kt;
@@ -1082,19 +1084,27 @@ __global__ __launch_bounds__(NT) void k_eigen(EigArgs e) {
       br.hi = br.gu;
     }
   }
-  // the eigenvalue by wave 0 (sh_rho), true if found
-  auto refine = [&](double slo, double shi, bool check) {
+  // the eigenvalue by wave 0 (sh_rho), its index by waves 0 and 1 side by side where y alone leads to it; true if found
+  auto refine = [&](double slo, double shi, bool near) {
     __syncthreads();
     if (tid < 64) {
       double rho = 0.0;
-      const bool ok = refine_eigenvalue(a, y, F, N, e.Tb, e.Tc, hnorm, j, slo, shi, check, &rho);
+      const bool ok = refine_eigenvalue(a, y, F, N, e.Tb, e.Tc, slo, shi, near, &rho);
       if (tid == 0) {
-        sh_ok = ok;
+        sh_ok[0] = sh_ok[1] = ok;
         sh_rho = rho;
       }
     }
     __syncthreads();
-    return sh_ok != 0;
+    if (near && sh_ok[0]) {
+      __syncthreads();
+      if (tid < 128) {
+        const bool ok = confirm_side(a, F, N, e.Tb, e.Tc, hnorm, j, sh_rho, tid >= 64);
+        if ((tid & 63) == 0) sh_ok[tid >> 6] = ok;
+      }
+      __syncthreads();
+    }
+    return sh_ok[0] && sh_ok[1];
   };
   // One round of counts: each shift by a pair of lanes, the even lane eliminating the top rows 0..kt-1 and
   // the odd lane the bottom rows N-1..kt+2 (half the recurrence each), joined through the 2x2 block of rows

@@ -69,13 +69,16 @@ void host_pivoted_solve(int N, const double* a, double* y, double b, double c, d
   std::vector<double> R((size_t)5 * N);
   qexband::pivoted_solve(a, y, R.data(), N, b, c, sigma, qexband::EPS * m.hnorm);
 }
-// the j-th eigenvalue from the vector y (qexband::refine_eigenvalue); 1 if found
-int host_refine(int N, const double* a, double* y, double b, double c, int j, double lo, double hi, int check, double* rho) {
+// the j-th eigenvalue from the vector y: refinement and, with near, the index; 1 if found
+int host_refine(int N, const double* a, double* y, double b, double c, int j, double lo, double hi, int near, double* rho) {
   Band m(N, a, b, c);
   int ok = 0;
   lanes::run(64, [&] {
     double r = 0.0;
-    const bool found = qexband::refine_eigenvalue(m.a.data(), y, m.F.data(), N, b, c, m.hnorm, j, lo, hi, check != 0, &r);
+    bool found = qexband::refine_eigenvalue(m.a.data(), y, m.F.data(), N, b, c, lo, hi, near != 0, &r);
+    if (found && near)
+      for (int above = 0; above < 2; ++above)
+        found = qexband::confirm_side(m.a.data(), m.F.data(), N, b, c, m.hnorm, j, r, above) && found;
     if (threadIdx.x == 0) {
       ok = found;
       *rho = r;

@@ -146,3 +146,25 @@ def test_refined_eigenvalues_match_lapack(lanes_lib):
                 assert ok and abs(rho - w[j]) < 1e-11
                 # the same vector asked for as another pair
                 assert not m.refine(y / np.linalg.norm(y), j + 1, w[0] - 1, w[-1] + 1, True)[0]
+
+
+@pytest.mark.parametrize("distance", [7.2, 7.8, 8.4, 9.0])
+def test_mixtures_of_a_close_pair_are_not_refined(lanes_lib, distance):
+    """Two wells whose lowest pair is split by 3e-10 .. 1e-7, and a vector between the two states (an orbital
+    of an earlier iteration): its residual is half the splitting and its quotient lies between the levels, so it
+    must not pass for either of them.  What passes is within 1e-11 of the value and 64 roundings of the operator."""
+    grids = 0.1 * (np.arange(401) - 200)
+    v = -6.0 * (np.exp(-((grids - distance / 2) ** 2)) + np.exp(-((grids + distance / 2) ** 2)))
+    m = Band(lanes_lib, grids, v)
+    w, V = np.linalg.eigh(m.H)
+    split = w[1] - w[0]
+    assert 3e-10 < split < 1e-7
+    tol = 1e-11 * abs(w[0]) + 64 * 2.2e-16 * m.hnorm + 1e-12  # (1e-12: LAPACK's own)
+    for angle in (0.25, 0.15, 0.4):
+        y = np.cos(angle * np.pi) * V[:, 0] + np.sin(angle * np.pi) * V[:, 1]
+        for j in (0, 1):
+            ok, rho, _ = m.refine(y, j, w[0] - 1, w[-1] + 1, True)
+            assert not ok or abs(rho - w[j]) < tol
+    for j in (0, 1):
+        ok, rho, _ = m.refine(V[:, j], j, w[0] - 1, w[-1] + 1, True)
+        assert not ok or abs(rho - w[j]) < tol
