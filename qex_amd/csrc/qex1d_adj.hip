@@ -30,6 +30,7 @@
 #include "band_wave.h"
 #include "prof.h"
 #include "qex.h"
+#include "tiles.h"
 
 namespace {
 
@@ -1104,16 +1105,28 @@ int qex1d_kohn_sham_vjp(const qex1d_problem* p, const qex1d_inputs* in, const qe
   }
   auto mlp = [&](const double* xin, const double* tin, const double* F1, const double* sf, const double* F2) {
     qexprof::Scope ps(qexprof::K_ADJ_MLP, st);
-    const long tiles = ((long)a.B * a.N + (tin ? 15 : 31)) / (tin ? 16 : 32);
-    const dim3 grid((unsigned)(tiles < ADJ_WG ? tiles : ADJ_WG)), block(ANT);
-    if (a.NL == 2 && tin)
-      hipLaunchKernelGGL((k_adj_mlp<2, true>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
-    else if (a.NL == 2)
-      hipLaunchKernelGGL((k_adj_mlp<2, false>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
-    else if (tin)
-      hipLaunchKernelGGL((k_adj_mlp<1, true>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
-    else
-      hipLaunchKernelGGL((k_adj_mlp<1, false>), grid, block, ADJ_MLP_LDS, st, a, xin, tin, F1, sf, F2);
+    qextile::for_launches(a.B, a.N, [&](int s0, int n) {
+      const size_t p0 = (size_t)s0 * a.N;
+      Adj q = a;
+      q.B = n;
+      q.fv += p0;
+      q.fdv += p0;
+      q.xbar += p0 * a.W;
+      const long tiles = ((long)n * a.N + (tin ? 15 : 31)) / (tin ? 16 : 32);
+      const dim3 grid((unsigned)(tiles < ADJ_WG ? tiles : ADJ_WG)), block(ANT);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, ADJ_MLP_LDS, st, q, xin + p0, tin ? tin + p0 : nullptr, F1 + p0, sf + s0,
+                           F2 ? F2 + p0 : nullptr);
+      };
+      if (a.NL == 2 && tin)
+        launch(k_adj_mlp<2, true>);
+      else if (a.NL == 2)
+        launch(k_adj_mlp<2, false>);
+      else if (tin)
+        launch(k_adj_mlp<1, true>);
+      else
+        launch(k_adj_mlp<1, false>);
+    });
   };
   // the global network: one workgroup per system (at most ADJ_WG, each then taking several in turn)
   const unsigned gG = (unsigned)(a.B < ADJ_WG ? a.B : ADJ_WG);

@@ -4,6 +4,7 @@
 #include "eigen1d.h"
 #include "symeig.h"
 #include "symeig_lds.h"
+#include "tiles.h"
 
 namespace {
 
@@ -85,6 +86,18 @@ int host_refine(int N, const double* a, double* y, double b, double c, int j, do
     }
   });
   return ok;
+}
+// the launches of a batch: first system and number of systems of each; returns how many
+int host_launches(int B, int N, int max, int* first, int* n) {
+  int k = 0;
+  qextile::for_launches(B, N, [&](int s0, int m) {
+    if (k < max) {
+      first[k] = s0;
+      n[k] = m;
+    }
+    ++k;
+  });
+  return k;
 }
 // two twisted inverse-iteration solves at sigma from y
 void host_twisted(int N, const double* a, double* y, double b, double c, double sigma) {

@@ -93,3 +93,17 @@ def test_symeig_slots_stay_a_permutation(lanes_lib, solver, value):
         A[at] = A[at[::-1]] = value
         perm = _eigh(lanes_lib, A, solver=solver)[2]
         assert sorted(perm) == list(range(n))
+
+
+@pytest.mark.parametrize("B,N", [(1, 5), (32, 513), (2093062, 513), (2093063, 513), (4186128, 513), (2**31 - 1, 1024)])
+def test_launches_cover_the_batch(lanes_lib, B, N):
+    """The launches of a network adjoint: every system once, in order, and no point number past 2^31 even in the
+    tiles past the end that the last round addresses (256 workgroups of 2 groups of 32 points)."""
+    first, n = np.zeros(4096, dtype=np.int32), np.zeros(4096, dtype=np.int32)
+    k = lanes_lib.host_launches(B, N, len(n), _p(first), _p(n))
+    assert 1 <= k <= len(n)
+    assert k == 1 or B * N > 2**30
+    ends = np.cumsum(n[:k].astype(np.int64))
+    assert ends[-1] == B and first[0] == 0 and (n[:k] > 0).all()
+    assert (first[1:k] == ends[:-1]).all()
+    assert n[:k].max() * N + 2 * 256 * 2 * 32 < 2**31
