@@ -293,6 +293,9 @@ __device__ __forceinline__ double row_sum(double x) {
 // One point per wave with one lane per unit (weights from LDS for every multiply, 0.25 flop a byte) took 255 us for
 // 32 x 513 points of a 17-64-64-1 network; as matrix products 64 us with tangents and 52 without, of which 14
 // and 7 are the matrix instructions at peak: bound by the barriers between the phases and the activations.
+// The LDS (153 KB for every network) leaves a CU to one workgroup.  Beside two streams that are never out of batches
+// of 48 molecules a training step takes 11.5 ms (5.5 alone) with FP32-grid molecules and 15.2 with FP64 ones; the
+// 97 KB kernel of one point a wave took 28.6 and 26.0 (17.2 alone), so the workgroups do get their CUs.
 // MFMA operand layout (16x16x4, one wave): lane l supplies A[l%16][l/16] and B[l/16][l%16]; it receives
 // D[4v + l/16][l%16] in element v.
 constexpr int AG = 2;              // groups of a workgroup
@@ -300,7 +303,6 @@ constexpr int ANT = AG * 256;      // its threads
 constexpr int AS = 66;             // LDS row stride (doubles)
 constexpr int AROWS = 32;          // rows of a tile
 constexpr int AW1 = (WMAXW + 3) / 4 * 4;  // rows of W1 in LDS
-constexpr int AKQ = HMAX / 4;      // k steps of a hidden layer
 constexpr int AXL = (AW1 + 7) / 8;  // window entries a thread fetches
 constexpr int ATILE = 3 * AROWS * AS + 4 * AROWS + AROWS;  // LDS of a group (doubles)
 constexpr size_t ADJ_MLP_LDS = (size_t)(AW1 * AS + HMAX * AS + AG * ATILE) * 8;
@@ -1092,7 +1094,6 @@ int qex1d_kohn_sham_vjp(const qex1d_problem* p, const qex1d_inputs* in, const qe
   const long BN = (long)a.B * a.N;
   const double s2 = -0.5 / (a.dx * a.dx);
   const double Td = s2 * -2.5, Tb = s2 * (4.0 / 3.0), Tc = s2 * (-1.0 / 12.0);
-  const int HL = a.NL == 2 ? a.H2 : a.H1;
   const size_t eig_lds = adj_eig_lds(a.N);
   const bool glob = p->xc_kind == QEX1D_XC_GLOBAL_MLP;
   const size_t gmlp_lds = (2 * (size_t)a.N + 2 * (NT / 64) * 64 + 12 * 64 + 8) * 8;

@@ -7,7 +7,7 @@
 //   k_eval_ao             phi[g][mu]
 //   k_rho                 rho_g = phi_g^T D phi_g, D in LDS (broadcast), phi_g in registers
 //   k_vxc                 LDA (Slater + VWN5) and per-chunk partials of phi^T diag(w v) phi
-//   k_coulomb             J (and K for Hartree-Fock) from the ERI pair matrix (HBM-bound GEMV)
+//   k_coulomb_*           J (and K for Hartree-Fock) from the ERI pair matrix (HBM-bound GEMV)
 //   k_scf_*               Fock build + CDIIS, generalized eigh (orthogonaliser X = L^-T of the
 //                         overlap Cholesky, parallel cyclic Jacobi warm-started from the previous
 //                         eigenvectors), density matrix, energy, convergence -- one workgroup each
@@ -1660,11 +1660,6 @@ __device__ __forceinline__ void coulomb_body(int bid, int nblk, int n, int npair
   }
 }
 
-__global__ __launch_bounds__(NT) void k_coulomb(int n, int npair, const double* eri, const double* dm, double* J,
-                                                double* K) {
-  coulomb_body(blockIdx.x, gridDim.x, n, npair, eri, dm, J, K);
-}
-
 // ---------------------------------------------------------------------------------------------
 // small dense linear algebra in one workgroup (row-major n x n, n <= 96)
 // ---------------------------------------------------------------------------------------------
@@ -2108,6 +2103,8 @@ __global__ __launch_bounds__(NT_EIG) void k_scf_step(const Scf3* __restrict__ ss
   __syncthreads();
   p.each(n, n, [&](int r, int c, double x) { A[r * S + c] = x; });
   __syncthreads();
+  // (two vectors more than the cycle uses: where levels of different blocks tie at n_occ within the multisection's
+  // 2^-48, their refined values may come in another order, and a slot without a vector must not come first)
   qexeig::symeig(n, A, Z, S, s.mo, s.eigf, sh, full ? n : nocc + 2);
   stage(n, n, s.X, A, S);
   __syncthreads();

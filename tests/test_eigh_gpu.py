@@ -135,7 +135,7 @@ def test_degen_eigh_autograd():
 
 @pytest.mark.parametrize("n", [4, 8, 9, 15, 17, 31, 32, 33, 63, 64, 65, 79, 81, 95])
 def test_register_patch_edges(geigh, n):
-    """Sizes at the edges of the register patches (8 columns, 32 rows) and of the size classes; a random
+    """Sizes at the edges of the register patches (8 columns; 64 rows, the Cholesky factor 32) and of the size classes; a random
     spectrum, one with 3 levels of multiplicity n / 3, a graded one and a shifted glued-Wilkinson-like
     tridiagonal with pairs closer than the cluster threshold, at norms 1, 1e-30 and 1e30."""
     rng = np.random.default_rng(100 + n)

@@ -86,8 +86,9 @@ def test_xc_evaluate_matches_oracle(name):
                                    [3, 5, 63, 33, 1], [33, 64, 64, 64, 64, 1], [7, 16, 8, 49, 12, 1]])
 @pytest.mark.parametrize("npts", [5, 16, 131])
 def test_matrix_core_network_sizes(sizes, npts):
-    """One to four hidden layers, windows, widths and point counts at the edges of the 16-point tiles and of
-    the 8-row k steps, more systems than waves: the bar of this file."""
+    """One to four hidden layers; windows and widths that are no multiples of the matrix instruction's 16 x 16 x 4,
+    and point counts that leave a 48-point tile (three row blocks of 16) nearly empty, full and ragged: the
+    bar of this file."""
     rng = np.random.default_rng(sum(sizes) + npts)
     W = [rng.standard_normal((a, b)) / np.sqrt(a) for a, b in zip(sizes[:-1], sizes[1:])]
     b = [0.1 * rng.standard_normal(k) for k in sizes[1:]]
