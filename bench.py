@@ -406,7 +406,7 @@ def run_c4(args):
 
     # algorithmic work of each kernel kind summed over the timed launches (active cycles only;
     # cycles enqueued after convergence return at once and are not counted as work)
-    work = {"rho": 0.0, "vxc": 0.0, "coulomb": 0.0, "scf_eigh": 0.0}
+    work = {"rho": 0.0, "vxc": 0.0, "coulomb": 0.0, "scf_eigh": 0.0, "scf_fock": 0.0}
     for n, m in zip(C4_CHAINS, mols):
         mf = last[n]
         nao, ng = m.nao, mf.grids.size
@@ -416,13 +416,14 @@ def run_c4(args):
         work["vxc"] += cyc * (2.0 * ng * nao * nao + (2.0 * ng * nao * (m.nelectron // 2) if mixed else 0.0))
         npair = nao * (nao + 1) // 2
         work["coulomb"] += cyc * 8.0 * npair * npair  # bytes: one pass over the ERI pair matrix
-        # the cycle's dense work is one launch: eigensolve and, past the guess, the Fock matrix and CDIIS
-        work["scf_eigh"] += cyc * 9.0 * nao ** 3 + mf.cycles * 8.0 * nao ** 3
+        # eigensolve and, past the guess, the Fock matrix and CDIIS: on the FP64 path one launch ("scf_eigh")
+        work["scf_eigh"] += cyc * 9.0 * nao ** 3
+        work["scf_fock" if mixed else "scf_eigh"] += mf.cycles * 8.0 * nao ** 3
     for k in work:
         work[k] *= args.steps
     kern = {name: (ms[i], cnt[i]) for i, name in enumerate(_lib.KERNEL_KINDS) if cnt[i]}
     dom = max(kern, key=lambda k: kern[k][0])
-    if dom in ("rho", "vxc", "scf_eigh"):
+    if dom in ("rho", "vxc", "scf_eigh", "scf_fock"):
         bound, unit, peak = ("mfma" if dom in ("rho", "vxc") else "fp64-latency"), "TFLOP/s", 78.6
         if mixed and dom == "vxc":
             peak = 157.3  # the fused FP32 grid kernel: dense FP32 MFMA peak
@@ -434,7 +435,7 @@ def run_c4(args):
         bound, unit, peak, achieved = "mfma", "TFLOP/s", 78.6, None
     rates = {}
     for k in work:
-        if k in kern and kern[k][0] > 0:
+        if k in kern and kern[k][0] > 0 and work[k] > 0:
             scale = 1e9 if k == "coulomb" else 1e12
             rates[k] = round(work[k] / (kern[k][0] * 1e-3) / scale, 3)
     all_lat = np.concatenate([np.array(v) for v in lat.values()])
@@ -590,7 +591,7 @@ def run_eri(args):
 
 # c3 kinds: the MLP adjoint and the eigen adjoint run on the FP64 vector units (no matrix cores); the
 # forward MLP on FP64 matrix cores; the forward eigensolver is latency-bound
-C3_BOUND = {"adj_mlp": "fp64-valu", "adj_eig": "fp64-latency", "mlp": "mfma", "eigen": "fp64-latency"}
+C3_BOUND = {"adj_mlp": "mfma", "adj_eig": "fp64-latency", "mlp": "mfma", "eigen": "fp64-latency"}
 
 
 def _c3_traffic():
@@ -693,10 +694,11 @@ def run_c3(args):
     kern = {name: (ms[i], cnt[i]) for i, name in enumerate(_lib.KERNEL_KINDS) if cnt[i]}
     dom = max(kern, key=lambda k_: kern[k_][0])
     value = B * args.steps / elapsed
-    # algorithmic FLOPs per launch: the MLP adjoint runs six network-sized GEMV passes per point
-    # (primal and tangent forward, primal and tangent backward, primal and tangent weight products)
+    # algorithmic FLOPs per launch: the MLP adjoint is six network-sized products per point (primal and tangent
+    # forward, primal and tangent backward, primal and tangent weight products); the energy pass, every
+    # second launch, has no tangents and three
     net = sum(WIDTHS[i] * WIDTHS[i + 1] for i in range(len(WIDTHS) - 1))
-    fl = {"adj_mlp": 12.0 * net * B * len(grids), "mlp": 6.0 * net * B * len(grids),
+    fl = {"adj_mlp": 9.0 * net * B * len(grids), "mlp": 6.0 * net * B * len(grids),
           "eigen": None, "adj_eig": 40.0 * len(grids) * B}
     avg = {k_: v[0] / v[1] for k_, v in kern.items()}
     achieved = (fl[dom] / (avg[dom] * 1e-3) / 1e12) if fl.get(dom) else None
@@ -813,17 +815,19 @@ def _work_1d(kind, b_ne):
     return 0.0
 
 
-def _work_3d(kind, nao, ngrid, cycles, nocc=0, fused=False):
+def _work_3d(kind, nao, ngrid, cycles, nocc=0, mixed=False):
     """Work of one molecule's launches of ``kind`` over its SCF (guess + cycles): FLOPs, or bytes for
-    the Coulomb kernel.  ``fused``: the FP32 grid kernel (rho from the occupied orbitals, 2 ng n nocc,
-    and the Vxc contraction, 2 ng n^2, in one pass)."""
+    the Coulomb kernel.  ``mixed``: the FP32 grid path (rho from the occupied orbitals, 2 ng n nocc,
+    and the Vxc contraction, 2 ng n^2, in one kernel; Fock and eigensolver in two)."""
     n, c = nao, cycles + 1
-    if kind == "vxc" and fused:
+    if kind == "vxc" and mixed:
         return c * (2.0 * ngrid * n * n + 2.0 * ngrid * n * nocc)
     if kind in ("rho", "vxc"):
         return c * 2.0 * ngrid * n * n
     if kind == "scf_eigh":
-        return c * 13.0 * n ** 3 + cycles * 8.0 * n ** 3  # (eigensolve, and the Fock matrix and CDIIS past the guess)
+        return c * 13.0 * n ** 3 + (0.0 if mixed else cycles * 8.0 * n ** 3)  # (FP64: with the Fock matrix and CDIIS)
+    if kind == "scf_fock":
+        return cycles * 8.0 * n ** 3
     if kind == "coulomb":
         P = n * (n + 1) // 2
         return c * 8.0 * P * P
@@ -834,7 +838,7 @@ ROOF = {  # kind -> (bound, peak, unit)
     "eigen": ("fp64-latency", 78.6, "TFLOP/s"), "mlp": ("mfma", 78.6, "TFLOP/s"),
     "potential": ("fp64-latency", 78.6, "TFLOP/s"), "rho": ("mfma", 78.6, "TFLOP/s"),
     "vxc": ("mfma", 78.6, "TFLOP/s"), "scf_eigh": ("fp64-latency", 78.6, "TFLOP/s"),
-    "coulomb": ("hbm", 8000.0, "GB/s"),
+    "scf_fock": ("fp64-latency", 78.6, "TFLOP/s"), "coulomb": ("hbm", 8000.0, "GB/s"),
 }
 
 
@@ -843,7 +847,7 @@ if os.path.exists(ERI_FLOPS):  # the ERI: executed FP64 operations per molecule 
     ROOF["eri"] = ("fp64-valu", 78.6, "TFLOP/s")
 
 
-def _stream_work(stats, kind, fused=False):
+def _stream_work(stats, kind, mixed=False):
     tot = 0.0
     if kind == "eri":  # one ERI computation per served 3D request
         ops = _eri_fp64_ops()
@@ -853,7 +857,7 @@ def _stream_work(stats, kind, fused=False):
             tot += T * _work_1d(kind, b_ne)
     else:
         for nao, ng, cyc, nocc in stats.work_3d:
-            tot += _work_3d(kind, nao, ng, cyc, nocc, fused)
+            tot += _work_3d(kind, nao, ng, cyc, nocc, mixed)
     return tot
 
 
@@ -993,9 +997,8 @@ def run_c5(args):
                                 "p99_ms_3d": round(s2.get("p99_ms_3d", float("nan")), 2),
                                 "converged": sum(1 for c in sw.completions if good(c))}
     # ---- roofline of the dominant kernel: algorithmic work of the timed launches / their summed time ----
-    fused = mixed and dom in ROOF_FP32_GRID
-    bound, peak, unit = ROOF_FP32_GRID[dom] if fused else ROOF[dom]
-    work = _stream_work(st, dom, fused)
+    bound, peak, unit = ROOF_FP32_GRID[dom] if mixed and dom in ROOF_FP32_GRID else ROOF[dom]
+    work = _stream_work(st, dom, mixed)
     scale = 1e9 if unit == "GB/s" else 1e12
     achieved = work / (dom_ms * 1e-3) / scale if dom_ms > 0 else None
     traffic = None
