@@ -32,9 +32,8 @@ struct Bar {
   int n = 0, count = 0, gen = 0;
 };
 struct Wave {
-  Bar bar[7];                 // groups of 1 << k lanes: bar of a group of 64; smaller ones below
   std::vector<Bar> group[7];  // [k]: 64 >> k groups of 1 << k lanes
-  uint64_t val[7][2][64];
+  uint64_t val[7][2][64];     // [k]: what the lanes exchange, alternating (a lane may be one exchange ahead)
 };
 struct Fiber {
   ucontext_t ctx;
@@ -174,7 +173,7 @@ inline int __builtin_amdgcn_update_dpp(int, int x, int ctrl, int, int, bool) {
   }
   return (int)lanes::exchange((uint64_t)(uint32_t)x, src, k);
 }
-// hardware reciprocals: relative error below 2^-24 (truncated here), exact for 0 and infinity
+// hardware reciprocals: cut to 24 bits after the leading one, exact for 0 and infinity
 inline double lanes_cut(double x) { return isfinite(x) ? lanes::value(lanes::bits(x) & ~((1ull << 28) - 1)) : x; }
 inline double __builtin_amdgcn_rcp(double x) { return lanes_cut(1.0 / x); }
 inline double __builtin_amdgcn_rsq(double x) { return lanes_cut(1.0 / sqrt(x)); }
